@@ -128,7 +128,7 @@ void g2_destroy(g2_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (DevBuf* b : {&c->rp, &c->cols, &c->src, &c->gm_task_off, &c->counters, &c->scratch,
                       &c->big_scratch, &c->list, &c->hist, &c->per_root, &c->order, &c->deg, &c->big_list2, &c->spans,
-                      &c->batch_off, &c->batch_progs, &c->batch_q, &c->donate, &c->taskbuild, &c->orient, &c->roots})
+                      &c->batch_progs, &c->batch_q, &c->donate, &c->taskbuild, &c->orient, &c->roots})
         release(c, *b);
     if (c->spill) (void)hipHostFree(c->spill);
     for (auto& ev : c->ev)
@@ -164,10 +164,11 @@ int g2_upload_view(g2_ctx* c, const uint64_t* rp, uint64_t nv, const uint32_t* c
     // below the root degree, which root no match).
     std::vector<uint64_t> task_off(ns + 1, 0), src_deg(ns);
     const uint32_t chunk = c->tune.gm_chunk;
-    uint64_t unclosed = 0;
+    uint64_t unclosed = 0, deg_sum = 0;
     for (uint64_t i = 0; i < ns; i++) {
         const uint64_t d = rp[src[i] + 1] - rp[src[i]];
         src_deg[i] = d;
+        deg_sum += d;
         uint64_t w = 1;
         if (chunk && d > chunk) w = (d + chunk - 1) / chunk;
         task_off[i + 1] = task_off[i] + w;
@@ -229,7 +230,8 @@ int g2_upload_view(g2_ctx* c, const uint64_t* rp, uint64_t nv, const uint32_t* c
     c->gm_task_chunk = chunk;
     c->h_gm_task_off.swap(task_off);
     c->h_src_deg.swap(src_deg);
-    c->batch_off_valid = false;
+    c->src_deg_sum = deg_sum;
+    c->batch_tasks_valid = false;
     c->view_ok = true;
     return G2_OK;
 }

@@ -97,6 +97,32 @@ __device__ __forceinline__ uint64_t fetch_tasks(unsigned long long* ctr, uint32_
     return uniform((uint64_t)t);
 }
 
+// Tasks [0, total) dealt over kQueues counters on lines of their own: counter
+// k holds tasks k, k + kQueues, ...  One counter serves about one atomic per
+// 12 ns, whichever wave asks (2M windows fetched singly from one counter held
+// a 3 ms launch for 26 ms), so a wave starts on counter `k` of its own choice
+// and moves to another with tasks left when that one is used up.  Returns
+// kNoTask when none is left.  (Wave barrier as in fetch_task; every round
+// either takes a task or leaves a counter that is used up for good.)
+constexpr uint32_t kQueues = 16;
+constexpr uint32_t kQueueStride = 16;  // u64 words: 128 bytes
+constexpr uint64_t kNoTask = ~0ull;
+__device__ __forceinline__ uint64_t queue_next(unsigned long long* q, uint32_t& k, uint64_t total) {
+    while (true) {
+        __builtin_amdgcn_wave_barrier();
+        unsigned long long i = 0;
+        if (lane_id() == 0) i = atomicAdd(&q[k * kQueueStride], 1ull);
+        const uint64_t t = uniform((uint64_t)i) * kQueues + k;
+        if (t < total) return t;
+        const uint32_t l = lane_id();
+        unsigned long long at = 0;
+        if (l < kQueues) at = __hip_atomic_load(&q[l * kQueueStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t open = (uint32_t)ballot(l < kQueues && at * kQueues + l < total);
+        if (!open) return kNoTask;
+        k = (k + (uint32_t)__builtin_ctz((open >> k) | (open << (kQueues - k)))) % kQueues;
+    }
+}
+
 // first index in [lo,hi) whose value is >= val (hi if none)
 __device__ __forceinline__ uint64_t lower_bound(const uint32_t* __restrict__ cols, uint64_t lo, uint64_t hi, uint32_t val) {
     while (lo < hi) {

@@ -30,7 +30,6 @@ struct GmStep {
     uint32_t nafter, after[G2_MAXQ];
     uint32_t nacond, acop[G2_MAXQ], acpos[G2_MAXQ];
     uint32_t store_prefix;        // strategy[id+1] == PREFIX (byte model only)
-    uint32_t pre_is_prev;         // the pre-intersection equals position id-1's candidate set
 };
 
 struct GmProgram {
@@ -38,18 +37,53 @@ struct GmProgram {
     GmStep step[G2_MAXQ];
 };
 
-// canonical matching kernel: counters, then its arguments
-enum { GCTR_NEXT = 0, GCTR_COUNT, GCTR_BYTES, GCTR_NODES, GCTR_N };
+// The counting walk's form of a plan (g2_gm_walk.hip): back neighbours and
+// conditions of a position split at the previous position.
+struct GmWalkStep {
+    uint32_t npre, pre[G2_MAXQ];  // back neighbours at positions < id-1
+    uint32_t prev;                // position id-1 is a back neighbour
+    uint32_t npc, pcop[2 * G2_MAXQ], pcpos[2 * G2_MAXQ];  // order conditions against positions < id-1 (0: <, 1: >)
+    uint32_t npneq, pneq[G2_MAXQ];        // positions < id-1 it must differ from
+    uint32_t prev_gt, prev_lt, prev_ne;   // conditions against position id-1
+    uint32_t alias;               // the candidates positions < id-1 leave are position id-1's list
+};
+
+struct GmWalk {
+    uint32_t n;
+    GmWalkStep step[G2_MAXQ];
+};
+
+// admissible values of a position: [lo, hi), hi 0xffffffff = no upper bound
+struct Range {
+    uint32_t lo, hi;
+};
+
+// canonical matching kernels: counters (next task of the accounting traversal,
+// matches, modelled bytes, extensions, listed windows, and from GCTR_QUEUE on
+// the walk's task queues, queue_next), then their arguments
+enum { GCTR_NEXT = 0, GCTR_COUNT, GCTR_BYTES, GCTR_NODES, GCTR_SPLIT, GCTR_QUEUE = 16, GCTR_N = GCTR_QUEUE + 16 * 16 };
 constexpr int kGmMaxBlockWaves = 4;
+
+// `len` entries of source `src`'s row from entry `first` on; part of their
+// position-2 candidates
+struct WalkWindow {
+    uint32_t src, first, len;
+    uint16_t part, parts;
+};
 
 struct GmArgs {
     const uint64_t* __restrict__ rp;
     const uint32_t* __restrict__ cols;
     const uint32_t* __restrict__ src;
-    const uint64_t* __restrict__ task_off;  // ns+1 window offsets per source (null: one task per source)
     uint64_t ns;
+    // accounting traversal
+    const uint64_t* __restrict__ task_off;  // ns+1 window offsets per source
     uint64_t ntasks;
     uint32_t chunk;                         // level-1 window length (0 = whole row)
+    // counting walk
+    const WalkWindow* __restrict__ heavy;   // windows of the rows longer than heavy_min (null: none listed)
+    uint64_t heavy_min;
+    uint32_t run;                           // other sources per task
     uint32_t* scratch;
     uint64_t cap;                           // entries per list
     unsigned long long* ctr;
@@ -109,6 +143,7 @@ struct g2_ctx {
     // matching
     bool has_plan = false;
     g2::GmProgram prog{};
+    g2::GmWalk walk{};
     bool local_ok = false;        // the plan qualifies for the oriented local-bitmap path
     g2::LocalProgram lprog{};
     g2::DevBuf big_list2;
@@ -119,11 +154,11 @@ struct g2_ctx {
 
     // batched matching
     std::vector<uint64_t> h_src_deg;  // host copy: degree of every source
-    g2::DevBuf batch_off;         // task offsets for a batch window != gm_task_chunk
-    uint32_t batch_window = 0;
+    uint64_t src_deg_sum = 0;
+    uint32_t batch_window = 0;        // root tasks of the last batch window
     uint64_t batch_ntasks = 0;
-    bool batch_off_valid = false;
-    g2::DevBuf batch_progs;       // GmProgram per query
+    bool batch_tasks_valid = false;
+    g2::DevBuf batch_progs;       // GmWalk per query
     g2::DevBuf batch_q;           // per-query counts, nodes, order, flags
 };
 
@@ -134,7 +169,7 @@ int set_err(g2_ctx* c, int code, const std::string& msg);
 // resident waves per CU of a persistent grid: the context's setting, else the
 // kernel's own default (measured on MI355X: latency-bound searches gain up to
 // the occupancy their register use allows)
-enum WaveKind { WK_MCE = 16, WK_GM = 16, WK_GM_LOCAL = 32, WK_FEATURES = 16 };
+enum WaveKind { WK_MCE = 16, WK_GM = 16, WK_WALK = 20, WK_GM_LOCAL = 32, WK_FEATURES = 16 };
 inline uint32_t waves_per_cu(const g2_ctx* c, WaveKind k) {
     return c->tune.waves_per_cu ? c->tune.waves_per_cu : (uint32_t)k;
 }
@@ -148,8 +183,17 @@ int gm_run(g2_ctx* c, uint32_t flags, uint64_t* count, uint64_t* per_root_count,
 int gm_compile(g2_ctx* c, const g2_plan* p);
 // plan tables re-indexed by position; G2_EINVAL with *why naming the first broken table
 int gm_program(const g2_plan* p, GmProgram* out, const char** why);
-// gm_kernel (no byte accounting) over `blocks` workgroups of block_waves waves
-hipError_t gm_launch(const GmArgs& a, const GmProgram& prog, uint64_t blocks, uint32_t block_waves, hipStream_t s);
+GmWalk walk_program(const GmProgram& g);
+// list the windows of the long root rows into a, for nq plans of up to n
+// positions (chunk: window length, 0 = by rule)
+int walk_split(g2_ctx* c, GmArgs& a, uint32_t n, uint32_t nq, uint32_t chunk);
+// sources per task of the counting walk: blocks of up to 16 where every wave
+// still gets several (short rows cost little more than their fetch)
+uint32_t walk_run(uint64_t ns, uint64_t waves);
+// the counting walk over `blocks` workgroups of block_waves waves
+hipError_t walk_launch(const GmArgs& a, const GmWalk& walk, uint64_t blocks, uint32_t block_waves, hipStream_t s);
+// the largest grid (at most nblocks) whose wave arenas fit the budget
+uint64_t fit_arenas(g2_ctx* c, uint64_t nblocks, uint64_t per_block);
 void gm_local_compile(g2_ctx* c, const g2_plan* p);
 // triangle count per rank (tri, u64) and triangle-carrying oriented entries
 // per rank (sup, u32) of the uploaded view, through its oriented rows (built

@@ -13,8 +13,9 @@
 #include "g2_internal.hpp"
 
 namespace g2 {
-constexpr uint64_t kNoAllocBytes = 64ull << 20;  // the array's size: 64 MiB
-constexpr uint64_t kNoAllocHead = 256;           // counters at the front; the arenas follow
+constexpr uint64_t kNoAllocHead = 2560;          // counters at the front; the arenas follow
+constexpr uint64_t kNoAllocArena = (64ull << 20) - 256;  // bytes of the arenas
+constexpr uint64_t kNoAllocBytes = kNoAllocHead + kNoAllocArena;
 constexpr int kNoAllocMaxDevices = 64;
 // counters after GCTR_*: largest degree, malformed row_ptrs / column / source
 enum { NCHK_MAXDEG = GCTR_N, NCHK_BADROW, NCHK_BADCOL, NCHK_BADSRC, NCHK_N };
@@ -28,7 +29,7 @@ namespace g2 {
 // the counters must start at zero on every call (a kernel, not a memset, so
 // that the sequence stays capturable)
 __global__ __launch_bounds__(64) void noalloc_clear_kernel(unsigned long long* head) {
-    if (threadIdx.x < kNoAllocHead / 8) head[threadIdx.x] = 0;
+    for (uint32_t i = threadIdx.x; i < kNoAllocHead / 8; i += blockDim.x) head[i] = 0;
 }
 
 // Largest degree and the bounds of the caller's CSR, read only within the
@@ -133,7 +134,7 @@ int g2_gm_run_noalloc(int device, const uint64_t* row_ptrs, uint64_t nv, const u
     // as long as the longest row, as in g2_gm_run
     const uint64_t cap = std::max<uint64_t>(h[NCHK_MAXDEG], 64);
     const uint64_t per_wave = cap * 2 * prog.n * 4;
-    const uint64_t fit = (kNoAllocBytes - kNoAllocHead) / per_wave;
+    const uint64_t fit = kNoAllocArena / per_wave;
     if (fit == 0) return noalloc_fail(G2_EBUDGET, "the largest degree needs a wave arena beyond the 64 MiB scratch");
     const uint64_t waves = std::min<uint64_t>((uint64_t)d.num_cus * WK_GM, fit);
     const uint32_t bw = (uint32_t)std::min<uint64_t>(kGmMaxBlockWaves, waves);
@@ -142,15 +143,14 @@ int g2_gm_run_noalloc(int device, const uint64_t* row_ptrs, uint64_t nv, const u
     a.rp = row_ptrs;
     a.cols = cols;
     a.src = sources;
-    a.task_off = nullptr;
     a.ns = ns;
-    a.ntasks = ns;
-    a.chunk = 0;
+    a.heavy_min = ~0ull;  // (no room for a list of windows: every row whole)
+    a.run = walk_run(ns, waves);
     a.scratch = (uint32_t*)((char*)d.ptr + kNoAllocHead);
     a.cap = cap;
     a.ctr = ctr;
     a.per_root = nullptr;
-    if ((e = gm_launch(a, prog, blocks, bw, 0)) != hipSuccess) return noalloc_fail(G2_EHIP, "gm launch", e);
+    if ((e = walk_launch(a, walk_program(prog), blocks, bw, 0)) != hipSuccess) return noalloc_fail(G2_EHIP, "gm launch", e);
     if ((e = hipMemcpy(h, ctr, GCTR_N * 8, hipMemcpyDeviceToHost)) != hipSuccess)
         return noalloc_fail(G2_EHIP, "D2H count", e);
     *count = h[GCTR_COUNT];
