@@ -62,24 +62,32 @@ namespace g2 {
 
 // counters: next task, matches, nodes, (deferred roots, their largest need)
 // per pass, largest need that fit no arena
-enum { LCTR_NEXT = 0, LCTR_COUNT, LCTR_NODES, LCTR_DEFER, LCTR_ERR = LCTR_DEFER + 8, LCTR_N };
+// (copied back to the host), then the first pass's task queues (queue_next)
+enum { LCTR_NEXT = 0, LCTR_COUNT, LCTR_NODES, LCTR_DEFER, LCTR_ERR = LCTR_DEFER + 8, LCTR_HOST, LCTR_QUEUE = 16,
+       LCTR_N = LCTR_QUEUE + kQueues * kQueueStride };
+static_assert(LCTR_HOST <= LCTR_QUEUE, "counters");
 
 constexpr int kLocalBlockWaves = 4;     // gm_local_kernel: __launch_bounds__(256)
 constexpr uint32_t kLRowWords = 448;    // per-wave LDS rows (u64 words)
-constexpr uint32_t kLU = 256;           // per-wave LDS copy of U (u32)
-// workgroup passes: threads, LDS row words, |U| limit, value buckets, and
-// workgroups per CU (the LDS each takes allows no more)
-constexpr int kB1Threads = 256, kB1RowWords = 3136, kB1U = 448, kB1Buckets = 2048, kB1PerCu = 4;     // 25 KiB rows: |U| 448 at stride 7
-constexpr int kB2Threads = 512, kB2RowWords = 7700, kB2U = 700, kB2Buckets = 2048, kB2PerCu = 2;      // 60 KiB rows: |U| 700 at stride 11
-constexpr int kB3Threads = 1024, kB3RowWords = 17664, kB3U = 1040, kB3Buckets = 2047, kB3PerCu = 1;  // 138 KiB rows: |U| 1039 at stride 17
+constexpr uint32_t kLU = 256;           // |U| limit of a wave (triangle features; rows allow kLMembers)
+constexpr uint32_t kLMembers = 149;     // members of a root whose rows fit kLRowWords
+constexpr uint32_t kLSlots = 512;       // hash slots over U, per wave
+// workgroup passes: threads, LDS row words, |U| limit, and workgroups per CU
+// (the LDS each takes allows no more)
+constexpr int kB1Threads = 256, kB1RowWords = 3136, kB1U = 448, kB1PerCu = 4;     // 25 KiB rows: |U| 448 at stride 7
+constexpr int kB2Threads = 512, kB2RowWords = 7700, kB2U = 700, kB2PerCu = 2;     // 60 KiB rows: |U| 700 at stride 11
+constexpr int kB3Threads = 1024, kB3RowWords = 17664, kB3U = 1040, kB3PerCu = 1;  // 138 KiB rows: |U| 1039 at stride 17
 constexpr uint32_t kRev = 0x80000000u;  // work-list flag: look the later members up in the row
-constexpr int kItems = 8;               // work items per thread in flight in the workgroup build
+constexpr int kVecs = 8;                // 64-entry row pieces per wave in flight in the workgroup build
+constexpr int kVecsW = 4;               // and in the wave build
+constexpr uint32_t kRevFactor = 12, kRevFactorFar = 24;  // row entries per later member from which members are looked up (build_rows)
+constexpr uint64_t kNearBytes = 128ull << 20;             // oriented rows this long stay in the last-level cache
+constexpr int kRevItems = 4;            // later members per lane in flight where a row is searched instead
+constexpr uint32_t kSlots = 4096;       // hash slots over U (workgroup build), by the rank's low bits
 constexpr int kItemsW = 2;              // work items per lane in flight in the wave build
 constexpr uint32_t kOwnScan = 8;        // a round or slice with at most this many owners after its first scans them
 constexpr int kRowUnroll = 8;           // row entries per lane in flight while building the oriented rows
-constexpr uint32_t kFetchRun = 8;       // roots per counter fetch in the first pass (a sweep of 4..64 favoured 8)
-constexpr uint32_t kWB = 256;           // value buckets over U for a root in the wave's LDS (|U| <= 149: u8 indices)
-constexpr uint32_t kWBMin = 32;         // smaller U: a search of all of U is as short
+constexpr uint32_t kFetchRun = 8;       // roots per fetch in the first pass, where every wave still gets many
 
 struct LocalArgs {
     const uint64_t* __restrict__ orp;   // oriented rows over ranks
@@ -87,6 +95,8 @@ struct LocalArgs {
     const uint32_t* __restrict__ list;  // roots of the large-root pass (nullable: roots = [0, ntasks))
     uint64_t ntasks;
     LocalProgram prog;
+    uint32_t run;                       // first pass: roots per fetch,
+    uint32_t factor;                    //   and build_rows' factor
     uint64_t* scratch;
     uint64_t scratch_words;
     uint32_t* big_list;                 // deferred roots (null in the last pass)
@@ -171,24 +181,9 @@ __device__ inline void cand_range(const LocalProgram& P, uint32_t i, const uint3
 // triangle (root, U_i, U_j): one count for each member in a.tri, one for the
 // root in hits, and the flags of its three oriented entries (root row from
 // entry xlo on).
-// Value buckets over U (optional): bucket(v) = floor((v - ulo) * NB / range)
-// by one high multiply (the identity when U spans at most NB ranks); a
-// lookup of w searches U[bkt[b], bkt[b+1]) for b = bucket(w), in hb halving
-// steps (hb: the highest power of two <= the largest bucket).
-struct UBuckets {
-    const uint8_t* bkt;  // null: search all of U
-    uint32_t nb, ulo, bmul, hb;
-    uint32_t imask;      // ~0 when U spans at most nb ranks (then bmul = 0 and the bucket is v - ulo), else 0
-    __device__ uint32_t bucket(uint32_t v) const {
-        const uint32_t d = v - ulo;
-        return min(__umulhi(d, bmul) + (d & imask), nb - 1);
-    }
-};
-
 template <int MODE>
 __device__ __forceinline__ void build_chunk(const LocalArgs& a, const uint32_t* U, uint64_t* rows, uint32_t m,
-                                            uint32_t W, uint32_t a0, uint64_t xlo, uint32_t& hits,
-                                            const UBuckets& B) {
+                                            uint32_t W, uint32_t a0, uint64_t xlo, uint32_t& hits) {
     const uint32_t lane = lane_id();
     const uint32_t na = umin32(kWave, m - 1 - a0);  // members with a later member
     uint32_t st = 0;  // (row offsets fit 32 bits: this path runs with fewer than 2^32 row entries)
@@ -285,25 +280,12 @@ __device__ __forceinline__ void build_chunk(const LocalArgs& a, const uint32_t* 
             w[q] = f[q] >= T ? 0u : (cj[q] & kRev) ? pos[q] : w[q];
             pos[q] = 0;
         }
-        uint32_t lim[kItemsW];
-        uint32_t hb = hb_u;
-#pragma unroll
-        for (int q = 0; q < kItemsW; q++) lim[q] = m;
-        if (B.bkt) {  // (an entry above U_{m-1} lands in the last bucket and misses)
-            hb = B.hb;
-#pragma unroll
-            for (int q = 0; q < kItemsW; q++) {
-                const uint32_t b = B.bucket(w[q]);
-                pos[q] = B.bkt[b];
-                lim[q] = B.bkt[b + 1];
-            }
-        }
-        for (uint32_t step = hb; step >= 1; step >>= 1) {  // stream: pos = |{U_j < w}|
+        for (uint32_t step = hb_u; step >= 1; step >>= 1) {  // stream: pos = |{U_j < w}|
 #pragma unroll
             for (int q = 0; q < kItemsW; q++) {  // (clamped read, no branch)
                 const uint32_t c = pos[q] + step;
                 const uint32_t v = U[min(c, m) - 1];
-                pos[q] = (!(cj[q] & kRev) && c <= lim[q] && v < w[q]) ? c : pos[q];
+                pos[q] = (!(cj[q] & kRev) && c <= m && v < w[q]) ? c : pos[q];
             }
         }
         // lookups: rpos = |{entries <= w}| in the member's row, with the entry
@@ -358,6 +340,167 @@ __device__ __forceinline__ void build_chunk(const LocalArgs& a, const uint32_t* 
                 }
             }
         }
+    }
+}
+
+// Hash index over U (in LDS): slot[rank mod T] holds the last member put
+// there, next[member] the one before it.  An entry is 0 (none) or member + 1
+// (11 bits) | 4 rank bits above the slot's (a mismatch is another rank) |
+// kChain when another member follows.
+constexpr uint32_t kChain = 0x8000u, kMember = 0x7ffu, kTag = 0x7800u;
+static_assert(kB3U < (int)kMember, "members fit an entry");
+template <uint32_t T>
+struct HashIndex {
+    uint16_t* slot;       // T
+    uint16_t* next;       // |U|
+    const uint32_t* U;
+    static __device__ __forceinline__ uint32_t tag(uint32_t w) { return (w / T << 11) & kTag; }
+    // put member i (rank u) at the head of its slot (a 16-bit half of a word)
+    __device__ __forceinline__ void put(uint32_t i, uint32_t u) const {
+        uint32_t* word = reinterpret_cast<uint32_t*>(slot) + ((u & (T - 1)) >> 1);
+        const uint32_t sh = (u & 1) * 16;
+        uint32_t old = *word;
+        while (true) {
+            const uint32_t head = (old >> sh) & 0xffffu;
+            next[i] = (uint16_t)head;
+            const uint32_t e = (i + 1) | tag(u) | (head ? kChain : 0u);
+            const uint32_t seen = atomicCAS(word, old, (old & ~(0xffffu << sh)) | (e << sh));
+            if (seen == old) break;
+            old = seen;
+        }
+    }
+};
+
+// Local rows of members i0, i0 + stride, .. (64 of them, one per lane) by one
+// wave: hit(i, j) for every pair i < j of members joined by an edge.  Member i
+// has either the n entries of N+(U_i) to look up in U, or, when n exceeds
+// (m-1-i) x factor, its m-1-i later members to look up in N+(U_i) (global
+// memory).  A lookup there is a chain of ~9 loads, a streamed entry a share of
+// one: factors of 5, 8, 12, 16 and 24 took the 256-thread pass of R-MAT 22 in
+// 17.4, 16.3, 15.8, 16.2 and 16.5 ms.  In the first pass, with few members per
+// root, 12 is best where the rows stay in the last-level cache (R-MAT 20, 63
+// MB: 2.8 ms, 3.4 at 24), and 24 where they do not and a chain's loads come
+// from HBM (R-MAT 22, 257 MB: 12.4 ms, 15.4 at 12).
+// What bounds it: instruction issue and LDS reads per streamed entry (25.7 G
+// of them for R-MAT 22, 8% hits).  So a row is cut into pieces of 64 entries,
+// VECS of them (of one or several members) in flight, and everything about a
+// piece but its entries is a scalar; an entry costs one LDS read of its hash
+// slot, and a second only where the tag agrees (the members themselves and 1
+// in 16 of the others that meet one).  Rows average 150-310 entries on R-MAT
+// 18-20, so pieces are 85-90% full.
+template <int VECS, uint32_t T, class Hit>
+__device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T>& H, uint32_t m, uint64_t lo, uint32_t i0,
+                                           uint32_t stride, uint32_t factor, Hit hit) {
+    const uint32_t lane = lane_id();
+    const uint32_t mi = i0 + lane * stride;
+    uint32_t st = 0, len = 0, rem = 0;  // (row offsets fit 32 bits: this path runs with fewer than 2^32 row entries)
+    bool rev = false;
+    if (mi + 1 < m) {
+        const uint32_t u = H.U[mi];
+        const uint64_t e0 = a.orp[u];
+        const uint64_t n = a.orp[u + 1] - e0;
+        rem = m - 1 - mi;
+        rev = (uint64_t)rem * factor < n;
+        st = (uint32_t)e0;
+        len = (uint32_t)n;
+    }
+    uint64_t todo = ballot(len && !rev);
+    uint32_t cst = 0, left = 0, ci = 0;
+    while (left || todo) {
+        uint32_t own[VECS], cnt[VECS], w[VECS], e[VECS], v[VECS];
+#pragma unroll
+        for (int q = 0; q < VECS; q++) {
+            if (!left && todo) {
+                const uint32_t k = (uint32_t)__builtin_ctzll(todo);
+                todo &= todo - 1;
+                cst = read_lane(st, k);
+                left = read_lane(len, k);
+                ci = i0 + k * stride;
+            }
+            own[q] = ci;
+            cnt[q] = umin32(left, kWave);
+            // (a lane past the piece's end reads the root's own row)
+            w[q] = a.ocols[lane < cnt[q] ? (uint64_t)cst + lane : lo];
+            cst += kWave;
+            left -= cnt[q];
+        }
+#pragma unroll
+        for (int q = 0; q < VECS; q++) e[q] = lane < cnt[q] ? H.slot[w[q] & (T - 1)] : 0u;
+        uint32_t more = 0;
+#pragma unroll
+        for (int q = 0; q < VECS; q++) {
+            const bool cand = (e[q] & kMember) && (e[q] & kTag) == H.tag(w[q]);
+            v[q] = cand ? H.U[(e[q] & kMember) - 1] : ~w[q];
+        }
+#pragma unroll
+        for (int q = 0; q < VECS; q++) more |= v[q] != w[q] ? e[q] & kChain : 0u;
+        if (ballot(more != 0)) {  // members that share a slot
+#pragma unroll
+            for (int q = 0; q < VECS; q++)
+                while (v[q] != w[q] && (e[q] & kChain)) {
+                    e[q] = H.next[(e[q] & kMember) - 1];
+                    v[q] = H.U[(e[q] & kMember) - 1];
+                }
+        }
+#pragma unroll
+        for (int q = 0; q < VECS; q++)
+            if (v[q] == w[q]) hit(own[q], (e[q] & kMember) - 1);
+    }
+    // reversed members: one work list of (member, later member) over the
+    // lanes; pos = |{entries <= w}| in the member's row, the entry at pos-1
+    // kept; a lane's searches interleave step by step
+    const uint32_t rl = rev ? rem : 0u;
+    if (!ballot(rl != 0)) return;
+    uint32_t incl = rl;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+        const uint32_t y = __shfl_up(incl, o, kWave);
+        if (lane >= (uint32_t)o) incl += y;
+    }
+    const uint32_t pref = incl - rl, total = read_lane(incl, kWave - 1);
+    for (uint32_t f0 = 0; f0 < total; f0 += kRevItems * kWave) {
+        const uint32_t flast = umin32(f0 + kRevItems * kWave, total) - 1;
+        const uint32_t o0 = __popcll(ballot(pref <= f0)) - 1, o1 = __popcll(ballot(pref <= flast)) - 1;
+        uint32_t own[kRevItems], later[kRevItems], w[kRevItems], rst[kRevItems], rlen[kRevItems], pos[kRevItems],
+            last[kRevItems], rmax = 0;
+#pragma unroll
+        for (int q = 0; q < kRevItems; q++) own[q] = o0;
+        for (uint32_t o = o0 + 1; o <= o1; o++) {
+            const uint32_t po = read_lane(pref, o);
+#pragma unroll
+            for (int q = 0; q < kRevItems; q++) own[q] = po <= f0 + q * kWave + lane ? o : own[q];
+        }
+#pragma unroll
+        for (int q = 0; q < kRevItems; q++) {
+            const uint32_t f = f0 + q * kWave + lane;
+            const uint32_t item = f - __shfl(pref, (int)own[q], kWave);
+            rst[q] = __shfl(st, (int)own[q], kWave);
+            rlen[q] = __shfl(len, (int)own[q], kWave);
+            if (f >= total) rlen[q] = 0;
+            rmax = umax32(rmax, rlen[q]);
+            own[q] = i0 + own[q] * stride;
+            later[q] = umin32(own[q] + 1 + item, m - 1);
+            w[q] = H.U[later[q]];
+            pos[q] = 0;
+            last[q] = ~0u;
+        }
+        uint32_t step = 1;
+        while (step * 2 <= rmax) step *= 2;
+        for (step = rmax ? step : 0; step >= 1; step >>= 1) {
+#pragma unroll
+            for (int q = 0; q < kRevItems; q++) {
+                if (step <= rlen[q] - pos[q]) {
+                    const uint32_t y = a.ocols[(uint64_t)rst[q] + pos[q] + step - 1];
+                    if (y <= w[q]) {
+                        pos[q] += step;
+                        last[q] = y;
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kRevItems; q++)
+            if (rlen[q] && last[q] == w[q]) hit(own[q], later[q]);
     }
 }
 
@@ -447,43 +590,48 @@ __device__ __forceinline__ void walk_from(const LocalProgram& P, uint32_t* M, ui
     }
 }
 
-// One root on one wave: build the local rows over U, then each lane walks the
-// matches of the position-1 candidates lane, lane+64, ...
+// Matches of one root's local rows on one wave.  Clique plans with more than
+// 4 positions share the (r1, r2) pairs over the lanes, queued 64 at a time (one
+// r1 can hold most of the root's matches: 5-cliques of R-MAT 16: 11.5 ms
+// with one r1 per lane, 2.0 so); the
+// others give each lane the position-1 candidates lane, lane+64, ...
 template <int N, bool CLQ>
-__device__ __forceinline__ void local_root(const LocalArgs& a, uint64_t lo, uint32_t m, uint64_t* rows,
-                                           const uint32_t* U, uint32_t* Ucopy, uint8_t* bkt, uint64_t& lane_total,
-                                           uint64_t& nodes) {
+__device__ __forceinline__ void count_root(const LocalProgram& P, uint32_t m, const uint64_t* rows, uint32_t* queue,
+                                           uint64_t& lane_total, uint64_t& nodes) {
     const uint32_t lane = lane_id();
     const uint32_t W = row_stride(m);
-    for (uint32_t i = lane; i < m * W; i += kWave) rows[i] = 0;
-    if (Ucopy)
-        for (uint32_t i = lane; i < m; i += kWave) Ucopy[i] = a.ocols[lo + i];
-    wave_sync();
-    UBuckets B{};
-    if (bkt && m > kWBMin) {  // value buckets over U (U in LDS, m <= 149)
-        const uint32_t range = U[m - 1] - U[0] + 1;
-        B.nb = kWB;
-        B.ulo = U[0];
-        // (uniform values made opaque to the compiler: it would otherwise
-        // widen the high multiply to 64 bits)
-        B.imask = __builtin_amdgcn_readfirstlane(range <= kWB ? ~0u : 0u);
-        B.bmul = __builtin_amdgcn_readfirstlane(range <= kWB ? 0u : (uint32_t)(((uint64_t)kWB << 32) / range));
-        for (uint32_t i = lane; i <= m; i += kWave) {  // buckets (bucket(U_{i-1}), bucket(U_i)] start at i
-            const uint32_t bi = i < m ? B.bucket(U[i]) : kWB;
-            for (uint32_t b = i == 0 ? 0 : B.bucket(U[i - 1]) + 1; b <= bi; b++) bkt[b] = (uint8_t)i;
+    if constexpr (CLQ && N > 4) {
+        if (queue) {
+            const uint32_t nw = (m + 63) >> 6;
+            uint32_t k = 0;
+            auto drain = [&](uint32_t nq) {
+                wave_sync();
+                if (lane < nq) {
+                    const uint32_t e = queue[lane];
+                    uint32_t off[N];
+                    off[1] = (e >> 16) * W;
+                    off[2] = (e & 0xffffu) * W;
+                    nodes++;
+                    clique_walk<N, 3>(rows, W, nw, off, e & 0xffffu, lane_total, nodes);
+                }
+                wave_sync();
+            };
+            for (uint32_t r1 = 0; r1 < m; r1++) {
+                for (uint32_t w = r1 >> 6; w < nw; w++) {
+                    const uint64_t cw = uniform(rows[r1 * W + w]);
+                    const uint32_t cnt = (uint32_t)__popcll(cw);
+                    if (k + cnt > kWave) {
+                        drain(k);
+                        k = 0;
+                    }
+                    if ((cw >> lane) & 1) queue[k + lanes_below(cw)] = (r1 << 16) | (w * 64 + lane);
+                    k += cnt;
+                }
+            }
+            if (k) drain(k);
+            if (lane == 0) nodes += m;
+            return;
         }
-        wave_sync();
-        uint32_t big = 0;
-        for (uint32_t b = lane; b < kWB; b += kWave) big = umax32(big, bkt[b + 1] - bkt[b]);
-        big = (uint32_t)wave_max((uint64_t)big);
-        B.hb = 1;
-        while (B.hb * 2 <= big) B.hb *= 2;
-        B.bkt = bkt;
-    }
-    for (uint32_t a0 = 0; a0 + 1 < m; a0 += kWave) {
-        uint32_t unused = 0;
-        build_chunk<CLQ ? 1 : 0>(a, U, rows, m, W, a0, 0, unused, B);
-        wave_sync();  // (the chunk's atomics complete before the walk reads rows)
     }
     if constexpr (CLQ) {
         const uint32_t nw = (m + 63) >> 6;
@@ -498,9 +646,71 @@ __device__ __forceinline__ void local_root(const LocalArgs& a, uint64_t lo, uint
         for (uint32_t r1 = lane; r1 < m; r1 += kWave) {
             M[1] = r1;
             nodes++;
-            walk_from<N>(a.prog, M, 2, rows, W, m, lane_total, nodes);
+            walk_from<N>(P, M, 2, rows, W, m, lane_total, nodes);
         }
     }
+}
+
+// LDS of one wave of the first pass (triangles need no rows)
+template <bool ROWS>
+struct WaveLocal {
+    uint64_t rows[ROWS ? kLRowWords : 1];
+    uint32_t U[kLMembers + 2];
+    uint16_t next[kLMembers + 2];
+    __align__(8) uint16_t slot[kLSlots];  // (the count's queue after the build)
+};
+
+// One root in the wave's LDS.
+template <int N, bool CLQ>
+__device__ __forceinline__ void wave_root(const LocalArgs& a, uint64_t lo, uint32_t m, WaveLocal<!(CLQ && N == 3)>& L,
+                                          uint64_t& lane_total, uint64_t& nodes) {
+    constexpr bool kTri = CLQ && N == 3;
+    const uint32_t lane = lane_id();
+    const uint32_t W = row_stride(m);
+    const HashIndex<kLSlots> H{L.slot, L.next, L.U};
+    wave_sync();  // (the previous root's reads are done)
+    if constexpr (!kTri)
+        for (uint32_t i = lane; i < m * W; i += kWave) L.rows[i] = 0;
+    for (uint32_t i = lane; i < kLSlots / 4; i += kWave) reinterpret_cast<uint64_t*>(L.slot)[i] = 0;
+    wave_sync();
+    for (uint32_t i = lane; i < m; i += kWave) {
+        const uint32_t u = a.ocols[lo + i];
+        L.U[i] = u;
+        H.put(i, u);
+    }
+    wave_sync();
+    uint32_t hits = 0;
+    for (uint32_t i0 = 0; i0 + 1 < m; i0 += kWave)
+        build_rows<kVecsW>(a, H, m, lo, i0, 1, a.factor, [&](uint32_t ia, uint32_t ib) {
+            if constexpr (kTri) {
+                hits++;
+            } else {
+                set_row_bit(L.rows, ia * W + (ib >> 6), ib);
+                if constexpr (!CLQ) set_row_bit(L.rows, ib * W + (ia >> 6), ia);
+            }
+        });
+    if constexpr (kTri) {
+        lane_total += hits;
+        if (lane == 0) nodes += m;
+    } else {
+        wave_sync();  // (the rows' atomics complete before the walk reads them)
+        count_root<N, CLQ>(a.prog, m, L.rows, reinterpret_cast<uint32_t*>(L.slot), lane_total, nodes);
+    }
+}
+
+// One root whose rows lie in a global arena.
+template <int N, bool CLQ>
+__device__ __forceinline__ void arena_root(const LocalArgs& a, uint64_t lo, uint32_t m, uint64_t* rows, uint64_t& lane_total,
+                                           uint64_t& nodes) {
+    const uint32_t W = row_stride(m);
+    for (uint64_t i = lane_id(); i < (uint64_t)m * W; i += kWave) rows[i] = 0;
+    wave_sync();
+    for (uint32_t a0 = 0; a0 + 1 < m; a0 += kWave) {
+        uint32_t unused = 0;
+        build_chunk<CLQ ? 1 : 0>(a, a.ocols + lo, rows, m, W, a0, 0, unused);
+        wave_sync();  // (the chunk's atomics complete before the walk reads rows)
+    }
+    count_root<N, CLQ>(a.prog, m, rows, nullptr, lane_total, nodes);
 }
 
 // put root x on the deferred list of the next pass
@@ -514,54 +724,66 @@ __device__ inline void defer_root(const LocalArgs& a, uint32_t x, uint64_t need)
     }
 }
 
-// Pass 1 (big_list set): roots whose rows fit the wave's LDS; the others are
-// deferred.  Pass 3 (big_list null): the roots too large for a block's LDS,
-// rows in per-wave global arenas of scratch_words.
+// Pass 1: roots whose rows fit the wave's LDS; the others are deferred.
+// Roots are taken from the top rank down: the roots with the largest local
+// graphs sit in the upper middle of the (degree, id) order and the low ranks
+// are the cheapest, so the pass ends on short roots instead of on a tail of
+// long ones (14.5 -> 13.7 ms on R-MAT 22, 4-cliques).  They come from 16
+// counters, a.run at a time: one by one where the waves get few (a run of 8
+// left R-MAT 10's 880 roots to 110 waves), up to 8 where there are millions.
 template <int N, bool CLQ>
-__global__ __launch_bounds__(256, (N <= 4 ? 8 : 4)) void gm_local_kernel(LocalArgs a) {
-    __shared__ uint64_t lrows[kLocalBlockWaves][kLRowWords];
-    __shared__ uint32_t lU[kLocalBlockWaves][kLU];
-    __shared__ uint8_t lB[kLocalBlockWaves][kWB + 4];
+__global__ __launch_bounds__(256, 7) void gm_local_kernel(LocalArgs a) {
+    __shared__ WaveLocal<!(CLQ && N == 3)> lds[kLocalBlockWaves];
     const uint32_t lane = lane_id();
     const uint32_t wid = threadIdx.x / kWave;
     const uint64_t gwave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + wid;
-    uint64_t* ws = a.scratch + gwave * a.scratch_words;
     uint64_t lane_total = 0, nodes = 0;
-
-    // roots come in runs of kFetchRun from the counter in the first pass (most
-    // of them are trivial, and one atomic per root would queue the waves on
-    // the counter), singly in the third (few, heavy roots).  The first pass
-    // takes its roots from the top rank down: the roots with the largest
-    // local graphs sit in the upper middle of the (degree, id) order and the
-    // low ranks are the cheapest, so the pass ends on short roots instead of
-    // on a tail of long ones (14.5 -> 13.7 ms on R-MAT 22, 4-cliques).
-    const uint32_t run = a.big_list ? kFetchRun : 1;
-    uint64_t t = 0, tend = 0;
+    const uint64_t total = (a.ntasks + a.run - 1) / a.run;
+    uint32_t queue = (uint32_t)(gwave % kQueues);
     while (true) {
-        if (t == tend) {
-            t = fetch_tasks(&a.ctr[LCTR_NEXT], run);
-            tend = umin64(t + run, a.ntasks);
-        }
-        if (t >= a.ntasks) break;
-        const uint64_t tt = a.big_list ? a.ntasks - 1 - t : t;
-        const uint32_t x = uniform(a.list ? a.list[tt] : (uint32_t)tt);
-        t++;
-        const uint64_t lo = uniform(a.orp[x]);
-        const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
-        if (m < (uint32_t)(N - 1)) continue;
-        if constexpr (N == 2) {
-            if (lane == 0) lane_total += m;
-            continue;
-        } else {
-            const uint64_t need = local_need(m);
-            if (m <= kLU && need <= kLRowWords) {
-                local_root<N, CLQ>(a, lo, m, lrows[wid], lU[wid], lU[wid], lB[wid], lane_total, nodes);
-            } else if (!a.big_list && need <= a.scratch_words) {
-                local_root<N, CLQ>(a, lo, m, ws, a.ocols + lo, nullptr, nullptr, lane_total, nodes);
-            } else if (lane == 0) {
-                defer_root(a, x, need);
+        const uint64_t b = queue_next(a.ctr + LCTR_QUEUE, queue, total);
+        if (b == kNoTask) break;
+        const uint64_t tend = umin64((b + 1) * a.run, a.ntasks);
+        for (uint64_t t = b * a.run; t < tend; t++) {
+            const uint64_t tt = a.ntasks - 1 - t;
+            const uint32_t x = uniform(a.list ? a.list[tt] : (uint32_t)tt);
+            const uint64_t lo = uniform(a.orp[x]);
+            const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
+            if (m < (uint32_t)(N - 1)) continue;
+            if constexpr (N == 2) {
+                if (lane == 0) lane_total += m;
+            } else {
+                const uint64_t need = local_need(m);
+                if (m <= kLU && need <= kLRowWords) wave_root<N, CLQ>(a, lo, m, lds[wid], lane_total, nodes);
+                else if (lane == 0) defer_root(a, x, need);
             }
         }
+    }
+    const uint64_t tot = wave_sum(lane_total);
+    const uint64_t nd = wave_sum(nodes);
+    if (lane == 0) {
+        if (tot) atomicAdd(&a.ctr[LCTR_COUNT], (unsigned long long)tot);
+        if (nd) atomicAdd(&a.ctr[LCTR_NODES], (unsigned long long)nd);
+    }
+}
+
+// Last pass: the roots too large for a workgroup's LDS, rows in per-wave
+// global arenas of scratch_words.
+template <int N, bool CLQ>
+__global__ __launch_bounds__(256, 4) void gm_local_arena_kernel(LocalArgs a) {
+    const uint32_t lane = lane_id();
+    const uint64_t gwave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
+    uint64_t* ws = a.scratch + gwave * a.scratch_words;
+    uint64_t lane_total = 0, nodes = 0;
+    while (true) {
+        const uint64_t t = fetch_task(&a.ctr[LCTR_NEXT]);
+        if (t >= a.ntasks) break;
+        const uint32_t x = uniform(a.list[t]);
+        const uint64_t lo = uniform(a.orp[x]);
+        const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
+        const uint64_t need = local_need(m);
+        if (need <= a.scratch_words) arena_root<N, CLQ>(a, lo, m, ws, lane_total, nodes);
+        else if (lane == 0) defer_root(a, x, need);
     }
     const uint64_t tot = wave_sum(lane_total);
     const uint64_t nd = wave_sum(nodes);
@@ -576,32 +798,34 @@ __global__ __launch_bounds__(256, (N <= 4 ? 8 : 4)) void gm_local_kernel(LocalAr
 // next pass.  Three shapes run in turn: 256 threads with 25 KB of rows (four
 // workgroups per CU, |U| <= 448), 512 threads with 60 KB (two per CU, |U| <=
 // 700), then 1024 threads with 138 KB (one per CU).
-// The build is one work list over all members and threads; then waves take
-// position-1 candidates r1 one at a time from an LDS counter, a wave's lanes
-// share the position-2 candidates of its r1, queued 64 at a time in LDS, and
-// each lane walks the rest of its (r1, r2) subtree.
-template <int N, bool CLQ, int BT, int ROWW, int BU, int NB>
+// Build: member i's row is one wave's work (wave i mod waves), cut into pieces
+// of 64 entries, kVecs pieces (of one or several members) in flight.  Which
+// member a piece belongs to is a scalar, and an entry is looked up by one LDS
+// read of its hash slot, a second only where the tag agrees (the members
+// themselves and 1 in 16 of the others).  Rows average ~400 entries on R-MAT
+// 22, of which 8% are hits.
+// Count: waves take position-1 candidates r1 one at a time from an LDS
+// counter, a wave's lanes share the position-2 candidates of its r1, queued 64
+// at a time in LDS, and each lane walks the rest of its (r1, r2) subtree.
+// Triangles (CLQ, N = 3) are the build's hits: no rows, no count.
+template <int N, bool CLQ, int BT, int ROWW, int BU>
 __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
     constexpr int kWaves = BT / kWave;
-    constexpr int kMembersPerThread = (BU + BT - 1) / BT;
-    __shared__ uint64_t rows[ROWW];
+    constexpr bool kTri = CLQ && N == 3;
+    __shared__ uint64_t rows[kTri ? 1 : ROWW];
     __shared__ uint32_t U[BU];
-    __shared__ uint32_t mpref[BU];   // members' first work item
-    __shared__ uint32_t mstart[BU];  // members' first entry in ocols
-    __shared__ uint32_t mcode[BU];   // members' entry count | kRev
-    __shared__ uint32_t wsum[kWaves];
+    __shared__ uint16_t next[BU];
     __shared__ unsigned long long s_task;
-    __shared__ uint32_t s_next, s_maxb;
-    // the build's value-bucket index (first index of U in each bucket) and the
-    // count's per-wave candidate queues share one buffer: a barrier separates
-    // the build from the count, and the next root's index from this count
-    constexpr int kQueueBytes = kWaves * kWave * 4, kBucketBytes = (NB + 1) * 2;
-    __shared__ __align__(16) uint8_t qb_raw[kQueueBytes > kBucketBytes ? kQueueBytes : kBucketBytes];
-    auto queue = reinterpret_cast<uint32_t (*)[kWave]>(qb_raw);
-    uint16_t* const ubkt = reinterpret_cast<uint16_t*>(qb_raw);
+    __shared__ uint32_t s_next;
+    // the build's hash slots and the count's per-wave candidate queues share
+    // one buffer: a barrier separates the build from the count, and the next
+    // root's slots from this count
+    __shared__ __align__(16) uint16_t slot[kSlots];
+    static_assert(kWaves * kWave * 4 <= (int)sizeof(slot), "queues fit the slots");
+    auto queue = reinterpret_cast<uint32_t (*)[kWave]>(slot);
+    const HashIndex<kSlots> H{slot, next, U};
     const uint32_t lane = lane_id();
-    const uint32_t wid = threadIdx.x / kWave;
-    const uint32_t nwaves = blockDim.x / kWave;
+    const uint32_t wid = uniform(threadIdx.x / kWave);
     const uint32_t tid = threadIdx.x;
     const LocalProgram& P = a.prog;
     uint64_t lane_total = 0, nodes = 0;
@@ -612,12 +836,13 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
             s_task = atomicAdd(&a.ctr[LCTR_NEXT], 1ull);
             s_next = 0;
         }
+        for (uint32_t i = tid; i < kSlots / 2; i += BT) reinterpret_cast<uint32_t*>(slot)[i] = 0;
         __syncthreads();
-        const uint64_t t = s_task;
+        const uint64_t t = uniform((uint64_t)s_task);
         if (t >= a.ntasks) break;
-        const uint32_t x = a.list[t];
-        const uint64_t lo = a.orp[x];
-        const uint32_t m = (uint32_t)(a.orp[x + 1] - lo);
+        const uint32_t x = uniform(a.list[t]);
+        const uint64_t lo = uniform(a.orp[x]);
+        const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
         const uint32_t W = row_stride(m);
         const uint64_t need = local_need(m);
         if (m < (uint32_t)(N - 1)) continue;
@@ -625,206 +850,28 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
             if (threadIdx.x == 0) defer_root(a, x, need);
             continue;
         }
-        for (uint32_t i = tid; i < need; i += blockDim.x) rows[i] = 0;
-        for (uint32_t i = tid; i < m; i += blockDim.x) U[i] = a.ocols[lo + i];
-        if (tid == 0) s_maxb = 0;
-        __syncthreads();
-        // value buckets over [U_0, U_{m-1}]: a lookup searches one bucket
-        const uint32_t ulo = U[0];
-        // bucket(v) = floor((v - ulo) * NB / range) by one 32-bit high multiply
-        // (the identity when U spans at most NB ranks); monotone, and below NB
-        // on [ulo, U_{m-1}]
-        const uint32_t range = U[m - 1] - ulo + 1;
-        // (uniform values made opaque to the compiler: it would otherwise
-        // widen the high multiply to 64 bits)
-        const uint32_t imask = __builtin_amdgcn_readfirstlane(range <= (uint32_t)NB ? ~0u : 0u);
-        const uint32_t bmul =
-            __builtin_amdgcn_readfirstlane(range <= (uint32_t)NB ? 0u : (uint32_t)(((uint64_t)NB << 32) / range));
-        auto bucket = [&](uint32_t v) {
-            const uint32_t d = v - ulo;
-            return __umulhi(d, bmul) + (d & imask);
-        };
-        for (uint32_t i = tid; i <= m; i += blockDim.x) {  // buckets (bucket(U_{i-1}), bucket(U_i)] start at i
-            const uint32_t bi = i < m ? bucket(U[i]) : NB;
-            for (uint32_t b = i == 0 ? 0 : bucket(U[i - 1]) + 1; b <= bi; b++) ubkt[b] = (uint16_t)i;
+        if constexpr (!kTri)
+            for (uint32_t i = tid; i < need; i += BT) rows[i] = 0;
+        for (uint32_t i = tid; i < m; i += BT) {
+            const uint32_t u = a.ocols[lo + i];
+            U[i] = u;
+            H.put(i, u);
         }
         __syncthreads();
-        {
-            uint32_t big = 0;
-            for (uint32_t b = tid; b < NB; b += blockDim.x) big = umax32(big, ubkt[b + 1] - ubkt[b]);
-            big = (uint32_t)wave_max((uint64_t)big);
-            if (lane == 0 && big) atomicMax(&s_maxb, big);
-        }
-        // ---- local rows: one work list over all members and threads ---------
-        // member i < m-1 has either n entries of N+(U_i) (restricted to
-        // [U_{i+1}, U_{m-1}]) to look up in U (LDS), or, when n exceeds
-        // (m-1-i) x (1 + log2 n), its m-1-i later members to look up in
-        // N+(U_i) (global).
-        // Thread t describes members t, t + BT, ...; their item counts go to
-        // mpref, which a block scan then turns into first items.
-#pragma unroll
-        for (int h = 0; h < kMembersPerThread; h++) {
-            const uint32_t i = tid + h * BT;
-            if (i + 1 < m) {
-                const uint32_t u = U[i];
-                uint64_t e0 = a.orp[u], e1 = a.orp[u + 1];
-                if (e1 - e0 > kWave) lower_bound2(a.ocols, e0, e1, U[i + 1], U[m - 1] + 1, &e0, &e1);
-                const uint64_t n = e1 - e0, rem = m - 1 - i;
-                const bool rev = n > (1u << 20) || rem * (1 + bitlen(n)) < n;
-                mstart[i] = (uint32_t)e0;
-                mcode[i] = rev ? ((uint32_t)n | kRev) : (uint32_t)n;
-                mpref[i] = rev ? (uint32_t)rem : (uint32_t)n;
-            } else if (i < m) {
-                mpref[i] = 0;
-            }
-        }
-        __syncthreads();
-        uint32_t T = 0;
-        {  // exclusive scan of mpref[0..m) in member order, contiguous runs per thread
-            const uint32_t per = (m + BT - 1) / BT;
-            const uint32_t c0 = min(tid * per, m), c1 = min(c0 + per, m);
-            uint32_t sum = 0;
-            for (uint32_t i = c0; i < c1; i++) sum += mpref[i];
-            uint32_t incl = sum;
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) {
-                const uint32_t y = __shfl_up(incl, o, kWave);
-                if (lane >= (uint32_t)o) incl += y;
-            }
-            if (lane == kWave - 1) wsum[wid] = incl;
-            __syncthreads();
-            uint32_t before = 0;
-            for (uint32_t q = 0; q < nwaves; q++) {
-                const uint32_t ws = wsum[q];
-                before += q < wid ? ws : 0;
-                T += ws;
-            }
-            uint32_t run = before + incl - sum;
-            for (uint32_t i = c0; i < c1; i++) {
-                const uint32_t l = mpref[i];
-                mpref[i] = run;
-                run += l;
-            }
-        }
-        __syncthreads();
-        const uint32_t nm = m - 1;  // members that own items
-        uint32_t hb_own = 1, hb_u = 1;  // highest powers of two <= nm-1 and <= the largest bucket
-        while (hb_own * 2 <= nm - 1) hb_own *= 2;
-        while (hb_u * 2 <= s_maxb) hb_u *= 2;
-        constexpr uint32_t kSlice = kItems * kWave;  // consecutive items per wave and round
-        for (uint32_t f0 = wid * kSlice; f0 < T; f0 += nwaves * kSlice) {
-            // the slice's first and last owners (wave-uniform searches, broadcast
-            // reads), then each lane searches only between them
-            const uint32_t flast = min(f0 + kSlice, T) - 1;
-            uint32_t o0 = 0, o1 = 0;
-            for (uint32_t step = hb_own; step >= 1; step >>= 1) {
-                if (o0 + step < nm && mpref[o0 + step] <= f0) o0 += step;
-                if (o1 + step < nm && mpref[o1 + step] <= flast) o1 += step;
-            }
-            o0 = __builtin_amdgcn_readfirstlane(o0);  // (wave-uniform: scalar from here)
-            o1 = __builtin_amdgcn_readfirstlane(o1);
-            uint32_t hb_r = 1;
-            while (hb_r * 2 <= o1 - o0) hb_r *= 2;
-            uint32_t f[kItems], own[kItems], w[kItems], pos[kItems];
-#pragma unroll
-            for (int q = 0; q < kItems; q++) {
-                f[q] = f0 + q * kWave + lane;
-                own[q] = o0;
-            }
-            if (o1 > o0 && o1 - o0 <= kOwnScan) {
-                // few owners: count the member starts at or below each item,
-                // each start read once per slice as a scalar
-                for (uint32_t o = o0 + 1; o <= o1; o++) {
-                    const uint32_t po = __builtin_amdgcn_readfirstlane(mpref[o]);
-#pragma unroll
-                    for (int q = 0; q < kItems; q++) own[q] += po <= f[q] ? 1u : 0u;
-                }
-            } else if (o1 > o0) {
-                for (uint32_t step = hb_r; step >= 1; step >>= 1) {
-#pragma unroll
-                    for (int q = 0; q < kItems; q++) {
-                        const uint32_t c = own[q] + step;
-                        if (c <= o1 && mpref[c] <= f[q]) own[q] = c;
-                    }
-                }
-            }
-            // w: the entry to look up in U, or for a reversed member the later
-            // member to look up in the member's row (rlen > 0: that row's length)
-            uint32_t rst[kItems], rlen[kItems], rmax = 0;
-            // every lane loads both candidates of all its items before any is
-            // used (no branch around a load, so no lane waits on a load that
-            // another path issued): a reversed member's row is longer than its
-            // later-member count, so rst + item stays inside it, and an invalid
-            // lane reads the root's own row
-#pragma unroll
-            for (int q = 0; q < kItems; q++) {
-                const uint32_t o = own[q], code = mcode[o], item = f[q] - mpref[o];
-                const bool valid = f[q] < T;
-                rst[q] = mstart[o];
-                rlen[q] = valid && (code & kRev) ? (code & ~kRev) : 0;
-                rmax = max(rmax, rlen[q]);
-                pos[q] = U[umin32(o + 1 + item, m - 1)];
-                w[q] = a.ocols[valid ? (uint64_t)rst[q] + item : lo];
-            }
-#pragma unroll
-            for (int q = 0; q < kItems; q++) w[q] = f[q] >= T ? ulo : rlen[q] ? pos[q] : w[q];
-            uint32_t lim[kItems];
-#pragma unroll
-            for (int q = 0; q < kItems; q++) {  // (an entry above U_{m-1} lands in the last bucket and misses)
-                const uint32_t b = umin32(bucket(w[q]), NB - 1);
-                pos[q] = ubkt[b];
-                lim[q] = ubkt[b + 1];
-            }
-            for (uint32_t step = hb_u; step >= 1; step >>= 1) {  // pos = |{U_j < w}|, within w's bucket
-#pragma unroll
-                for (int q = 0; q < kItems; q++) {
-                    const uint32_t c = pos[q] + step;
-                    if (c <= lim[q] && U[c - 1] < w[q]) pos[q] = c;
-                }
-            }
-            // reversed members: rpos = |{entries <= w}| in the member's row, the
-            // entry at rpos-1 kept; the items' searches interleave step by step
-            // so their global loads overlap
-            uint32_t rpos[kItems], last[kItems];
-#pragma unroll
-            for (int q = 0; q < kItems; q++) {
-                rpos[q] = 0;
-                last[q] = ~0u;
-            }
-            uint32_t rstep = 1;
-            while (rstep * 2 <= rmax) rstep *= 2;
-            for (uint32_t step = rmax ? rstep : 0; step >= 1; step >>= 1) {
-#pragma unroll
-                for (int q = 0; q < kItems; q++) {
-                    const uint32_t c = rpos[q] + step;
-                    if (c <= rlen[q]) {
-                        const uint32_t v = a.ocols[(uint64_t)rst[q] + c - 1];
-                        if (v <= w[q]) {
-                            rpos[q] = c;
-                            last[q] = v;
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < kItems; q++) {
-                if (f[q] >= T) continue;
-                const uint32_t ia = own[q];
-                uint32_t ib;
-                bool hit;
-                if (rlen[q]) {
-                    ib = ia + 1 + (f[q] - mpref[ia]);
-                    hit = last[q] == w[q];
-                } else {
-                    ib = pos[q];
-                    hit = ib < m && U[ib] == w[q];
-                }
-                if (hit) {  // (row offsets within the LDS rows fit 32 bits)
+        uint32_t hits = 0;
+        for (uint32_t i0 = wid; i0 + 1 < m; i0 += kWaves * kWave)
+            build_rows<kVecs>(a, H, m, lo, i0, kWaves, kRevFactor, [&](uint32_t ia, uint32_t ib) {
+                if constexpr (kTri) {
+                    hits++;
+                } else {  // (row offsets within the LDS rows fit 32 bits)
                     set_row_bit(rows, ia * W + (ib >> 6), ib);
-                    if constexpr (!CLQ)
-                        set_row_bit(rows, ib * W + (ia >> 6), ia);
+                    if constexpr (!CLQ) set_row_bit(rows, ib * W + (ia >> 6), ia);
                 }
-            }
+            });
+        if constexpr (kTri) {
+            lane_total += hits;
+            if (tid == 0) nodes += m;
+            continue;
         }
         __syncthreads();
 
@@ -1182,7 +1229,7 @@ __global__ __launch_bounds__(256) void tri_kernel(LocalArgs a) {
             U = lU[wid];
         }
         uint32_t hits = 0;
-        for (uint32_t a0 = 0; a0 + 1 < m; a0 += kWave) build_chunk<2>(a, U, nullptr, m, 0, a0, lo, hits, UBuckets{});
+        for (uint32_t a0 = 0; a0 + 1 < m; a0 += kWave) build_chunk<2>(a, U, nullptr, m, 0, a0, lo, hits);
         const uint64_t tot = wave_sum((uint64_t)hits);
         if (lane == 0 && tot) atomicAdd(&a.tri[x], (unsigned long long)tot);
     }
@@ -1321,23 +1368,26 @@ void gm_local_compile(g2_ctx* c, const g2_plan* p) {
     c->local_ok = true;
 }
 
-enum class LocalPass { Wave, Group256, Group512, Group1024 };
+enum class LocalPass { Wave, Group256, Group512, Group1024, Arena };
 
 template <int N, bool CLQ>
 static void launch_local(LocalPass pass, uint64_t blocks, uint32_t bw, hipStream_t s, const LocalArgs& a) {
     if constexpr (N > 2) {
         switch (pass) {
             case LocalPass::Group256:
-                hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB1Threads, kB1RowWords, kB1U, kB1Buckets>), dim3(blocks),
+                hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB1Threads, kB1RowWords, kB1U>), dim3(blocks),
                                    dim3(kB1Threads), 0, s, a);
                 return;
             case LocalPass::Group512:
-                hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB2Threads, kB2RowWords, kB2U, kB2Buckets>), dim3(blocks),
+                hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB2Threads, kB2RowWords, kB2U>), dim3(blocks),
                                    dim3(kB2Threads), 0, s, a);
                 return;
             case LocalPass::Group1024:
-                hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB3Threads, kB3RowWords, kB3U, kB3Buckets>), dim3(blocks),
+                hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB3Threads, kB3RowWords, kB3U>), dim3(blocks),
                                    dim3(kB3Threads), 0, s, a);
+                return;
+            case LocalPass::Arena:
+                hipLaunchKernelGGL((gm_local_arena_kernel<N, CLQ>), dim3(blocks), dim3(bw * kWave), 0, s, a);
                 return;
             default:
                 break;
@@ -1399,7 +1449,7 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
         }
         return hipGetLastError();
     };
-    unsigned long long h[LCTR_N];
+    unsigned long long h[LCTR_HOST];
     double pass_ms[5] = {0, 0, 0, 0, 0};
     int pass_no = 0;
     auto timed = [&](LocalPass pass, uint64_t blocks) -> int {
@@ -1418,6 +1468,8 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     // pass 1: every root, rows in the wave's LDS
     a.list = all ? nullptr : (const uint32_t*)c->roots.ptr;
     a.ntasks = nroots;
+    a.run = (uint32_t)std::min<uint64_t>(kFetchRun, std::max<uint64_t>(1, nroots / (nblocks * bw * 16)));
+    a.factor = c->ne * 2 > kNearBytes ? kRevFactorFar : kRevFactor;  // (ne / 2 oriented entries of 4 bytes)
     a.scratch = nullptr;
     a.scratch_words = 0;
     a.big_list = lists[0];
@@ -1454,7 +1506,7 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
         a.scratch = (uint64_t*)c->big_scratch.ptr;
         a.scratch_words = need;
         a.big_list = nullptr;
-        if ((rc = timed(LocalPass::Wave, bwaves / bw))) return rc;
+        if ((rc = timed(LocalPass::Arena, bwaves / bw))) return rc;
         launches++;
         pass_roots[4] = n;
     }
