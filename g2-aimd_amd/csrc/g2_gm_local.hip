@@ -60,17 +60,19 @@
 
 namespace g2 {
 
-// counters: next task, matches, nodes, (deferred roots, their largest need)
-// per pass, largest need that fit no arena
-// (copied back to the host), then the first pass's task queues (queue_next)
-enum { LCTR_NEXT = 0, LCTR_COUNT, LCTR_NODES, LCTR_DEFER, LCTR_ERR = LCTR_DEFER + 8, LCTR_HOST, LCTR_QUEUE = 16,
-       LCTR_N = LCTR_QUEUE + kQueues * kQueueStride };
+// counters: matches, nodes, next task of every pass (copied back to the host),
+// modelled bytes per pass (the accounting run), then the first pass's task
+// queues (queue_next)
+constexpr int kPasses = 5;
+enum { LCTR_COUNT = 0, LCTR_NODES, LCTR_NEXT, LCTR_BYTES = LCTR_NEXT + kPasses, LCTR_HOST = LCTR_BYTES + kPasses,
+       LCTR_QUEUE = 16, LCTR_N = LCTR_QUEUE + kQueues * kQueueStride };
 static_assert(LCTR_HOST <= LCTR_QUEUE, "counters");
 
 constexpr int kLocalBlockWaves = 4;     // gm_local_kernel: __launch_bounds__(256)
 constexpr uint32_t kLRowWords = 448;    // per-wave LDS rows (u64 words)
 constexpr uint32_t kLU = 256;           // |U| limit of a wave (triangle features; rows allow kLMembers)
 constexpr uint32_t kLMembers = 149;     // members of a root whose rows fit kLRowWords
+constexpr uint32_t kLMemberRegs = (kLMembers + 63) / 64;
 constexpr uint32_t kLSlots = 512;       // hash slots over U, per wave
 // workgroup passes: threads, LDS row words, |U| limit, and workgroups per CU
 // (the LDS each takes allows no more)
@@ -92,15 +94,14 @@ constexpr uint32_t kFetchRun = 8;       // roots per fetch in the first pass, wh
 struct LocalArgs {
     const uint64_t* __restrict__ orp;   // oriented rows over ranks
     const uint32_t* __restrict__ ocols;
-    const uint32_t* __restrict__ list;  // roots of the large-root pass (nullable: roots = [0, ntasks))
+    const uint32_t* __restrict__ list;  // the pass's roots (null: every rank)
     uint64_t ntasks;
     LocalProgram prog;
     uint32_t run;                       // first pass: roots per fetch,
     uint32_t factor;                    //   and build_rows' factor
     uint64_t* scratch;
     uint64_t scratch_words;
-    uint32_t* big_list;                 // deferred roots (null in the last pass)
-    uint32_t defer_ctr;                 // LCTR_DEFER + 2 * pass: count of big_list, need next to it
+    uint32_t pass;
     unsigned long long* ctr;
     unsigned long long* tri;            // triangle features: count per rank
     uint8_t* flag;                      // triangle features: flag per oriented entry
@@ -660,7 +661,28 @@ struct WaveLocal {
     __align__(8) uint16_t slot[kLSlots];  // (the count's queue after the build)
 };
 
-// One root in the wave's LDS.
+// Members and their index of one root, from registers, and cleared rows.
+template <int N, bool CLQ>
+__device__ __forceinline__ void wave_index(uint32_t m, const uint32_t* u, WaveLocal<!(CLQ && N == 3)>& L) {
+    const uint32_t lane = lane_id();
+    const HashIndex<kLSlots> H{L.slot, L.next, L.U};
+    wave_sync();  // (the previous root's reads are done)
+    if constexpr (!(CLQ && N == 3))
+        for (uint32_t i = lane; i < m * row_stride(m); i += kWave) L.rows[i] = 0;
+    for (uint32_t i = lane; i < kLSlots / 4; i += kWave) reinterpret_cast<uint64_t*>(L.slot)[i] = 0;
+    wave_sync();
+#pragma unroll
+    for (uint32_t h = 0; h < kLMemberRegs; h++) {
+        const uint32_t i = h * kWave + lane;
+        if (i < m) {
+            L.U[i] = u[h];
+            H.put(i, u[h]);
+        }
+    }
+    wave_sync();
+}
+
+// One root in the wave's LDS (wave_index has run).
 template <int N, bool CLQ>
 __device__ __forceinline__ void wave_root(const LocalArgs& a, uint64_t lo, uint32_t m, WaveLocal<!(CLQ && N == 3)>& L,
                                           uint64_t& lane_total, uint64_t& nodes) {
@@ -668,17 +690,6 @@ __device__ __forceinline__ void wave_root(const LocalArgs& a, uint64_t lo, uint3
     const uint32_t lane = lane_id();
     const uint32_t W = row_stride(m);
     const HashIndex<kLSlots> H{L.slot, L.next, L.U};
-    wave_sync();  // (the previous root's reads are done)
-    if constexpr (!kTri)
-        for (uint32_t i = lane; i < m * W; i += kWave) L.rows[i] = 0;
-    for (uint32_t i = lane; i < kLSlots / 4; i += kWave) reinterpret_cast<uint64_t*>(L.slot)[i] = 0;
-    wave_sync();
-    for (uint32_t i = lane; i < m; i += kWave) {
-        const uint32_t u = a.ocols[lo + i];
-        L.U[i] = u;
-        H.put(i, u);
-    }
-    wave_sync();
     uint32_t hits = 0;
     for (uint32_t i0 = 0; i0 + 1 < m; i0 += kWave)
         build_rows<kVecsW>(a, H, m, lo, i0, 1, a.factor, [&](uint32_t ia, uint32_t ib) {
@@ -713,24 +724,15 @@ __device__ __forceinline__ void arena_root(const LocalArgs& a, uint64_t lo, uint
     count_root<N, CLQ>(a.prog, m, rows, nullptr, lane_total, nodes);
 }
 
-// put root x on the deferred list of the next pass
-__device__ inline void defer_root(const LocalArgs& a, uint32_t x, uint64_t need) {
-    if (a.big_list) {
-        const unsigned long long idx = atomicAdd(&a.ctr[a.defer_ctr], 1ull);
-        a.big_list[idx] = x;
-        atomicMax(&a.ctr[a.defer_ctr + 1], (unsigned long long)need);
-    } else {
-        atomicMax(&a.ctr[LCTR_ERR], (unsigned long long)need);
-    }
-}
-
-// Pass 1: roots whose rows fit the wave's LDS; the others are deferred.
-// Roots are taken from the top rank down: the roots with the largest local
-// graphs sit in the upper middle of the (degree, id) order and the low ranks
-// are the cheapest, so the pass ends on short roots instead of on a tail of
-// long ones (14.5 -> 13.7 ms on R-MAT 22, 4-cliques).  They come from 16
-// counters, a.run at a time: one by one where the waves get few (a run of 8
-// left R-MAT 10's 880 roots to 110 waves), up to 8 where there are millions.
+// Pass 1: roots whose rows fit the wave's LDS (the others are passed over:
+// they are on the other passes' lists).  Roots are taken from the top rank
+// down: the roots with the largest local graphs sit in the upper middle of the
+// (degree, id) order and the low ranks are the cheapest, so the pass ends on
+// short roots instead of on a tail of long ones (14.5 -> 13.7 ms on R-MAT 22,
+// 4-cliques).  They come from 16 counters, a.run at a time: one by one where
+// the waves get few (a run of 8 left R-MAT 10's 880 roots to 110 waves), up to
+// 8 where there are millions; a run's row offsets are then one load, and the
+// next root's members are on their way while this one's rows are built.
 template <int N, bool CLQ>
 __global__ __launch_bounds__(256, 7) void gm_local_kernel(LocalArgs a) {
     __shared__ WaveLocal<!(CLQ && N == 3)> lds[kLocalBlockWaves];
@@ -743,19 +745,38 @@ __global__ __launch_bounds__(256, 7) void gm_local_kernel(LocalArgs a) {
     while (true) {
         const uint64_t b = queue_next(a.ctr + LCTR_QUEUE, queue, total);
         if (b == kNoTask) break;
-        const uint64_t tend = umin64((b + 1) * a.run, a.ntasks);
-        for (uint64_t t = b * a.run; t < tend; t++) {
-            const uint64_t tt = a.ntasks - 1 - t;
-            const uint32_t x = uniform(a.list ? a.list[tt] : (uint32_t)tt);
-            const uint64_t lo = uniform(a.orp[x]);
-            const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
-            if (m < (uint32_t)(N - 1)) continue;
-            if constexpr (N == 2) {
-                if (lane == 0) lane_total += m;
-            } else {
-                const uint64_t need = local_need(m);
-                if (m <= kLU && need <= kLRowWords) wave_root<N, CLQ>(a, lo, m, lds[wid], lane_total, nodes);
-                else if (lane == 0) defer_root(a, x, need);
+        // lane l: the run's root l
+        uint64_t rlo = 0;
+        uint32_t rm = 0;
+        if (lane < a.run && b * a.run + lane < a.ntasks) {
+            const uint64_t t = a.ntasks - 1 - (b * a.run + lane);
+            const uint64_t x = a.list ? a.list[t] : t;
+            rlo = a.orp[x];
+            rm = (uint32_t)(a.orp[x + 1] - rlo);
+        }
+        if constexpr (N == 2) {
+            lane_total += rm;
+        } else {
+            const bool mine = rm >= (uint32_t)(N - 1) && rm <= kLU && local_need(rm) <= kLRowWords;
+            uint64_t todo = ballot(mine);
+            uint32_t u[kLMemberRegs];
+            uint64_t lo = 0;
+            uint32_t m = 0;
+            auto fetch = [&](uint32_t l) {  // root l's members, kWave per register
+                lo = read_lane(rlo, l);
+                m = read_lane(rm, l);
+#pragma unroll
+                for (uint32_t h = 0; h < kLMemberRegs; h++)
+                    if (h * kWave < m) u[h] = a.ocols[lo + umin32(h * kWave + lane, m - 1)];
+            };
+            if (todo) fetch((uint32_t)__builtin_ctzll(todo));
+            while (todo) {
+                todo &= todo - 1;
+                const uint64_t clo = lo;
+                const uint32_t cm = m;
+                wave_index<N, CLQ>(cm, u, lds[wid]);
+                if (todo) fetch((uint32_t)__builtin_ctzll(todo));
+                wave_root<N, CLQ>(a, clo, cm, lds[wid], lane_total, nodes);
             }
         }
     }
@@ -768,7 +789,7 @@ __global__ __launch_bounds__(256, 7) void gm_local_kernel(LocalArgs a) {
 }
 
 // Last pass: the roots too large for a workgroup's LDS, rows in per-wave
-// global arenas of scratch_words.
+// global arenas of scratch_words (the largest root's need).
 template <int N, bool CLQ>
 __global__ __launch_bounds__(256, 4) void gm_local_arena_kernel(LocalArgs a) {
     const uint32_t lane = lane_id();
@@ -776,14 +797,12 @@ __global__ __launch_bounds__(256, 4) void gm_local_arena_kernel(LocalArgs a) {
     uint64_t* ws = a.scratch + gwave * a.scratch_words;
     uint64_t lane_total = 0, nodes = 0;
     while (true) {
-        const uint64_t t = fetch_task(&a.ctr[LCTR_NEXT]);
+        const uint64_t t = fetch_task(&a.ctr[LCTR_NEXT + a.pass]);
         if (t >= a.ntasks) break;
         const uint32_t x = uniform(a.list[t]);
         const uint64_t lo = uniform(a.orp[x]);
         const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
-        const uint64_t need = local_need(m);
-        if (need <= a.scratch_words) arena_root<N, CLQ>(a, lo, m, ws, lane_total, nodes);
-        else if (lane == 0) defer_root(a, x, need);
+        arena_root<N, CLQ>(a, lo, m, ws, lane_total, nodes);
     }
     const uint64_t tot = wave_sum(lane_total);
     const uint64_t nd = wave_sum(nodes);
@@ -793,9 +812,8 @@ __global__ __launch_bounds__(256, 4) void gm_local_arena_kernel(LocalArgs a) {
     }
 }
 
-// Pass 2: one root per workgroup of BT threads, its rows in the workgroup's
-// LDS (up to ROWW words, |U| <= BU); roots beyond that are deferred to the
-// next pass.  Three shapes run in turn: 256 threads with 25 KB of rows (four
+// Passes 2 to 4: one root per workgroup of BT threads, its rows in the workgroup's
+// LDS (up to ROWW words, |U| <= BU).  Three shapes run in turn: 256 threads with 25 KB of rows (four
 // workgroups per CU, |U| <= 448), 512 threads with 60 KB (two per CU, |U| <=
 // 700), then 1024 threads with 138 KB (one per CU).
 // Build: member i's row is one wave's work (wave i mod waves), cut into pieces
@@ -833,7 +851,7 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
     while (true) {
         __syncthreads();  // every wave is done with the previous root's rows
         if (threadIdx.x == 0) {
-            s_task = atomicAdd(&a.ctr[LCTR_NEXT], 1ull);
+            s_task = atomicAdd(&a.ctr[LCTR_NEXT + a.pass], 1ull);
             s_next = 0;
         }
         for (uint32_t i = tid; i < kSlots / 2; i += BT) reinterpret_cast<uint32_t*>(slot)[i] = 0;
@@ -845,11 +863,6 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
         const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
         const uint32_t W = row_stride(m);
         const uint64_t need = local_need(m);
-        if (m < (uint32_t)(N - 1)) continue;
-        if (m > BU || need > ROWW) {
-            if (threadIdx.x == 0) defer_root(a, x, need);
-            continue;
-        }
         if constexpr (!kTri)
             for (uint32_t i = tid; i < need; i += BT) rows[i] = 0;
         for (uint32_t i = tid; i < m; i += BT) {
@@ -1132,6 +1145,46 @@ __global__ __launch_bounds__(256) void local_bytes_kernel(const uint64_t* __rest
             if (acc[k]) atomicAdd(&out[k], (unsigned long long)acc[k]);
 }
 
+// Roots of the passes after the first, by their member count: counted
+// (FILL = false), then listed pass after pass (FILL; the counts place the
+// lists).  A wave adds its roots of one pass with one atomic.
+struct PassRoots {
+    unsigned long long count[kPasses];  // per pass (the first is not listed)
+    unsigned long long need;            // largest row words of the last pass
+    unsigned long long filled[kPasses];
+};
+template <bool FILL>
+__global__ __launch_bounds__(256) void pass_roots_kernel(const uint64_t* __restrict__ orp, const uint32_t* __restrict__ roots,
+                                                         uint64_t nroots, PassRoots* p, uint32_t* list) {
+    const uint32_t lane = lane_id();
+    const uint64_t nw = (uint64_t)gridDim.x * blockDim.x / kWave;
+    uint64_t need = 0;
+    for (uint64_t b = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave; b * kWave < nroots; b += nw) {
+        // (from the top rank down: the passes start on their largest roots)
+        uint32_t x = 0;
+        int pass = 0;
+        if (b * kWave + lane < nroots) {
+            const uint64_t t = nroots - 1 - (b * kWave + lane);
+            x = roots ? roots[t] : (uint32_t)t;
+            const uint64_t m = orp[x + 1] - orp[x];
+            pass = local_pass_of(3, m);
+            if (pass == kPasses - 1) need = umax64(need, local_need(m));
+        }
+        uint64_t before = 0;
+        for (int k = 1; k < kPasses; k++) {
+            const uint64_t mask = ballot(pass == k);
+            const uint32_t cnt = (uint32_t)__popcll(mask);
+            if (cnt) {
+                const uint64_t base = fetch_tasks(FILL ? &p->filled[k] : &p->count[k], cnt);
+                if (FILL && pass == k) list[before + base + lanes_below(mask)] = x;
+            }
+            if (FILL) before += uniform((uint64_t)p->count[k]);
+        }
+    }
+    need = wave_max(need);
+    if (!FILL && lane == 0 && need) atomicMax(&p->need, (unsigned long long)need);
+}
+
 // Ranks of the sources: the roots of a view whose sources are a subset.
 __global__ __launch_bounds__(256) void oroot_kernel(const uint32_t* __restrict__ src, uint64_t ns,
                                                     const uint32_t* __restrict__ pi, uint32_t* __restrict__ roots) {
@@ -1396,10 +1449,45 @@ static void launch_local(LocalPass pass, uint64_t blocks, uint32_t bw, hipStream
     hipLaunchKernelGGL((gm_local_kernel<N, CLQ>), dim3(blocks), dim3(bw * kWave), 0, s, a);
 }
 
+// Lists of the roots of every pass after the first, built once per view and
+// kept with it (they depend on its rows only).
+static int pass_roots(g2_ctx* c, const uint64_t* orp, const uint32_t* rank, uint64_t nroots) {
+    if (c->pass_roots_valid) return G2_OK;
+    hipError_t e;
+    const bool all = c->sources_all;
+    const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>((nroots + 255) / 256, 8192));
+    if (!all && c->ns) {
+        hipLaunchKernelGGL(oroot_kernel, dim3(grid), dim3(256), 0, c->stream, (const uint32_t*)c->src.ptr, c->ns, rank,
+                           (uint32_t*)c->roots.ptr);
+        if ((e = hipGetLastError())) return hip_err(c, e, "root ranks");
+    }
+    for (auto& n : c->pass_count) n = 0;
+    c->pass_need = 0;
+    if (c->max_degree > kLMembers) {  // (no root has more members than neighbours)
+        const uint32_t* roots = all ? nullptr : (const uint32_t*)c->roots.ptr;
+        auto* p = (PassRoots*)c->big_list2.ptr;
+        auto* list = (uint32_t*)(p + 1);
+        PassRoots h{};
+        if ((e = hipMemsetAsync(p, 0, sizeof(h), c->stream))) return hip_err(c, e, "memset pass roots");
+        hipLaunchKernelGGL(pass_roots_kernel<false>, dim3(grid), dim3(256), 0, c->stream, orp, roots, nroots, p, list);
+        if ((e = hipGetLastError())) return hip_err(c, e, "pass roots launch");
+        if ((e = hipMemcpyAsync(&h, p, sizeof(h), hipMemcpyDeviceToHost, c->stream))) return hip_err(c, e, "D2H pass roots");
+        if ((e = hipStreamSynchronize(c->stream))) return hip_err(c, e, "pass roots sync");
+        uint64_t listed = 0;
+        for (int k = 1; k < kPasses; k++) listed += c->pass_count[k] = h.count[k];
+        c->pass_need = h.need;
+        if (listed)
+            hipLaunchKernelGGL(pass_roots_kernel<true>, dim3(grid), dim3(256), 0, c->stream, orp, roots, nroots, p, list);
+        if ((e = hipGetLastError())) return hip_err(c, e, "pass roots launch");
+    }
+    c->pass_roots_valid = true;
+    return G2_OK;
+}
+
 // Passes over the roots: rows in a wave's LDS; in a 256-, 512- and
 // 1024-thread workgroup's LDS; in per-wave global arenas sized to the largest
-// remaining root.  Each pass takes the roots the previous one deferred; the
-// deferred lists alternate between two buffers.
+// root left.  Which roots a pass takes is known before the first one starts,
+// so the passes are enqueued back to back and waited for once.
 int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     if (c->nv + 1 > 0x7fffffffull) return set_err(c, G2_EINVAL, "local-bitmap matching supports fewer than 2^31-1 vertices");
     const uint32_t bw = std::min<uint32_t>(c->tune.block_waves, kLocalBlockWaves);
@@ -1411,24 +1499,37 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     const uint64_t list_len = std::max<uint64_t>(nroots, 1);
     int rc;
     if ((rc = ensure(c, c->counters, LCTR_N * 8, "counters"))) return rc;
-    if ((rc = ensure(c, c->big_list2, list_len * 4, "deferred roots"))) return rc;
-    if ((rc = ensure(c, c->list, list_len * 4, "deferred roots"))) return rc;
-    if (!all && (rc = ensure(c, c->roots, list_len * 4, "root ranks"))) return rc;
+    if (!c->pass_roots_valid) {  // (a grown buffer loses its contents)
+        if ((rc = ensure(c, c->big_list2, sizeof(PassRoots) + list_len * 4, "pass roots"))) return rc;
+        if (!all && (rc = ensure(c, c->roots, list_len * 4, "root ranks"))) return rc;
+    }
     hipError_t e;
     auto* ctr = (unsigned long long*)c->counters.ptr;
-    uint32_t* lists[2] = {(uint32_t*)c->big_list2.ptr, (uint32_t*)c->list.ptr};
-    float tot = 0;
-    double kernel_ms = 0;
-    if ((e = hipEventRecord(c->ev[0], c->stream))) return hip_err(c, e, "event");
+    int nev = 0;
+    auto mark = [&]() -> int {
+        if ((e = hipEventRecord(c->ev[nev], c->stream))) return hip_err(c, e, "event");
+        nev++;
+        return G2_OK;
+    };
+    const bool first = !c->orient_valid || !c->pass_roots_valid;
+    if (first && (rc = mark())) return rc;
     const uint64_t* orp = nullptr;
     const uint32_t* ocols = nullptr;
     const uint32_t* pi = nullptr;
     if ((rc = build_oriented(c, &orp, &ocols, &pi))) return rc;
-    if (!all && c->ns) {
-        const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>((c->ns + 255) / 256, 8192));
-        hipLaunchKernelGGL(oroot_kernel, dim3(grid), dim3(256), 0, c->stream, (const uint32_t*)c->src.ptr, c->ns, pi,
-                           (uint32_t*)c->roots.ptr);
-        if ((e = hipGetLastError())) return hip_err(c, e, "root ranks");
+    if ((rc = pass_roots(c, orp, pi, nroots))) return rc;
+    const uint32_t n = c->lprog.n;
+    uint64_t roots[kPasses] = {nroots, 0, 0, 0, 0};
+    for (int k = 1; k < kPasses && n > 2; k++) {
+        roots[k] = c->pass_count[k];
+        roots[0] -= roots[k];
+    }
+    // last pass: per-wave global arenas
+    uint64_t bwaves = std::min<uint64_t>(std::max<uint32_t>(c->tune.big_waves, 1), roots[kPasses - 1]);
+    if (bwaves) {
+        while (bwaves > 1 && c->budget && c->used - c->big_scratch.bytes + bwaves * c->pass_need * 8 > c->budget) bwaves /= 2;
+        bwaves = (bwaves + bw - 1) / bw * bw;
+        if ((rc = ensure(c, c->big_scratch, bwaves * c->pass_need * 8, "large-root arenas"))) return rc;
     }
     if ((e = hipMemsetAsync(ctr, 0, LCTR_N * 8, c->stream))) return hip_err(c, e, "memset counters");
     LocalArgs a{};
@@ -1436,9 +1537,10 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     a.ocols = ocols;
     a.prog = c->lprog;
     a.ctr = ctr;
+    a.factor = c->ne * 2 > kNearBytes ? kRevFactorFar : kRevFactor;  // (ne / 2 oriented entries of 4 bytes)
     auto launch = [&](LocalPass pass, uint64_t blocks) {
         const bool clq = c->lprog.clique != 0;
-        switch (c->lprog.n) {
+        switch (n) {
             case 2: launch_local<2, false>(pass, blocks, bw, c->stream, a); break;
             case 3: clq ? launch_local<3, true>(pass, blocks, bw, c->stream, a) : launch_local<3, false>(pass, blocks, bw, c->stream, a); break;
             case 4: clq ? launch_local<4, true>(pass, blocks, bw, c->stream, a) : launch_local<4, false>(pass, blocks, bw, c->stream, a); break;
@@ -1449,100 +1551,68 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
         }
         return hipGetLastError();
     };
-    unsigned long long h[LCTR_HOST];
-    double pass_ms[5] = {0, 0, 0, 0, 0};
-    int pass_no = 0;
-    auto timed = [&](LocalPass pass, uint64_t blocks) -> int {
-        if ((e = hipMemsetAsync(ctr + LCTR_NEXT, 0, 8, c->stream))) return hip_err(c, e, "memset next");
-        if ((e = hipEventRecord(c->ev[1], c->stream))) return hip_err(c, e, "event");
-        if ((e = launch(pass, blocks))) return hip_err(c, e, "local launch");
-        if ((e = hipEventRecord(c->ev[2], c->stream))) return hip_err(c, e, "event");
-        if ((e = hipMemcpyAsync(h, ctr, sizeof(h), hipMemcpyDeviceToHost, c->stream))) return hip_err(c, e, "D2H counters");
-        if ((e = hipStreamSynchronize(c->stream))) return hip_err(c, e, "local sync");
-        float ms = 0;
-        (void)hipEventElapsedTime(&ms, c->ev[1], c->ev[2]);
-        kernel_ms += ms;
-        pass_ms[pass_no] = ms;
-        return G2_OK;
-    };
-    // pass 1: every root, rows in the wave's LDS
-    a.list = all ? nullptr : (const uint32_t*)c->roots.ptr;
-    a.ntasks = nroots;
-    a.run = (uint32_t)std::min<uint64_t>(kFetchRun, std::max<uint64_t>(1, nroots / (nblocks * bw * 16)));
-    a.factor = c->ne * 2 > kNearBytes ? kRevFactorFar : kRevFactor;  // (ne / 2 oriented entries of 4 bytes)
-    a.scratch = nullptr;
-    a.scratch_words = 0;
-    a.big_list = lists[0];
-    a.defer_ctr = LCTR_DEFER;
-    if ((rc = timed(LocalPass::Wave, nblocks))) return rc;
-    uint32_t launches = 1;
-    const uint64_t n1 = h[LCTR_DEFER];
-    uint64_t n = n1, need = h[LCTR_DEFER + 1];
-    uint64_t pass_roots[5] = {nroots - n1, 0, 0, 0, 0};
-    int in = 0;  // list holding the roots of the next pass
-    const struct { LocalPass pass; int per_cu; } groups[3] = {
-        {LocalPass::Group256, kB1PerCu}, {LocalPass::Group512, kB2PerCu}, {LocalPass::Group1024, kB3PerCu}};
-    for (int g = 0; g < 3 && n; g++) {  // workgroup passes
-        pass_no = g + 1;
-        a.list = lists[in];
-        a.ntasks = n;
-        a.big_list = lists[in ^ 1];
-        a.defer_ctr = LCTR_DEFER + 2 * (g + 1);
-        if ((rc = timed(groups[g].pass, std::min<uint64_t>((uint64_t)c->num_cus * groups[g].per_cu, n)))) return rc;
-        launches++;
-        pass_roots[g + 1] = n - h[a.defer_ctr];
-        n = h[a.defer_ctr];
-        need = h[a.defer_ctr + 1];
-        in ^= 1;
-    }
-    if (n) {  // last pass: per-wave global arenas
-        pass_no = 4;
-        uint64_t bwaves = std::min<uint64_t>(std::max<uint32_t>(c->tune.big_waves, 1), n);
-        while (bwaves > 1 && c->budget && c->used - c->big_scratch.bytes + bwaves * need * 8 > c->budget) bwaves /= 2;
-        bwaves = (bwaves + bw - 1) / bw * bw;
-        if ((rc = ensure(c, c->big_scratch, bwaves * need * 8, "large-root arenas"))) return rc;
-        a.list = lists[in];
-        a.ntasks = n;
+    const int ev0 = nev;
+    if ((rc = mark())) return rc;
+    const uint32_t* list = (const uint32_t*)((PassRoots*)c->big_list2.ptr + 1);
+    const struct { LocalPass pass; uint64_t most; } shape[kPasses] = {
+        {LocalPass::Wave, nblocks},
+        {LocalPass::Group256, (uint64_t)c->num_cus * kB1PerCu},
+        {LocalPass::Group512, (uint64_t)c->num_cus * kB2PerCu},
+        {LocalPass::Group1024, (uint64_t)c->num_cus * kB3PerCu},
+        {LocalPass::Arena, bwaves / bw}};
+    int pass_ev[kPasses] = {-1, -1, -1, -1, -1};
+    for (int k = 0; k < kPasses; k++) {
+        if (k && !roots[k]) continue;
+        a.pass = k;
+        if (k == 0) {  // every root, those of the other passes passed over
+            a.list = all ? nullptr : (const uint32_t*)c->roots.ptr;
+            a.ntasks = nroots;
+            a.run = (uint32_t)std::min<uint64_t>(kFetchRun, std::max<uint64_t>(1, nroots / (nblocks * bw * 16)));
+        } else {
+            a.list = list;
+            a.ntasks = roots[k];
+            list += roots[k];
+        }
         a.scratch = (uint64_t*)c->big_scratch.ptr;
-        a.scratch_words = need;
-        a.big_list = nullptr;
-        if ((rc = timed(LocalPass::Arena, bwaves / bw))) return rc;
-        launches++;
-        pass_roots[4] = n;
+        a.scratch_words = c->pass_need;
+        // (a workgroup takes one root at a time; a wave of the others up to a run)
+        const uint64_t blocks = k == kPasses - 1 ? shape[k].most : std::min<uint64_t>(shape[k].most, std::max<uint64_t>(a.ntasks, 1));
+        if ((e = launch(shape[k].pass, blocks))) return hip_err(c, e, "local launch");
+        pass_ev[k] = nev;
+        if ((rc = mark())) return rc;
     }
-    if ((e = hipEventRecord(c->ev[3], c->stream))) return hip_err(c, e, "event");
+    unsigned long long h[LCTR_HOST];
+    if ((e = hipMemcpyAsync(h, ctr, sizeof(h), hipMemcpyDeviceToHost, c->stream))) return hip_err(c, e, "D2H counters");
     if ((e = hipStreamSynchronize(c->stream))) return hip_err(c, e, "local sync");
-    (void)hipEventElapsedTime(&tot, c->ev[0], c->ev[3]);
-    if (h[LCTR_ERR]) return set_err(c, G2_EBUDGET, "a root did not fit the large-root arena");
-    unsigned long long pass_bytes[5] = {0, 0, 0, 0, 0};
     if (bytes) {  // accounting (untimed): the oriented rows each pass had to read
-        if ((e = hipMemsetAsync(ctr + LCTR_DEFER, 0, 5 * 8, c->stream))) return hip_err(c, e, "memset bytes");
         const uint64_t grid = std::max<uint64_t>(1, std::min<uint64_t>((nroots + 3) / 4, (uint64_t)c->num_cus * 32));
         hipLaunchKernelGGL(local_bytes_kernel, dim3(grid), dim3(256), 0, c->stream, orp, ocols,
-                           all ? nullptr : (const uint32_t*)c->roots.ptr, nroots, c->lprog.n, ctr + LCTR_DEFER);
+                           all ? nullptr : (const uint32_t*)c->roots.ptr, nroots, n, ctr + LCTR_BYTES);
         if ((e = hipGetLastError())) return hip_err(c, e, "local bytes launch");
-        if ((e = hipMemcpyAsync(pass_bytes, ctr + LCTR_DEFER, sizeof(pass_bytes), hipMemcpyDeviceToHost, c->stream)))
-            return hip_err(c, e, "D2H bytes");
+        if ((e = hipMemcpyAsync(h, ctr, sizeof(h), hipMemcpyDeviceToHost, c->stream))) return hip_err(c, e, "D2H bytes");
         if ((e = hipStreamSynchronize(c->stream))) return hip_err(c, e, "local bytes sync");
     }
     if (count) *count = h[LCTR_COUNT];
     if (st) {
-        st->kernel_ms = kernel_ms;
-        st->launches = launches;
+        for (int k = 0, prev = ev0; k < kPasses; k++) {
+            st->local_pass_roots[k] = roots[k];
+            st->local_pass_bytes[k] = h[LCTR_BYTES + k];
+            st->alg_bytes += h[LCTR_BYTES + k];
+            if (pass_ev[k] < 0) continue;
+            float ms = 0;
+            (void)hipEventElapsedTime(&ms, c->ev[prev], c->ev[pass_ev[k]]);
+            prev = pass_ev[k];
+            st->local_pass_ms[k] = ms;
+            st->kernel_ms += ms;
+            st->launches++;
+        }
+        float tot = 0;
+        (void)hipEventElapsedTime(&tot, c->ev[0], c->ev[nev - 1]);
         st->total_ms = tot;
         st->nodes = h[LCTR_NODES];
-        st->alg_bytes = 0;
-        for (int k = 0; k < 5; k++) {
-            st->alg_bytes += pass_bytes[k];
-            st->local_pass_bytes[k] = pass_bytes[k];
-            st->local_pass_ms[k] = pass_ms[k];
-        }
-        st->big_roots = n1;
-        st->max_scratch_words = need;
-        st->wave_idle_frac = 0;
-        st->donations = 0;
+        st->big_roots = nroots - roots[0];
+        st->max_scratch_words = c->pass_need;
         st->local_bitmap = 1;
-        for (int k = 0; k < 5; k++) st->local_pass_roots[k] = pass_roots[k];
     }
     return G2_OK;
 }

@@ -111,7 +111,7 @@ struct g2_ctx {
     uint64_t used = 0;
     g2_tuning tune{};
     hipStream_t stream = nullptr;
-    hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+    hipEvent_t ev[8] = {};
     std::string err;
 
     // view
@@ -146,7 +146,10 @@ struct g2_ctx {
     g2::GmWalk walk{};
     bool local_ok = false;        // the plan qualifies for the oriented local-bitmap path
     g2::LocalProgram lprog{};
-    g2::DevBuf big_list2;
+    g2::DevBuf big_list2;         // local-bitmap path: roots of every pass after the first
+    bool pass_roots_valid = false;  // big_list2, pass_count, pass_need and roots are the current view's
+    uint64_t pass_count[5] = {};
+    uint64_t pass_need = 0;       // row words of the last pass's largest root
     g2::DevBuf orient;            // oriented relabelled rows of the local-bitmap path
     bool orient_valid = false;    // orient holds the rows of the current view
     g2::DevBuf roots;             // local-bitmap path: ranks of the sources of a partial view
