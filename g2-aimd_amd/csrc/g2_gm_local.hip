@@ -47,8 +47,7 @@
 //      position is a popcount over the words its order range leaves.
 // The roots go through passes, each taking the roots the previous one
 // deferred: one wave per root with the rows in the wave's LDS (|U| <= 149);
-// one workgroup of 256, 512 or 1024 threads per root with the rows in the
-// workgroup's LDS (|U| <= 448, 700, 1039); one wave per root with the rows in
+// one workgroup per root with the rows in the workgroup's LDS (|U| <= 448, 700, 1039); one wave per root with the rows in
 // a global arena sized to the largest remaining root.
 #include <algorithm>
 #include <vector>
@@ -76,8 +75,8 @@ constexpr uint32_t kLMemberRegs = (kLMembers + 63) / 64;
 constexpr uint32_t kLSlots = 512;       // hash slots over U, per wave
 // workgroup passes: threads, LDS row words, |U| limit, and workgroups per CU
 // (the LDS each takes allows no more)
-constexpr int kB1Threads = 256, kB1RowWords = 3136, kB1U = 448, kB1PerCu = 4;     // 25 KiB rows: |U| 448 at stride 7
-constexpr int kB2Threads = 512, kB2RowWords = 7700, kB2U = 700, kB2PerCu = 2;     // 60 KiB rows: |U| 700 at stride 11
+constexpr int kB1Threads = 512, kB1RowWords = 3136, kB1U = 448, kB1PerCu = 4;     // 25 KiB rows: |U| 448 at stride 7
+constexpr int kB2Threads = 1024, kB2RowWords = 7700, kB2U = 700, kB2PerCu = 2;     // 60 KiB rows: |U| 700 at stride 11
 constexpr int kB3Threads = 1024, kB3RowWords = 17664, kB3U = 1040, kB3PerCu = 1;  // 138 KiB rows: |U| 1039 at stride 17
 constexpr uint32_t kRev = 0x80000000u;  // work-list flag: look the later members up in the row
 constexpr int kVecs = 8;                // 64-entry row pieces per wave in flight in the workgroup build
@@ -345,31 +344,38 @@ __device__ __forceinline__ void build_chunk(const LocalArgs& a, const uint32_t* 
 }
 
 // Hash index over U (in LDS): slot[rank mod T] holds the last member put
-// there, next[member] the one before it.  An entry is 0 (none) or member + 1
-// (11 bits) | 4 rank bits above the slot's (a mismatch is another rank) |
-// kChain when another member follows.
-constexpr uint32_t kChain = 0x8000u, kMember = 0x7ffu, kTag = 0x7800u;
-static_assert(kB3U < (int)kMember, "members fit an entry");
-template <uint32_t T>
+// there, next[member] the one before it.  An entry is 4 x member, the byte
+// offset into U (13 bits), with kChain set when another member follows; an
+// empty slot names member NONE, whose U is no rank, so that a lookup reads U
+// without a branch.
+constexpr uint32_t kChain = 0x8000u, kMember4 = 0x7ffcu;
+static_assert(kB3U * 4 <= (int)kMember4, "members fit an entry");
+template <uint32_t T, uint32_t NONE>
 struct HashIndex {
     uint16_t* slot;       // T
     uint16_t* next;       // |U|
-    const uint32_t* U;
-    static __device__ __forceinline__ uint32_t tag(uint32_t w) { return (w / T << 11) & kTag; }
+    uint32_t* U;          // NONE + 1
+    // clear the index: threads tid, tid + n, ..
+    __device__ __forceinline__ void clear(uint32_t tid, uint32_t n) const {
+        for (uint32_t i = tid; i < T / 4; i += n) reinterpret_cast<uint64_t*>(slot)[i] = NONE * 4 * 0x0001000100010001ull;
+        if (tid == 0) U[NONE] = ~0u;
+    }
     // put member i (rank u) at the head of its slot (a 16-bit half of a word)
     __device__ __forceinline__ void put(uint32_t i, uint32_t u) const {
+        U[i] = u;
         uint32_t* word = reinterpret_cast<uint32_t*>(slot) + ((u & (T - 1)) >> 1);
         const uint32_t sh = (u & 1) * 16;
         uint32_t old = *word;
         while (true) {
             const uint32_t head = (old >> sh) & 0xffffu;
             next[i] = (uint16_t)head;
-            const uint32_t e = (i + 1) | tag(u) | (head ? kChain : 0u);
+            const uint32_t e = i * 4 | (head != NONE * 4 ? kChain : 0u);
             const uint32_t seen = atomicCAS(word, old, (old & ~(0xffffu << sh)) | (e << sh));
             if (seen == old) break;
             old = seen;
         }
     }
+    __device__ __forceinline__ uint32_t member(uint32_t e) const { return (e & kMember4) >> 2; }
 };
 
 // Local rows of members i0, i0 + stride, .. (64 of them, one per lane) by one
@@ -377,7 +383,7 @@ struct HashIndex {
 // has either the n entries of N+(U_i) to look up in U, or, when n exceeds
 // (m-1-i) x factor, its m-1-i later members to look up in N+(U_i) (global
 // memory).  A lookup there is a chain of ~9 loads, a streamed entry a share of
-// one: factors of 5, 8, 12, 16 and 24 took the 256-thread pass of R-MAT 22 in
+// one: factors of 5, 8, 12, 16 and 24 took the second pass of R-MAT 22 in
 // 17.4, 16.3, 15.8, 16.2 and 16.5 ms.  In the first pass, with few members per
 // root, 12 is best where the rows stay in the last-level cache (R-MAT 20, 63
 // MB: 2.8 ms, 3.4 at 24), and 24 where they do not and a chain's loads come
@@ -385,12 +391,12 @@ struct HashIndex {
 // What bounds it: instruction issue and LDS reads per streamed entry (25.7 G
 // of them for R-MAT 22, 8% hits).  So a row is cut into pieces of 64 entries,
 // VECS of them (of one or several members) in flight, and everything about a
-// piece but its entries is a scalar; an entry costs one LDS read of its hash
-// slot, and a second only where the tag agrees (the members themselves and 1
-// in 16 of the others that meet one).  Rows average 150-310 entries on R-MAT
-// 18-20, so pieces are 85-90% full.
-template <int VECS, uint32_t T, class Hit>
-__device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T>& H, uint32_t m, uint64_t lo, uint32_t i0,
+// piece but its entries is a scalar (the row's address too); an entry costs
+// its hash slot and the member that slot names, both read without a branch (the
+// empty slots all read one word), ~13 vector instructions a piece with the hit.
+// Rows average 150-310 entries on R-MAT 18-20, so pieces are 85-90% full.
+template <int VECS, uint32_t T, uint32_t NONE, class Hit>
+__device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T, NONE>& H, uint32_t m, uint64_t lo, uint32_t i0,
                                            uint32_t stride, uint32_t factor, Hit hit) {
     const uint32_t lane = lane_id();
     const uint32_t mi = i0 + lane * stride;
@@ -420,32 +426,32 @@ __device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T
             }
             own[q] = ci;
             cnt[q] = umin32(left, kWave);
-            // (a lane past the piece's end reads the root's own row)
-            w[q] = a.ocols[lane < cnt[q] ? (uint64_t)cst + lane : lo];
+            // (a lane past the piece's end reads its last entry, a piece past
+            // the last one the root's own row)
+            const char* piece = reinterpret_cast<const char*>(a.ocols + (cnt[q] ? (uint64_t)cst : lo));
+            w[q] = *reinterpret_cast<const uint32_t*>(piece + umin32(lane * 4, cnt[q] ? cnt[q] * 4 - 4 : 0u));
             cst += kWave;
             left -= cnt[q];
         }
 #pragma unroll
-        for (int q = 0; q < VECS; q++) e[q] = lane < cnt[q] ? H.slot[w[q] & (T - 1)] : 0u;
-        uint32_t more = 0;
+        for (int q = 0; q < VECS; q++) e[q] = H.slot[w[q] & (T - 1)];
+        uint32_t all = 0;
 #pragma unroll
         for (int q = 0; q < VECS; q++) {
-            const bool cand = (e[q] & kMember) && (e[q] & kTag) == H.tag(w[q]);
-            v[q] = cand ? H.U[(e[q] & kMember) - 1] : ~w[q];
+            v[q] = H.U[H.member(e[q])];
+            all = umax32(all, e[q]);
         }
-#pragma unroll
-        for (int q = 0; q < VECS; q++) more |= v[q] != w[q] ? e[q] & kChain : 0u;
-        if (ballot(more != 0)) {  // members that share a slot
+        if (ballot(all >= kChain)) {  // members that share a slot
 #pragma unroll
             for (int q = 0; q < VECS; q++)
-                while (v[q] != w[q] && (e[q] & kChain)) {
-                    e[q] = H.next[(e[q] & kMember) - 1];
-                    v[q] = H.U[(e[q] & kMember) - 1];
+                while (v[q] != w[q] && e[q] >= kChain) {
+                    e[q] = H.next[H.member(e[q])];
+                    v[q] = H.U[H.member(e[q])];
                 }
         }
 #pragma unroll
         for (int q = 0; q < VECS; q++)
-            if (v[q] == w[q]) hit(own[q], (e[q] & kMember) - 1);
+            if (v[q] == w[q] && lane < cnt[q]) hit(own[q], H.member(e[q]));
     }
     // reversed members: one work list of (member, later member) over the
     // lanes; pos = |{entries <= w}| in the member's row, the entry at pos-1
@@ -656,28 +662,25 @@ __device__ __forceinline__ void count_root(const LocalProgram& P, uint32_t m, co
 template <bool ROWS>
 struct WaveLocal {
     uint64_t rows[ROWS ? kLRowWords : 1];
-    uint32_t U[kLMembers + 2];
-    uint16_t next[kLMembers + 2];
     __align__(8) uint16_t slot[kLSlots];  // (the count's queue after the build)
+    uint32_t U[kLMembers + 1];
+    uint16_t next[kLMembers + 1];
 };
 
 // Members and their index of one root, from registers, and cleared rows.
 template <int N, bool CLQ>
 __device__ __forceinline__ void wave_index(uint32_t m, const uint32_t* u, WaveLocal<!(CLQ && N == 3)>& L) {
     const uint32_t lane = lane_id();
-    const HashIndex<kLSlots> H{L.slot, L.next, L.U};
+    const HashIndex<kLSlots, kLMembers> H{L.slot, L.next, L.U};
     wave_sync();  // (the previous root's reads are done)
     if constexpr (!(CLQ && N == 3))
         for (uint32_t i = lane; i < m * row_stride(m); i += kWave) L.rows[i] = 0;
-    for (uint32_t i = lane; i < kLSlots / 4; i += kWave) reinterpret_cast<uint64_t*>(L.slot)[i] = 0;
+    H.clear(lane, kWave);
     wave_sync();
 #pragma unroll
     for (uint32_t h = 0; h < kLMemberRegs; h++) {
         const uint32_t i = h * kWave + lane;
-        if (i < m) {
-            L.U[i] = u[h];
-            H.put(i, u[h]);
-        }
+        if (i < m) H.put(i, u[h]);
     }
     wave_sync();
 }
@@ -689,7 +692,7 @@ __device__ __forceinline__ void wave_root(const LocalArgs& a, uint64_t lo, uint3
     constexpr bool kTri = CLQ && N == 3;
     const uint32_t lane = lane_id();
     const uint32_t W = row_stride(m);
-    const HashIndex<kLSlots> H{L.slot, L.next, L.U};
+    const HashIndex<kLSlots, kLMembers> H{L.slot, L.next, L.U};
     uint32_t hits = 0;
     for (uint32_t i0 = 0; i0 + 1 < m; i0 += kWave)
         build_rows<kVecsW>(a, H, m, lo, i0, 1, a.factor, [&](uint32_t ia, uint32_t ib) {
@@ -812,26 +815,34 @@ __global__ __launch_bounds__(256, 4) void gm_local_arena_kernel(LocalArgs a) {
     }
 }
 
+// waves per SIMD the registers are held to: what the LDS of the pass allows,
+// for the plans whose walk fits them (triangles, 4-cliques)
+constexpr int block_waves(int n, bool clq, int bu) { return bu < kB3U && clq && n <= 4 ? 8 : 4; }
+
 // Passes 2 to 4: one root per workgroup of BT threads, its rows in the workgroup's
-// LDS (up to ROWW words, |U| <= BU).  Three shapes run in turn: 256 threads with 25 KB of rows (four
-// workgroups per CU, |U| <= 448), 512 threads with 60 KB (two per CU, |U| <=
-// 700), then 1024 threads with 138 KB (one per CU).
+// LDS (up to ROWW words, |U| <= BU).  Three shapes run in turn: 512 threads with
+// 25 KB of rows (four workgroups per CU, |U| <= 448), 1024 threads with 60 KB
+// (two per CU, |U| <= 700), then 1024 threads with 138 KB (one per CU).  The LDS
+// sets the workgroups per CU, so the threads are as many as give 32 waves per
+// CU: with half of them the first two took 13.7 and 7.9 ms on R-MAT 22
+// (4-cliques) where they take 10.9 and 6.7.
 // Build: member i's row is one wave's work (wave i mod waves), cut into pieces
 // of 64 entries, kVecs pieces (of one or several members) in flight.  Which
 // member a piece belongs to is a scalar, and an entry is looked up by one LDS
 // read of its hash slot, a second only where the tag agrees (the members
 // themselves and 1 in 16 of the others).  Rows average ~400 entries on R-MAT
 // 22, of which 8% are hits.
-// Count: waves take position-1 candidates r1 one at a time from an LDS
-// counter, a wave's lanes share the position-2 candidates of its r1, queued 64
-// at a time in LDS, and each lane walks the rest of its (r1, r2) subtree.
+// Count: waves take the position-1 candidates r1 in turn; a wave's lanes share
+// their position-2 candidates, queued in LDS (cliques: the pairs of successive
+// r1 together, for 4-cliques two per lane so that four rows are read at a
+// time), and each lane walks the rest of its (r1, r2) subtree.
 // Triangles (CLQ, N = 3) are the build's hits: no rows, no count.
 template <int N, bool CLQ, int BT, int ROWW, int BU>
-__global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
+__global__ __launch_bounds__(BT, block_waves(N, CLQ, BU)) void gm_local_block_kernel(LocalArgs a) {
     constexpr int kWaves = BT / kWave;
     constexpr bool kTri = CLQ && N == 3;
     __shared__ uint64_t rows[kTri ? 1 : ROWW];
-    __shared__ uint32_t U[BU];
+    __shared__ uint32_t U[BU + 1];
     __shared__ uint16_t next[BU];
     __shared__ unsigned long long s_task;
     __shared__ uint32_t s_next;
@@ -839,9 +850,9 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
     // one buffer: a barrier separates the build from the count, and the next
     // root's slots from this count
     __shared__ __align__(16) uint16_t slot[kSlots];
-    static_assert(kWaves * kWave * 4 <= (int)sizeof(slot), "queues fit the slots");
-    auto queue = reinterpret_cast<uint32_t (*)[kWave]>(slot);
-    const HashIndex<kSlots> H{slot, next, U};
+    static_assert(kWaves * 2 * kWave * 4 <= (int)sizeof(slot), "queues fit the slots");
+    auto queue = reinterpret_cast<uint32_t (*)[2 * kWave]>(slot);
+    const HashIndex<kSlots, BU> H{slot, next, U};
     const uint32_t lane = lane_id();
     const uint32_t wid = uniform(threadIdx.x / kWave);
     const uint32_t tid = threadIdx.x;
@@ -854,7 +865,7 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
             s_task = atomicAdd(&a.ctr[LCTR_NEXT + a.pass], 1ull);
             s_next = 0;
         }
-        for (uint32_t i = tid; i < kSlots / 2; i += BT) reinterpret_cast<uint32_t*>(slot)[i] = 0;
+        H.clear(tid, BT);
         __syncthreads();
         const uint64_t t = uniform((uint64_t)s_task);
         if (t >= a.ntasks) break;
@@ -865,11 +876,7 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
         const uint64_t need = local_need(m);
         if constexpr (!kTri)
             for (uint32_t i = tid; i < need; i += BT) rows[i] = 0;
-        for (uint32_t i = tid; i < m; i += BT) {
-            const uint32_t u = a.ocols[lo + i];
-            U[i] = u;
-            H.put(i, u);
-        }
+        for (uint32_t i = tid; i < m; i += BT) H.put(i, a.ocols[lo + i]);
         __syncthreads();
         uint32_t hits = 0;
         for (uint32_t i0 = wid; i0 + 1 < m; i0 += kWaves * kWave)
@@ -889,47 +896,61 @@ __global__ __launch_bounds__(BT, 4) void gm_local_block_kernel(LocalArgs a) {
         __syncthreads();
 
         if constexpr (CLQ) {
-            // position-1 members r1 one at a time per wave; the (r1, r2)
-            // pairs of successive r1 share the wave's queue, 64 at a time
+            // position-1 members r1 by wave (r1 mod waves); the (r1, r2) pairs
+            // of successive r1 share the wave's queue, kPairs at a time
+            constexpr uint32_t kPairs = N == 4 ? 2 * kWave : kWave;
             const uint32_t nw = (m + 63) >> 6;
             uint32_t k = 0;
             auto drain_pairs = [&](uint32_t nq) {
                 wave_sync();
-                if (lane < nq) {
-                    const uint32_t e = queue[wid][lane];
-                    uint32_t off[N];
-                    off[1] = (e >> 16) * W;
-                    off[2] = (e & 0xffffu) * W;
-                    nodes++;
-                    clique_walk<N, 3>(rows, W, nw, off, e & 0xffffu, lane_total, nodes);
-                }
-                wave_sync();
-            };
-            while (true) {
-                __builtin_amdgcn_wave_barrier();
-                uint32_t r1 = 0;
-                if (lane == 0) r1 = atomicAdd(&s_next, 1u);
-                r1 = uniform(r1);
-                if (r1 >= m) break;
-                if (lane == 0) nodes++;
-                if constexpr (N == 3) {
-                    for (uint32_t w = (r1 >> 6) + lane; w < nw; w += kWave) lane_total += __popcll(rows[r1 * W + w]);
+                if constexpr (N == 4) {
+                    // two pairs per lane, their words' reads in flight together
+                    // (a lane without a pair reads the last member's row, which is empty)
+                    uint32_t a0 = (m - 1) * W, b0 = a0, w0 = nw, a1 = a0, b1 = a0, w1 = nw, c = 0;
+                    if (lane < nq) {
+                        const uint32_t e = queue[wid][lane];
+                        a0 = (e >> 16) * W;
+                        b0 = (e & 0xffffu) * W;
+                        w0 = (e & 0xffffu) >> 6;
+                    }
+                    if (lane + kWave < nq) {
+                        const uint32_t e = queue[wid][lane + kWave];
+                        a1 = (e >> 16) * W;
+                        b1 = (e & 0xffffu) * W;
+                        w1 = (e & 0xffffu) >> 6;
+                    }
+                    for (uint32_t w = umin32(w0, w1); w < nw; w++) {
+                        const uint64_t x0 = rows[a0 + w] & rows[b0 + w], x1 = rows[a1 + w] & rows[b1 + w];
+                        c += (uint32_t)__popcll(x0) + (uint32_t)__popcll(x1);
+                    }
+                    lane_total += c;
                 } else {
-                    for (uint32_t w = r1 >> 6; w < nw; w++) {
-                        const uint64_t cw = rows[r1 * W + w];
-                        const uint32_t cnt = (uint32_t)__popcll(cw);
-                        if (k + cnt > kWave) {
-                            drain_pairs(k);
-                            k = 0;
-                        }
-                        if ((cw >> lane) & 1) queue[wid][k + lanes_below(cw)] = (r1 << 16) | (w * 64 + lane);
-                        k += cnt;
+                    if (lane < nq) {
+                        const uint32_t e = queue[wid][lane];
+                        uint32_t off[N];
+                        off[1] = (e >> 16) * W;
+                        off[2] = (e & 0xffffu) * W;
+                        clique_walk<N, 3>(rows, W, nw, off, e & 0xffffu, lane_total, nodes);
                     }
                 }
+                if (lane == 0) nodes += nq;
+                wave_sync();
+            };
+            for (uint32_t r1 = wid; r1 < m; r1 += kWaves) {
+                const uint64_t own = lane < nw ? rows[r1 * W + lane] : 0;
+                for (uint32_t w = r1 >> 6; w < nw; w++) {
+                    const uint64_t cw = read_lane(own, w);
+                    const uint32_t cnt = (uint32_t)__popcll(cw);
+                    if (k + cnt > kPairs) {
+                        drain_pairs(k);
+                        k = 0;
+                    }
+                    if ((cw >> lane) & 1) queue[wid][k + lanes_below(cw)] = (r1 << 16) | (w * 64 + lane);
+                    k += cnt;
+                }
             }
-            if constexpr (N > 3) {
-                if (k) drain_pairs(k);
-            }
+            if (k) drain_pairs(k);
+            if (tid == 0) nodes += m;
             continue;
         }
         uint32_t M[N];
@@ -1421,21 +1442,21 @@ void gm_local_compile(g2_ctx* c, const g2_plan* p) {
     c->local_ok = true;
 }
 
-enum class LocalPass { Wave, Group256, Group512, Group1024, Arena };
+enum class LocalPass { Wave, Group1, Group2, Group3, Arena };
 
 template <int N, bool CLQ>
 static void launch_local(LocalPass pass, uint64_t blocks, uint32_t bw, hipStream_t s, const LocalArgs& a) {
     if constexpr (N > 2) {
         switch (pass) {
-            case LocalPass::Group256:
+            case LocalPass::Group1:
                 hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB1Threads, kB1RowWords, kB1U>), dim3(blocks),
                                    dim3(kB1Threads), 0, s, a);
                 return;
-            case LocalPass::Group512:
+            case LocalPass::Group2:
                 hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB2Threads, kB2RowWords, kB2U>), dim3(blocks),
                                    dim3(kB2Threads), 0, s, a);
                 return;
-            case LocalPass::Group1024:
+            case LocalPass::Group3:
                 hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB3Threads, kB3RowWords, kB3U>), dim3(blocks),
                                    dim3(kB3Threads), 0, s, a);
                 return;
@@ -1484,8 +1505,8 @@ static int pass_roots(g2_ctx* c, const uint64_t* orp, const uint32_t* rank, uint
     return G2_OK;
 }
 
-// Passes over the roots: rows in a wave's LDS; in a 256-, 512- and
-// 1024-thread workgroup's LDS; in per-wave global arenas sized to the largest
+// Passes over the roots: rows in a wave's LDS; in three sizes of workgroup LDS;
+// in per-wave global arenas sized to the largest
 // root left.  Which roots a pass takes is known before the first one starts,
 // so the passes are enqueued back to back and waited for once.
 int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
@@ -1554,11 +1575,12 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     const int ev0 = nev;
     if ((rc = mark())) return rc;
     const uint32_t* list = (const uint32_t*)((PassRoots*)c->big_list2.ptr + 1);
+    const bool tri = n == 3 && c->lprog.clique;  // (no rows in LDS)
     const struct { LocalPass pass; uint64_t most; } shape[kPasses] = {
         {LocalPass::Wave, nblocks},
-        {LocalPass::Group256, (uint64_t)c->num_cus * kB1PerCu},
-        {LocalPass::Group512, (uint64_t)c->num_cus * kB2PerCu},
-        {LocalPass::Group1024, (uint64_t)c->num_cus * kB3PerCu},
+        {LocalPass::Group1, (uint64_t)c->num_cus * kB1PerCu},
+        {LocalPass::Group2, (uint64_t)c->num_cus * kB2PerCu},
+        {LocalPass::Group3, (uint64_t)c->num_cus * (tri ? 2 : kB3PerCu)},
         {LocalPass::Arena, bwaves / bw}};
     int pass_ev[kPasses] = {-1, -1, -1, -1, -1};
     for (int k = 0; k < kPasses; k++) {

@@ -76,7 +76,7 @@ typedef struct g2_stats {
     uint32_t local_bitmap;        /* matching: 1 if the oriented local-bitmap passes counted the run */
     uint32_t reserved;
     uint64_t local_pass_roots[5]; /* local-bitmap matching: roots each pass took to the end (rows in
-                                     a wave's LDS; in a 256-, 512-, 1024-thread workgroup's LDS;
+                                     a wave's LDS; in three sizes of workgroup LDS;
                                      in per-wave global arenas) */
     uint64_t host_spill_bytes;    /* MCE: page-locked host memory the large-root arenas used because
                                      the device budget could not hold one wave's arena (0 = none) */
