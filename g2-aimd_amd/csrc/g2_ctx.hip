@@ -53,7 +53,7 @@ static void apply_tuning_defaults(g2_ctx* c) {
     if (!c->tune.wave_scratch_words) c->tune.wave_scratch_words = 1ull << 16;
     if (!c->tune.big_waves) c->tune.big_waves = 256;
     if (!c->tune.mce_small_max) c->tune.mce_small_max = 64;
-    if (!c->tune.mce_donate_every) c->tune.mce_donate_every = 256;
+    if (!c->tune.mce_donate_every) c->tune.mce_donate_every = 8;
 }
 
 }  // namespace g2
@@ -127,7 +127,7 @@ void g2_destroy(g2_ctx* c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (DevBuf* b : {&c->rp, &c->cols, &c->src, &c->gm_task_off, &c->counters, &c->scratch,
-                      &c->big_scratch, &c->list, &c->hist, &c->per_root, &c->order, &c->deg, &c->big_list2, &c->spans,
+                      &c->big_scratch, &c->list, &c->per_root, &c->order, &c->deg, &c->big_list2, &c->spans,
                       &c->batch_progs, &c->batch_q, &c->donate, &c->taskbuild, &c->orient, &c->roots})
         release(c, *b);
     if (c->spill) (void)hipHostFree(c->spill);

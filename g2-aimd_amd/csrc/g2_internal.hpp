@@ -131,7 +131,6 @@ struct g2_ctx {
     g2::DevBuf scratch;           // per-wave arenas
     g2::DevBuf big_scratch;
     g2::DevBuf list;              // deferred roots
-    g2::DevBuf hist;
     g2::DevBuf per_root;
     g2::DevBuf order;
     g2::DevBuf spans;
