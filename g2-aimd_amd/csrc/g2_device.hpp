@@ -53,6 +53,34 @@ __device__ __forceinline__ uint64_t wave_max(uint64_t x) {
     return x;
 }
 
+// Reductions of one 32-bit value over the 64 lanes by DPP moves: within rows of
+// 16 (shifts by 1, 2, 4, 8), then across rows (broadcasts of lanes 15 and 31
+// of each pair), the result in lane 63.  Six VALU steps, where six shuffles are
+// six LDS-crossbar round trips of ~100 cycles.  All lanes must be active.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, ROWS, 0xf, false);
+}
+__device__ __forceinline__ uint32_t wave_max32(uint32_t x) {
+    auto up = [&](uint32_t y) { x = y > x ? y : x; };
+    up(dpp_or_zero<0x111, 0xf>(x));
+    up(dpp_or_zero<0x112, 0xf>(x));
+    up(dpp_or_zero<0x114, 0xf>(x));
+    up(dpp_or_zero<0x118, 0xf>(x));
+    up(dpp_or_zero<0x142, 0xa>(x));
+    up(dpp_or_zero<0x143, 0xc>(x));
+    return read_lane(x, kWave - 1);
+}
+__device__ __forceinline__ uint32_t wave_sum32(uint32_t x) {
+    x += dpp_or_zero<0x111, 0xf>(x);
+    x += dpp_or_zero<0x112, 0xf>(x);
+    x += dpp_or_zero<0x114, 0xf>(x);
+    x += dpp_or_zero<0x118, 0xf>(x);
+    x += dpp_or_zero<0x142, 0xa>(x);
+    x += dpp_or_zero<0x143, 0xc>(x);
+    return read_lane(x, kWave - 1);
+}
+
 __device__ __forceinline__ uint64_t wave_sum(uint64_t x) {
 #pragma unroll
     for (int m = 32; m >= 1; m >>= 1) x += shfl_xor(x, m);

@@ -172,13 +172,23 @@ __device__ inline unsigned int* ring_place(const MceArgs& a, uint32_t r, unsigne
 struct RingLook {
     uint32_t r;            // ring looked at (wave-uniform)
     unsigned int waiting;  // registered waves there at the last look
+    uint64_t begin;        // clock at the task's start
+    uint64_t from;         // clock from which its frames may be handed on
 };
-__device__ inline RingLook ring_start(uint32_t gwave) { return RingLook{gwave % kRings, 0}; }
+__device__ inline RingLook ring_start(uint32_t gwave) { return RingLook{gwave % kRings, 0, 0, 0}; }
+// A taker builds the root's bitsets again, so a task hands nothing on before
+// it has walked for half as long as its own build took.  Wall ms of R-MAT 11 /
+// R-MAT 9 / 5k-vertex Chung-Lu: 2.54 / 0.51 / 0.48 without this rule, 2.55 /
+// 0.53 / 0.39 with it, 3.04 / 0.46 / 0.33 with the whole of the build's time.
+__device__ inline void walk_begins(RingLook& k) {
+    const uint64_t now = clock64();
+    k.from = now + (now - k.begin) / 2;
+}
 
 // a registered wave of the ring seen non-empty at the last look, taken off it; ~0 when there is none
 __device__ inline uint32_t ring_take(const MceArgs& a, RingLook& k) {
     uint32_t got = ~0u;
-    if (uniform(k.waiting) != 0) {
+    if (uniform(k.waiting) != 0 && (uint64_t)clock64() >= k.from) {
         __builtin_amdgcn_wave_barrier();
         uint32_t w = ~0u;
         if (lane_id() == 0) {
@@ -255,6 +265,7 @@ __device__ inline bool wait_record(const MceArgs& a, uint32_t gwave) {
 constexpr int kMaxBlockWaves = 4;  // __launch_bounds__(256)
 constexpr int kScoreWords = 2;     // candidate words scored per round (arena path)
 constexpr int kLdsArena = 896;     // u64 words of LDS per wave for the walk of a medium root
+constexpr uint32_t kWideX = 256;   // largest |X'| of the register walk over several words (384 and 512 spill more and gain nothing)
 constexpr int kMinLdsFrames = 16; // frames that must fit next to the rows for the LDS layout
 constexpr int kBuildItems = 4;    // neighbourhood-build items per lane in flight (C in LDS)
 constexpr uint32_t kPB = 255;      // value buckets over a root's P0 part in the build (C in LDS)
@@ -275,15 +286,6 @@ __device__ inline uint32_t lds_lower_bound(const uint32_t* A, uint32_t lo, uint3
         if (A[mid] < val) lo = mid + 1; else hi = mid;
     }
     return lo;
-}
-
-__device__ inline uint32_t wave_max32(uint32_t x) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-        const uint32_t y = __shfl_xor(x, m, kWave);
-        x = y > x ? y : x;
-    }
-    return x;
 }
 
 // Roots with d <= 64: the whole subtree in registers.  Position k of C maps
@@ -378,6 +380,7 @@ __device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s,
     const uint32_t lane = lane_id();
     const uint32_t p0 = d - s;
     // ---- depth-first walk (depth relative to `base`, the start node's depth) ----
+    walk_begins(look);
     uint64_t P = ones(p0), XP = 0, XX = ones(s), Q = 0;
     uint32_t base = 0;
     bool fresh = true;
@@ -474,6 +477,131 @@ __device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s,
     return nodes;
 }
 
+// The register walk of a root with |P0| <= 64 and |X'| <= 64 R: lane j holds
+// P0 member j's row over P0 (rowPP) and its rows over X' (rowX, word r = X'
+// positions 64 r ..), lane l the rows over P0 of X' members l, l + 64, ..
+// (rowXP).  A node is P, XP, Q and the R words of XX, all scalars, and the
+// stack is spread over the lanes as in small_walk, so a node costs no memory:
+// 0.6 us where the arena path's frames and rows in LDS took 1.4 (R-MAT 11, the
+// root with 53 later neighbours of 178).  The tree, the pivot rule (positions:
+// X', then P0) and the child order are the arena path's; so is a record, W = 1
+// and wx words of XX.
+template <int R>
+__device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uint32_t s2, uint32_t p0, uint64_t rowPP,
+                                              const uint64_t* rowXP, const uint64_t* rowX, uint32_t wx, uint32_t part,
+                                              uint32_t parts, const uint64_t* rec, RingLook& look, uint64_t& cliques,
+                                              uint64_t& hcount, uint64_t& hbig) {
+    const uint32_t lane = lane_id();
+    walk_begins(look);
+    uint64_t P = ones(p0), XP = 0, Q = 0, XX[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) XX[r] = s2 > 64u * r ? ones(s2 - 64 * r) : 0;
+    uint32_t base = 0;
+    bool fresh = true;
+    if (rec) {
+        const unsigned long long* d = (const unsigned long long*)rec;
+        const uint64_t w = lane < 5 + wx ? ld_dev(d + lane) : 0;
+        base = (uint32_t)read_lane(w, 1);
+        P = read_lane(w, 2);
+        XP = read_lane(w, 3);
+        Q = read_lane(w, 4);
+#pragma unroll
+        for (int r = 0; r < R; r++) XX[r] = read_lane(w, 5 + r);
+        fresh = false;
+    }
+    uint64_t fP = 0, fXP = 0, fQ = 0, fXX[R];  // frame of depth == lane
+#pragma unroll
+    for (int r = 0; r < R; r++) fXX[r] = 0;
+    uint32_t depth = 0, child = 0, since = 0;
+    uint64_t nodes = 0;
+    while (true) {
+        if (fresh) {
+            if (base + depth > 0 || part == 0) nodes++;
+            if (a.donate_every && ++since >= a.donate_every && nodes >= (uint64_t)kDonateFrom * a.donate_every) {
+                // as in small_walk
+                since = 0;
+                const uint32_t first = (base == 0 && parts > 1) ? 1u : 0u;
+                const uint64_t open = ballot(lane < depth && lane >= first && fQ != 0);
+                const uint32_t to = open ? ring_take(a, look) : ~0u;
+                if (to != ~0u) {
+                    const uint32_t i = __builtin_ctzll(open);
+                    const uint64_t fp = read_lane(fP, i), fxp = read_lane(fXP, i), fq = read_lane(fQ, i);
+                    const uint32_t nq = __popcll(fq);
+                    const uint64_t keep = nq >= 2 ? lowest_bits(fq, nq - nq / 2) : 0;
+                    uint64_t w = lane == 0 ? (uint64_t)si : lane == 1 ? (uint64_t)(base + i)
+                               : lane == 2 ? (fp & ~keep) : lane == 3 ? (fxp | keep) : (fq & ~keep);
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        const uint64_t fx = read_lane(fXX[r], i);
+                        w = lane == 5u + r ? fx : w;
+                    }
+                    record_made(a);
+                    if (lane < 5 + wx) st_dev((unsigned long long*)&a.area[(uint64_t)to * kRecWords + lane], w);
+                    record_send(a, to);
+                    fQ = lane == i ? keep : fQ;
+                }
+            }
+            if (P == 0) {
+                uint64_t x = XP;
+#pragma unroll
+                for (int r = 0; r < R; r++) x |= XX[r];
+                if (x == 0) {  // maximal clique, |R| = base + depth + 1
+                    cliques++;
+                    const uint32_t sz = base + depth + 1;
+                    if (sz < kWave) hcount += (lane == sz);
+                    else hbig += (lane == sz - kWave);
+                }
+            } else {
+                uint32_t key = (((P | XP) >> lane) & 1) ? ((uint32_t)__popcll(rowPP & P) << 10) | (64u * R + lane) : 0u;
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    const uint32_t kx = ((XX[r] >> lane) & 1) ? ((uint32_t)__popcll(rowXP[r] & P) << 10) | (64u * r + lane) : 0u;
+                    key = umax32(key, kx);
+                }
+                const uint32_t pivot = wave_max32(key) & 0x3ffu;
+                uint64_t prow = read_lane(rowPP, pivot & 63u);
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    if ((pivot >> 6) == (uint32_t)r) prow = read_lane(rowXP[r], pivot & 63u);
+                Q = P & ~prow;
+            }
+            fresh = false;
+        }
+        if (Q != 0) {
+            const uint32_t j = __builtin_ctzll(Q);
+            const uint64_t m = 1ull << j;
+            Q &= ~m;
+            P &= ~m;
+            XP |= m;
+            if (base + depth == 0 && (child++ % parts) != part) continue;  // another part's child
+            const bool mine = lane == depth;
+            fP = mine ? P : fP;
+            fXP = mine ? XP : fXP;
+            fQ = mine ? Q : fQ;
+#pragma unroll
+            for (int r = 0; r < R; r++) {
+                fXX[r] = mine ? XX[r] : fXX[r];
+                XX[r] &= read_lane(rowX[r], j);
+            }
+            const uint64_t qrow = read_lane(rowPP, j);
+            P &= qrow;
+            XP &= qrow;
+            Q = 0;
+            depth++;
+            fresh = true;
+        } else {
+            if (depth == 0) break;
+            depth--;
+            P = read_lane(fP, depth);
+            XP = read_lane(fXP, depth);
+            Q = read_lane(fQ, depth);
+#pragma unroll
+            for (int r = 0; r < R; r++) XX[r] = read_lane(fXX[r], depth);
+        }
+    }
+    return nodes;
+}
+
 template <bool ACCOUNT>
 __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
     __shared__ unsigned long long lhist[64];
@@ -506,6 +634,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
         const uint64_t d = uniform(a.rp[v + 1]) - lo;
         const uint32_t* __restrict__ C = a.cols + lo;
         uint64_t root_nodes = 0;
+        look.begin = clock64();
 
         if (d == 0) return;  // no subgraph is generated for an isolated root
         const uint64_t s = uniform(lower_bound(C, 0, d, v));
@@ -783,6 +912,49 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
             }
             const uint64_t s2 = read_lane(incl, kWave - 1);
             const uint64_t WX2 = (s2 + 63) / 64, FW2 = 3 * W + WX2;
+            if (W == 1 && s2 + p0 > kWave && s2 <= kWideX) {
+                // register walk: X' rows, then P0's rows over X', are compressed in
+                // LDS one after the other and taken into registers
+                SL.start[lane] = xmw;  // (the build's work list is no longer needed)
+                SL.pref[lane] = incl - cnt;
+                for (uint64_t t = 0; t < WX; t++) {  // rows of X' in position order
+                    const uint64_t xm = read_lane(xmw, (uint32_t)t);
+                    if ((xm >> lane) & 1) SA[read_lane(incl - cnt, (uint32_t)t) + lanes_below(xm)] = adjP[t * 64 + lane];
+                }
+                const uint64_t rowPP = lane < p0 ? adjP[s + lane] : 0;
+                wave_sync();
+                uint64_t rowXP[kWideX / 64], rowX[kWideX / 64];
+#pragma unroll
+                for (uint32_t r = 0; r < kWideX / 64; r++) rowXP[r] = r * 64 + lane < s2 ? SA[r * 64 + lane] : 0;
+                wave_sync();
+                for (uint64_t i = lane; i < p0 * WX2; i += kWave) SA[i] = 0;
+                wave_sync();
+                for (uint64_t f = lane; f < p0 * WX; f += kWave) {
+                    const uint64_t j = f / WX, t = f - j * WX;
+                    const uint64_t xm = SL.start[t], before = SL.pref[t];
+                    uint64_t word = adjX[j * WX + t];
+                    while (word) {
+                        const uint32_t b = __builtin_ctzll(word);
+                        word &= word - 1;
+                        const uint64_t c = before + __popcll(xm & ((1ull << b) - 1));
+                        atomicOr((unsigned long long*)&SA[j * WX2 + (c >> 6)], 1ull << (c & 63));
+                    }
+                }
+                wave_sync();
+#pragma unroll
+                for (uint32_t r = 0; r < kWideX / 64; r++) rowX[r] = lane < p0 && r < WX2 ? SA[lane * WX2 + r] : 0;
+                const uint32_t wx = (uint32_t)WX2, sx = (uint32_t)s2, pp = (uint32_t)p0;
+                if (wx <= 2)
+                    root_nodes = wide_walk<2>(a, si, sx, pp, rowPP, rowXP, rowX, wx, part, parts, rec, look, small_cliques,
+                                              small_hist, small_big);
+                else
+                    root_nodes = wide_walk<kWideX / 64>(a, si, sx, pp, rowPP, rowXP, rowX, wx, part, parts, rec, look,
+                                                        small_cliques, small_hist, small_big);
+                my_nodes += root_nodes;
+                if (a.per_root && lane == 0 && root_nodes) atomicAdd(&a.per_root[si], (unsigned long long)root_nodes);
+                t_end = wall_clock64();
+                return;
+            }
             const uint64_t rows2 = (s2 + p0) * W + p0 * WX2;
             const uint64_t nfr = rows2 < kLdsArena ? (kLdsArena - rows2) / FW2 : 0;
             if (nfr >= kMinLdsFrames) {
@@ -836,6 +1008,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
         auto frame = [&](uint64_t dep) -> uint64_t* { return dep < DL ? lfr + dep * FWE : frames + dep * FWE; };
 
         // ---- depth-first walk of the root's subtree -----------------------
+        walk_begins(look);
         uint64_t pw = 0, xpw = 0, qw = 0;
         uint64_t base = 0;   // depth of the start node (a donated frame's depth)
         bool fresh = true;
@@ -955,7 +1128,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                             }
                         }
                     };
-                    const uint64_t npw = wave_sum(__popcll(pw));  // |P|
+                    const uint64_t npw = wave_sum32((uint32_t)__popcll(pw));  // |P|
                     // column scoring costs ~|P|/4 rounds of loads, candidate scoring
                     // ~(nonzero X words)/kScoreWords rounds: take the cheaper
                     const uint64_t xw0 = (WXE <= kWave && lane < WXE) ? XX[lane] : 0;
@@ -1015,8 +1188,9 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                         const uint64_t uw = pw | xpw;
                         score_words(uw, ballot(uw != 0), sE);
                     }
-                    best = wave_max(best);
-                    const uint64_t pivot = best & 0xffffffffull;
+                    // (the largest score, then the largest position with it)
+                    const uint32_t top = wave_max32((uint32_t)(best >> 32));
+                    const uint64_t pivot = wave_max32((uint32_t)(best >> 32) == top ? (uint32_t)best : 0u);
                     const uint64_t* prow = aP + pivot * W;
                     qw = lane < W ? (pw & ~prow[lane]) : 0;
                     if (ACCOUNT && own) {
