@@ -171,7 +171,7 @@ int set_err(g2_ctx* c, int code, const std::string& msg);
 // resident waves per CU of a persistent grid: the context's setting, else the
 // kernel's own default (measured on MI355X: latency-bound searches gain up to
 // the occupancy their register use allows)
-enum WaveKind { WK_MCE = 16, WK_GM = 16, WK_WALK = 20, WK_GM_LOCAL = 28, WK_FEATURES = 16 };
+enum WaveKind { WK_MCE = 16, WK_GM = 16, WK_WALK = 20, WK_GM_LOCAL = 28, WK_SKETCH = 32, WK_FEATURES = 16 };
 inline uint32_t waves_per_cu(const g2_ctx* c, WaveKind k) {
     return c->tune.waves_per_cu ? c->tune.waves_per_cu : (uint32_t)k;
 }

@@ -48,6 +48,7 @@ struct FeatArgs {
     const uint32_t* sup;
     const uint32_t* rank;
     const uint8_t* sketch;  // nv x 64 HyperLogLog registers of the closed rows N[u]
+    uint32_t run;           // roots per counter fetch
     double lc[65];          // linear counting: lc[V] = 64 ln(64 / V), from the host's libm
 };
 
@@ -69,7 +70,9 @@ __device__ inline void hll_put(uint32_t* reg, uint32_t w) {
 }
 
 // registers of every vertex's closed row N[u] = N(u) u {u}: one wave per
-// vertex, the maxima taken in the wave's 64 LDS words
+// vertex, the maxima taken in the wave's 64 LDS words (a chain of row offsets,
+// row and LDS per vertex, so as many waves as fit: 200k-vertex social graph
+// 43 us, 63 with 16 waves per CU)
 __global__ __launch_bounds__(256) void sketch_kernel(const uint64_t* __restrict__ rp, const uint32_t* __restrict__ cols,
                                                      uint64_t nv, uint8_t* __restrict__ sk) {
     __shared__ uint32_t regs[4][kWave];
@@ -88,38 +91,89 @@ __global__ __launch_bounds__(256) void sketch_kernel(const uint64_t* __restrict_
     }
 }
 
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+
+// maximum over the wave's 16 groups of four lanes (lanes of equal lane % 4)
+__device__ __forceinline__ uint32_t group_max(uint32_t x) {
+    auto up = [&](uint32_t y) {
+        x = __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, x), __builtin_bit_cast(u16x2, y)));
+    };
+    up(dpp_or_zero<0x124, 0xf>(x));  // within 16 lanes: rotated by 4, by 8
+    up(dpp_or_zero<0x128, 0xf>(x));
+    up((uint32_t)__shfl_xor((int)x, 16, kWave));
+    up((uint32_t)__shfl_xor((int)x, 32, kWave));
+    return x;
+}
+
+// One wave per root.  What bounds it: the neighbours' 64 register bytes (a
+// gather of 64 B per row entry, mostly from beyond the 4 MB L2 of an XCD for a
+// 13 MB table).  So four lanes read a neighbour's row, 16 bytes each, and an
+// instruction reads 16 neighbours' (four of them in flight); the bytes are
+// folded as packed 16-bit maxima and the 16 groups once per root.  One byte per
+// lane and eight neighbours in flight took 5.3 ms where this takes 0.52
+// (200k-vertex social graph; 8, 12, 24 and 32 waves per CU: 0.63, 0.59, 0.54,
+// 0.63 -- more waves share the L2, fewer leave it idle).
 __global__ __launch_bounds__(256) void feature_kernel(FeatArgs a) {
     const uint32_t lane = lane_id();
-    // sources come in runs of 16 per counter fetch: a root's features cost a
-    // few row walks, and one atomic per root would queue the waves on it
-    constexpr uint32_t kRun = 16;
+    const uint32_t group = lane / 4, part = lane % 4;
+    const uint4* sketch = reinterpret_cast<const uint4*>(a.sketch);
     uint64_t t = 0, tend = 0;
     while (true) {
         if (t == tend) {
-            t = fetch_tasks(a.next, kRun);
-            tend = umin64(t + kRun, a.ns);
+            t = fetch_tasks(a.next, a.run);
+            tend = umin64(t + a.run, a.ns);
         }
         if (t >= a.ns) break;
         const uint64_t ti = t++;
         const uint32_t v = uniform(a.src[ti]);
-        const uint64_t lo = a.rp[v], hi = a.rp[v + 1], d = hi - lo;
-        uint64_t p0 = 0, tri2 = 0, shared = 0;
-        for (uint64_t e = lo + lane; e < hi; e += kWave) p0 += a.cols[e] > v;
-        // 2-hop ball: register-wise maximum over N[v] and the N[u], u in N(v)
-        // (lane l holds register l; 8 neighbours' registers in flight)
-        uint32_t reg = a.sketch[(uint64_t)v * kWave + lane];
-        for (uint64_t e0 = lo; e0 < hi; e0 += 8) {
-            uint32_t r[8];
-#pragma unroll
-            for (int q = 0; q < 8; q++) {
-                const uint64_t e = e0 + q;
-                r[q] = e < hi ? a.sketch[(uint64_t)uniform(a.cols[e]) * kWave + lane] : 0u;
-            }
-#pragma unroll
-            for (int q = 0; q < 8; q++) reg = umax32(reg, r[q]);
+        const uint64_t lo = uniform(a.rp[v]), hi = uniform(a.rp[v + 1]), d = hi - lo;
+        uint64_t tri2 = 0, shared = 0;
+        if (a.tri) {
+            const uint32_t x = uniform(a.rank[v]);
+            tri2 = a.tri[x];
+            shared = a.sup[x];
         }
-        const uint64_t hsum = wave_sum(1ull << (32 - reg));
-        const uint64_t zeros = wave_sum(reg == 0);
+        // 2-hop ball: register-wise maximum over N[v] and the N[u], u in N(v);
+        // even and odd registers of the lane's 16 apart, as 16-bit values
+        uint32_t even[4] = {0, 0, 0, 0}, odd[4] = {0, 0, 0, 0};
+        auto fold = [&](const uint4& r) {
+            const uint32_t w[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const auto up = [](uint32_t x, uint32_t y) {
+                    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2, x), __builtin_bit_cast(u16x2, y)));
+                };
+                even[k] = up(even[k], w[k] & 0x00ff00ffu);
+                odd[k] = up(odd[k], (w[k] >> 8) & 0x00ff00ffu);
+            }
+        };
+        const uint4 own = sketch[(uint64_t)v * 4 + part];
+        uint32_t later = 0;
+        for (uint64_t e0 = lo; e0 < hi; e0 += kWave) {
+            const uint32_t n = (uint32_t)umin64(hi - e0, kWave);
+            const uint32_t u = lane < n ? a.cols[e0 + lane] : v;  // (v itself adds nothing)
+            later += (uint32_t)__popcll(ballot(u > v));
+            uint4 r[4];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++)
+                if (q * 16 < n) r[q] = sketch[(uint64_t)(uint32_t)__shfl((int)u, (int)(q * 16 + group), kWave) * 4 + part];
+#pragma unroll
+            for (uint32_t q = 0; q < 4; q++)
+                if (q * 16 < n) fold(r[q]);
+        }
+        fold(own);
+        // lane l: register 16 (l % 4) + l / 4
+        uint32_t word = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t ev = group_max(even[k]), od = group_max(odd[k]);
+            if (group / 4 == (uint32_t)k) word = group & 1 ? od : ev;
+        }
+        const uint32_t reg = group & 2 ? word >> 16 : word & 0xffffu;
+        // sum 2^(32 - reg), exactly: empty registers apart, the others' 16-bit halves
+        const uint32_t zeros = (uint32_t)__popcll(ballot(reg == 0));
+        const uint32_t term = reg ? 1u << (32 - reg) : 0u;
+        const uint64_t hsum = ((uint64_t)zeros << 32) + ((uint64_t)wave_sum32(term >> 16) << 16) + wave_sum32(term & 0xffffu);
         for (uint64_t e = a.tri ? hi : lo; e < hi; e++) {
             const uint32_t u = a.cols[e];
             const uint64_t ulo = a.rp[u], uhi = a.rp[u + 1];
@@ -133,7 +187,6 @@ __global__ __launch_bounds__(256) void feature_kernel(FeatArgs a) {
             tri2 += c;
             shared += c > 0;
         }
-        p0 = wave_sum(p0);
         if (lane == 0) {
             // E = alpha_64 m^2 / sum 2^-reg; linear counting below 5m/2 when a
             // register is empty
@@ -142,9 +195,9 @@ __global__ __launch_bounds__(256) void feature_kernel(FeatArgs a) {
             int64_t* o = a.out + ti * G2_NFEAT_INT;
             o[0] = (int64_t)d;
             o[1] = (int64_t)(est + 0.5);
-            o[2] = a.tri ? (int64_t)a.tri[a.rank[v]] : (int64_t)(tri2 / 2);
-            o[3] = a.tri ? (int64_t)a.sup[a.rank[v]] : (int64_t)shared;
-            o[4] = (int64_t)p0;
+            o[2] = (int64_t)(a.tri ? tri2 : tri2 / 2);
+            o[3] = (int64_t)shared;
+            o[4] = (int64_t)later;
         }
     }
 }
@@ -342,13 +395,17 @@ static int features_dev(g2_ctx* c, int64_t* dfeat) {
         }
     } sk_buf{c, {}};
     if ((rc = ensure(c, sk_buf.b, nv1 * kWave, "2-hop sketches"))) return rc;
-    const uint64_t blocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, WK_FEATURES) / 4);
-    if (c->nv) hipLaunchKernelGGL(sketch_kernel, dim3(blocks), dim3(256), 0, c->stream, (const uint64_t*)c->rp.ptr,
+    const uint64_t sblocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, WK_SKETCH) / 4);
+    if (c->nv) hipLaunchKernelGGL(sketch_kernel, dim3(sblocks), dim3(256), 0, c->stream, (const uint64_t*)c->rp.ptr,
                                   (const uint32_t*)c->cols.ptr, c->nv, (uint8_t*)sk_buf.b.ptr);
     if ((e = hipGetLastError())) return hip_err(c, e, "sketch launch");
     if ((e = hipMemsetAsync(c->counters.ptr, 0, 8, c->stream))) return hip_err(c, e, "memset");
+    const uint64_t blocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, WK_FEATURES) / 4);
+    // roots per counter fetch: four fetches a wave, and at most 16 roots at a
+    // time (one counter serves about one atomic per 12 ns)
+    const uint32_t run = (uint32_t)std::min<uint64_t>(16, std::max<uint64_t>(1, c->ns / (blocks * 16)));
     FeatArgs a{(const uint64_t*)c->rp.ptr, (const uint32_t*)c->cols.ptr, (const uint32_t*)c->src.ptr, c->ns,
-               (unsigned long long*)c->counters.ptr, dfeat, tri, sup, rank, (const uint8_t*)sk_buf.b.ptr, {}};
+               (unsigned long long*)c->counters.ptr, dfeat, tri, sup, rank, (const uint8_t*)sk_buf.b.ptr, run, {}};
     a.lc[0] = 0.0;
     for (int z = 1; z <= 64; z++) a.lc[z] = 64.0 * std::log(64.0 / (double)z);
     hipLaunchKernelGGL(feature_kernel, dim3(blocks), dim3(256), 0, c->stream, a);
