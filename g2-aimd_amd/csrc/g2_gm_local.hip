@@ -379,7 +379,8 @@ struct HashIndex {
 };
 
 // Local rows of members i0, i0 + stride, .. (64 of them, one per lane) by one
-// wave: hit(i, j) for every pair i < j of members joined by an edge.  Member i
+// wave: hit(i, j, e) for every pair i < j of members joined by an edge, U_j at
+// entry e of the oriented rows.  Member i
 // has either the n entries of N+(U_i) to look up in U, or, when n exceeds
 // (m-1-i) x factor, its m-1-i later members to look up in N+(U_i) (global
 // memory).  A lookup there is a chain of ~9 loads, a streamed entry a share of
@@ -414,7 +415,7 @@ __device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T
     uint64_t todo = ballot(len && !rev);
     uint32_t cst = 0, left = 0, ci = 0;
     while (left || todo) {
-        uint32_t own[VECS], cnt[VECS], w[VECS], e[VECS], v[VECS];
+        uint32_t own[VECS], cnt[VECS], at[VECS], w[VECS], e[VECS], v[VECS];
 #pragma unroll
         for (int q = 0; q < VECS; q++) {
             if (!left && todo) {
@@ -425,6 +426,7 @@ __device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T
                 ci = i0 + k * stride;
             }
             own[q] = ci;
+            at[q] = cst;
             cnt[q] = umin32(left, kWave);
             // (a lane past the piece's end reads its last entry, a piece past
             // the last one the root's own row)
@@ -451,7 +453,7 @@ __device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T
         }
 #pragma unroll
         for (int q = 0; q < VECS; q++)
-            if (v[q] == w[q] && lane < cnt[q]) hit(own[q], H.member(e[q]));
+            if (v[q] == w[q] && lane < cnt[q]) hit(own[q], H.member(e[q]), at[q] + lane);
     }
     // reversed members: one work list of (member, later member) over the
     // lanes; pos = |{entries <= w}| in the member's row, the entry at pos-1
@@ -507,7 +509,7 @@ __device__ __forceinline__ void build_rows(const LocalArgs& a, const HashIndex<T
         }
 #pragma unroll
         for (int q = 0; q < kRevItems; q++)
-            if (rlen[q] && last[q] == w[q]) hit(own[q], later[q]);
+            if (rlen[q] && last[q] == w[q]) hit(own[q], later[q], rst[q] + pos[q] - 1);
     }
 }
 
@@ -695,7 +697,7 @@ __device__ __forceinline__ void wave_root(const LocalArgs& a, uint64_t lo, uint3
     const HashIndex<kLSlots, kLMembers> H{L.slot, L.next, L.U};
     uint32_t hits = 0;
     for (uint32_t i0 = 0; i0 + 1 < m; i0 += kWave)
-        build_rows<kVecsW>(a, H, m, lo, i0, 1, a.factor, [&](uint32_t ia, uint32_t ib) {
+        build_rows<kVecsW>(a, H, m, lo, i0, 1, a.factor, [&](uint32_t ia, uint32_t ib, uint32_t) {
             if constexpr (kTri) {
                 hits++;
             } else {
@@ -880,7 +882,7 @@ __global__ __launch_bounds__(BT, block_waves(N, CLQ, BU)) void gm_local_block_ke
         __syncthreads();
         uint32_t hits = 0;
         for (uint32_t i0 = wid; i0 + 1 < m; i0 += kWaves * kWave)
-            build_rows<kVecs>(a, H, m, lo, i0, kWaves, kRevFactor, [&](uint32_t ia, uint32_t ib) {
+            build_rows<kVecs>(a, H, m, lo, i0, kWaves, kRevFactor, [&](uint32_t ia, uint32_t ib, uint32_t) {
                 if constexpr (kTri) {
                     hits++;
                 } else {  // (row offsets within the LDS rows fit 32 bits)
@@ -1276,36 +1278,140 @@ static int build_oriented(g2_ctx* c, const uint64_t** orp, const uint32_t** ocol
 
 // ---- triangle features (learned scheduler) ---------------------------------
 // Every triangle x < y < z (ranks) is found once, at its lowest rank x, as
-// the pair (y, z) of U(x) = N+(x) with z in N+(y): the local rows' work list
-// without the rows (build_chunk MODE 2).  Its three vertices get one count
-// each and its three oriented entries (x,y), (x,z), (y,z) their flags.
-__global__ __launch_bounds__(256) void tri_kernel(LocalArgs a) {
-    __shared__ uint32_t lU[kLocalBlockWaves][kLU];
+// the pair (y, z) of U(x) = N+(x) with z in N+(y).  Its three vertices get one
+// count each and its three oriented entries (x,y), (x,z), (y,z) their flags.
+// Members' counts are kept in LDS next to their index (build_rows), so a
+// triangle costs two LDS atomics and one byte store, and a member one global
+// atomic per root: with a global atomic per triangle and member, and members
+// searched in U by halving, the 200k-vertex social graph took 2.09 ms,
+// now 0.60.
+template <uint32_t T, uint32_t NONE>
+struct TriLocal {
+    __align__(8) uint16_t slot[T];
+    uint32_t U[NONE + 1], count[NONE];
+    uint16_t next[NONE + 1];
+};
+
+// Triangles of one root's members i0, i0 + stride, .. by one wave
+template <int VECS, uint32_t T, uint32_t NONE>
+__device__ __forceinline__ void tri_rows(const LocalArgs& a, TriLocal<T, NONE>& L, uint64_t lo, uint32_t m, uint32_t i0,
+                                         uint32_t stride) {
+    const HashIndex<T, NONE> H{L.slot, L.next, L.U};
+    build_rows<VECS>(a, H, m, lo, i0, stride, a.factor, [&](uint32_t ia, uint32_t ib, uint32_t e) {
+        atomicAdd(&L.count[ia], 1u);
+        atomicAdd(&L.count[ib], 1u);
+        a.flag[e] = 1;
+    });
+}
+
+// Counts of one root's members to their vertices and flags to its entries,
+// threads tid, tid + n, ..; returns this thread's share of twice the root's count
+template <uint32_t T, uint32_t NONE>
+__device__ __forceinline__ uint32_t tri_flush(const LocalArgs& a, const TriLocal<T, NONE>& L, uint64_t lo, uint32_t m,
+                                              uint32_t tid, uint32_t n) {
+    uint32_t sum = 0;
+    for (uint32_t i = tid; i < m; i += n) {
+        const uint32_t k = L.count[i];
+        if (!k) continue;
+        sum += k;
+        atomicAdd(&a.tri[L.U[i]], (unsigned long long)k);
+        a.flag[lo + i] = 1;
+    }
+    return sum;
+}
+
+// roots of up to kLMembers members, one per wave, a run of ranks per fetch
+__global__ __launch_bounds__(256, 7) void tri_kernel(LocalArgs a) {
+    __shared__ TriLocal<kLSlots, kLMembers> lds[kLocalBlockWaves];
     const uint32_t lane = lane_id();
     const uint32_t wid = threadIdx.x / kWave;
-    uint64_t t = 0, tend = 0;
+    TriLocal<kLSlots, kLMembers>& L = lds[wid];
+    const HashIndex<kLSlots, kLMembers> H{L.slot, L.next, L.U};
+    const uint64_t total = (a.ntasks + a.run - 1) / a.run;
+    uint32_t queue = (uint32_t)(((uint64_t)blockIdx.x * kLocalBlockWaves + wid) % kQueues);
     while (true) {
-        if (t == tend) {
-            t = fetch_tasks(&a.ctr[LCTR_NEXT], kFetchRun);
-            tend = umin64(t + kFetchRun, a.ntasks);
+        const uint64_t b = queue_next(a.ctr + LCTR_QUEUE, queue, total);
+        if (b == kNoTask) break;
+        // lane l: the run's root l, from the top rank down
+        uint64_t rlo = 0;
+        uint32_t rm = 0;
+        if (lane < a.run && b * a.run + lane < a.ntasks) {
+            const uint64_t x = a.ntasks - 1 - (b * a.run + lane);
+            rlo = a.orp[x];
+            rm = (uint32_t)(a.orp[x + 1] - rlo);
         }
-        if (t >= a.ntasks) break;
-        const uint32_t x = uniform((uint32_t)t);
-        t++;
-        const uint64_t lo = uniform(a.orp[x]);
-        const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
-        if (m < 2) continue;
-        const uint32_t* U = a.ocols + lo;
-        wave_sync();  // (the previous root's reads of lU are done)
-        if (m <= kLU) {
-            for (uint32_t i = lane; i < m; i += kWave) lU[wid][i] = U[i];
+        uint64_t todo = ballot(rm >= 2 && rm <= kLMembers);
+        while (todo) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(todo);
+            todo &= todo - 1;
+            const uint64_t lo = read_lane(rlo, l);
+            const uint32_t m = read_lane(rm, l);
+            wave_sync();  // (the previous root's reads are done)
+            H.clear(lane, kWave);
             wave_sync();
-            U = lU[wid];
+            for (uint32_t i = lane; i < m; i += kWave) {
+                H.put(i, a.ocols[lo + i]);
+                L.count[i] = 0;
+            }
+            wave_sync();
+            for (uint32_t i0 = 0; i0 + 1 < m; i0 += kWave) tri_rows<kVecsW>(a, L, lo, m, i0, 1);
+            wave_sync();
+            const uint32_t sum = wave_sum32(tri_flush(a, L, lo, m, lane, kWave));
+            if (lane == 0 && sum) atomicAdd(&a.tri[a.ntasks - 1 - (b * a.run + l)], (unsigned long long)(sum / 2));
         }
-        uint32_t hits = 0;
-        for (uint32_t a0 = 0; a0 + 1 < m; a0 += kWave) build_chunk<2>(a, U, nullptr, m, 0, a0, lo, hits);
-        const uint64_t tot = wave_sum((uint64_t)hits);
-        if (lane == 0 && tot) atomicAdd(&a.tri[x], (unsigned long long)tot);
+    }
+}
+
+// larger roots, one per workgroup: ranks blockIdx.x, blockIdx.x + gridDim.x, ..
+// (the large ones are neighbours in rank, so this spreads them); beyond the
+// index's members a wave searches U in global memory instead
+__global__ __launch_bounds__(512) void tri_block_kernel(LocalArgs a) {
+    __shared__ TriLocal<kSlots, kB3U> L;
+    __shared__ uint32_t twice;  // the root's members' counts
+    const uint32_t lane = lane_id(), tid = threadIdx.x;
+    if (tid == 0) twice = 0;
+    const uint32_t wid = uniform(tid / kWave), nw = blockDim.x / kWave;
+    const HashIndex<kSlots, kB3U> H{L.slot, L.next, L.U};
+    for (uint64_t x0 = blockIdx.x; x0 < a.ntasks; x0 += (uint64_t)gridDim.x * kWave) {
+        const uint64_t xl = x0 + (uint64_t)lane * gridDim.x;
+        uint64_t rlo = 0;
+        uint32_t rm = 0;
+        if (xl < a.ntasks) {
+            rlo = a.orp[xl];
+            rm = (uint32_t)(a.orp[xl + 1] - rlo);
+        }
+        uint64_t todo = ballot(rm > kLMembers);  // (the same in every wave)
+        while (todo) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(todo);
+            todo &= todo - 1;
+            const uint64_t lo = read_lane(rlo, l), x = x0 + (uint64_t)l * gridDim.x;
+            const uint32_t m = read_lane(rm, l);
+            if (m > kB3U) {
+                uint32_t hits = 0;
+                for (uint32_t a0 = wid * kWave; a0 + 1 < m; a0 += nw * kWave)
+                    build_chunk<2>(a, a.ocols + lo, nullptr, m, 0, a0, lo, hits);
+                const uint32_t sum = wave_sum32(hits);
+                if (lane == 0 && sum) atomicAdd(&a.tri[x], (unsigned long long)sum);
+                continue;
+            }
+            __syncthreads();  // (the previous root's reads are done)
+            H.clear(tid, blockDim.x);
+            __syncthreads();
+            for (uint32_t i = tid; i < m; i += blockDim.x) {
+                H.put(i, a.ocols[lo + i]);
+                L.count[i] = 0;
+            }
+            __syncthreads();
+            for (uint32_t i0 = wid; i0 + 1 < m; i0 += nw * kWave) tri_rows<kVecsW>(a, L, lo, m, i0, nw);
+            __syncthreads();
+            const uint32_t sum = wave_sum32(tri_flush(a, L, lo, m, tid, blockDim.x));
+            if (lane == 0 && sum) atomicAdd(&twice, sum);
+            __syncthreads();
+            if (tid == 0) {
+                if (twice) atomicAdd(&a.tri[x], (unsigned long long)(twice / 2));
+                twice = 0;
+            }
+        }
     }
 }
 
@@ -1350,7 +1456,10 @@ int local_triangle_features(g2_ctx* c, unsigned long long* tri, uint32_t* sup, u
     a.tri = tri;
     a.flag = flag;
     const uint64_t blocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, WK_GM_LOCAL) / kLocalBlockWaves);
+    a.factor = c->ne * 2 > kNearBytes ? kRevFactorFar : kRevFactor;
+    a.run = (uint32_t)std::min<uint64_t>(kFetchRun, std::max<uint64_t>(1, nv / (blocks * kLocalBlockWaves * 16)));
     hipLaunchKernelGGL(tri_kernel, dim3(blocks), dim3(kLocalBlockWaves * kWave), 0, c->stream, a);
+    hipLaunchKernelGGL(tri_block_kernel, dim3(c->num_cus * 4), dim3(512), 0, c->stream, a);
     const uint64_t wgrid = std::max<uint64_t>(1, (uint64_t)c->num_cus * 32 / 4);
     hipLaunchKernelGGL(sup_kernel, dim3(wgrid), dim3(256), 0, c->stream, orp, ocols, (const uint8_t*)flag, nv, sup);
     if ((e = hipGetLastError())) return hip_err(c, e, "triangle feature kernels");
