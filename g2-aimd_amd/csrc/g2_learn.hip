@@ -19,8 +19,9 @@
 //   weights and Adam.  A wave owns 16 samples: layer 1 is 4 MFMA tiles (K padded
 //   8 -> 16), layer 2 is 4x4 tiles, layer 3 a 16-lane reduction.  The backward
 //   pass forms dW2 = h1^T dh2, dW1 = x^T dh1 and dh1 = dh2 W2^T on the same
-//   instruction and accumulates each wave's gradient in registers before one
-//   atomic flush.
+//   instruction.  Small batches run an epoch in one launch of one workgroup
+//   (mlp_epoch_kernel); large ones take three launches a step, each wave's
+//   gradient in its own slot, added in a fixed order.
 #include <algorithm>
 #include <cmath>
 #include <random>
@@ -730,15 +731,373 @@ struct AdamArgs {
     float lr, b1, b2, eps, c1, c2;  // c1 = 1/(1-b1^t), c2 = 1/(1-b2^t)
 };
 
+__device__ __forceinline__ void adam_update(float g, float& p, float& m, float& v, float lr, float b1, float b2,
+                                            float eps, float c1, float c2) {
+    m = b1 * m + (1 - b1) * g;
+    v = b2 * v + (1 - b2) * g * g;
+    p -= lr * (m * c1) / (sqrtf(v * c2) + eps);
+}
+
 __global__ void adam_kernel(AdamArgs a) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < kNParam; i += gridDim.x * blockDim.x) {
-        const float g = a.grad[i];
-        const float m = a.b1 * a.m[i] + (1 - a.b1) * g;
-        const float v = a.b2 * a.v[i] + (1 - a.b2) * g * g;
-        a.m[i] = m;
-        a.v[i] = v;
-        a.params[i] -= a.lr * (m * a.c1) / (sqrtf(v * a.c2) + a.eps);
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < kNParam; i += gridDim.x * blockDim.x)
+        adam_update(a.grad[i], a.params[i], a.m[i], a.v[i], a.lr, a.b1, a.b2, a.eps, a.c1, a.c2);
+}
+
+// One epoch of small mini-batches in one launch of one workgroup.
+//
+// A step of the three kernels above is a chain of launches that each hold a few
+// CUs for microseconds (30 us a step of 512 samples: the launches, their
+// reloads of the weights and the slots' round trip through memory).  Here the
+// weights stay in LDS, the master copy and Adam's moments in registers, and a
+// step needs two barriers per 256 samples:
+//   * wave w takes tile w of a group of 16 tiles of 16 samples.  Activations
+//     are formed in both layouts (samples along the lanes, and along the
+//     registers) by swapping the operands of the same product, so each
+//     product's result is the next one's operand where it stands: the only LDS
+//     traffic of a tile is the weights' fragments (8 bytes a lane,
+//     consecutive lanes consecutive) and what the gradients need;
+//   * then wave w owns the 16 x 16 block (w / 4, w % 4) of W2 and adds the
+//     tiles' products in tile order, waves 0-3 a block of W1 each, waves 4-7
+//     the biases, W3 and the squared errors: the same products and the same
+//     order of sums as mlp_train_kernel and mlp_reduce_kernel, so the same
+//     parameters bit for bit;
+//   * the owners apply Adam and rewrite their fragments.
+// 50,001 samples, 3 epochs, whole call: batches of 16 (5,000 samples) 17.5 ->
+// 4.0 ms, of 100 33.5 -> 7.9, of 256 14.9 -> 4.5, of 512 8.9 -> 4.3, of 1024
+// 5.65 -> 4.1.  Bound by one CU's vector and LDS issue, 6.7 us a group.
+struct EpochArgs {
+    float *params, *m, *v;
+    const float* __restrict__ x;         // n x 8
+    const float* __restrict__ yt;        // n targets
+    const uint32_t* __restrict__ idx;    // the epoch's sample order
+    const float2* __restrict__ coef;     // per step: Adam's c1, c2
+    uint32_t n, batch;
+    float inv_batch, inv_last;           // 1 / samples of a step, of the last one
+    float lr, b1, b2, eps;
+    float* loss;                         // the epoch's sum of squared errors
+};
+
+constexpr uint32_t kEpochTiles = 16;     // tiles per group, one per wave
+// Largest batch that takes this path.  It costs the same 27 ns a sample at any
+// batch, the three kernels less and less as more CUs work on a step: 3 epochs
+// of 50,001 samples in batches of 1536 take 4.06 ms here and 4.65 there, in
+// batches of 2048 about 4.1 and 4.1, in batches of 4096 3.4 there.
+constexpr uint32_t kEpochBatch = 1536;
+
+struct EpochTile {
+    bf16x4 h[4][kWave];                  // layer-1 activations, dh2, dh1: register i of lane (q, r) holds
+    bf16x4 g[4][kWave];                  //   sample 4q + i, column 16t + r
+    bf16x4 d[4][kWave];
+    bf16x4 x[16][4];                     // inputs, K padded
+    float col[3][kH];                    // column sums: db1, db2, dW3
+    float gb3, sse;
+};
+
+struct alignas(16) EpochShared {
+    bf16x4 w2[4][4][kWave];              // [s][t]: register i of lane (q, r) holds W2[16s + 4q + i][16t + r]
+    bf16x4 w2t[4][4][kWave];             // [t][s]: W2[16t + r][16s + 4q + i]
+    bf16x4 w1[4][kWave];                 // [t]: W1[4q + i][16t + r], zero for 4q + i >= kIn
+    float b1[kH], b2[kH], w3[kH], b3;
+    EpochTile tile[kEpochTiles];
+};
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ bf16x4 pack4(float a, float b, float c, float d) {
+    const bf16x2_t lo = __builtin_convertvector((f32x2_t){a, b}, bf16x2_t);
+    const bf16x2_t hi = __builtin_convertvector((f32x2_t){c, d}, bf16x2_t);
+    uint32_t w[2];
+    __builtin_memcpy(&w[0], &lo, 4);
+    __builtin_memcpy(&w[1], &hi, 4);
+    bf16x4 r;
+    __builtin_memcpy(&r, w, 8);
+    return r;
+}
+
+// x plus lane (l + N) % 16's x within each row of 16 lanes; N = 8, 4, 2, 1 in
+// turn add the same pairs as xor shuffles do (after a step the values repeat
+// with period N)
+template <int N>
+__device__ __forceinline__ float add_ror(float x) {
+    return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x120 + N, 0xf, 0xf, false));
+}
+
+__global__ __launch_bounds__(1024) void mlp_epoch_kernel(EpochArgs a) {
+    __shared__ EpochShared S;
+    const uint32_t lane = lane_id(), r = lane % 16, q = lane / 16;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), wp = w / 4, wt = w % 4;
+    // the parameters this thread owns: four of W2, and extra ones (W1 by waves
+    // 0-3, b1, b2, W3 and b3 by waves 4-7)
+    float P[4], Mo[4], Vo[4], E[4] = {0, 0, 0, 0}, EM[4] = {0, 0, 0, 0}, EV[4] = {0, 0, 0, 0};
+    const uint32_t pi = oW2 + (16 * wp + 4 * q) * kH + 16 * wt + r;
+    uint32_t ei = 0, ne = 0;
+    if (w < 4) {
+        ei = oW1 + (4 * q) * kH + 16 * w + r;
+        ne = q < 2 ? 4 : 0;
+    } else if (w < 7) {
+        ei = (w == 4 ? oB1 : w == 5 ? oB2 : oW3) + lane;
+        ne = 1;
+    } else if (w == 7) {
+        ei = oB3;
+        ne = lane == 0 ? 1 : 0;
     }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+        P[i] = a.params[pi + i * kH];
+        Mo[i] = a.m[pi + i * kH];
+        Vo[i] = a.v[pi + i * kH];
+        if (i < ne) {
+            E[i] = a.params[ei + i * kH];
+            EM[i] = a.m[ei + i * kH];
+            EV[i] = a.v[ei + i * kH];
+        }
+    }
+    auto publish = [&]() {
+        const bf16x4 f = pack4(P[0], P[1], P[2], P[3]);
+        S.w2[wp][wt][lane] = f;
+        uint16_t* ft = (uint16_t*)&S.w2t[wp][wt][16 * (r / 4) + 4 * q] + r % 4;
+#pragma unroll
+        for (int i = 0; i < 4; i++) ft[4 * i] = (uint16_t)f[i];
+        if (w < 4) S.w1[w][lane] = pack4(E[0], E[1], E[2], E[3]);
+        else if (w == 4) S.b1[lane] = E[0];
+        else if (w == 5) S.b2[lane] = E[0];
+        else if (w == 6) S.w3[lane] = bf2f(f2bf(E[0]));
+        else if (w == 7 && lane == 0) S.b3 = E[0];
+    };
+    publish();
+
+    // a wave's tile of the next group is fetched one group ahead, its sample
+    // ids two groups ahead
+    const uint32_t group = 16 * kEpochTiles;
+    auto advance = [&](uint32_t& b0, uint32_t& g0) {  // next group: batch start, first sample within it
+        g0 += group;
+        if (g0 >= umin32(a.batch, a.n - b0)) {
+            b0 = a.n - b0 > a.batch ? b0 + a.batch : a.n;
+            g0 = 0;
+        }
+    };
+    constexpr uint32_t kNoSample = ~0u;
+    auto sample = [&](uint32_t b0, uint32_t g0) {
+        const uint32_t o = g0 + 16 * w + r;
+        return b0 < a.n && o < umin32(a.batch, a.n - b0) ? a.idx[b0 + o] : kNoSample;
+    };
+    auto fetch = [&](uint32_t s, float4& x, float& y) {
+        x = float4{0, 0, 0, 0};
+        y = 0;
+        if (s != kNoSample) {
+            if (q < 2) x = *(const float4*)(a.x + (uint64_t)s * kIn + 4 * q);
+            y = a.yt[s];
+        }
+    };
+    uint32_t nb = 0, ng = 0;             // the group whose sample ids are loaded next
+    float4 cx;
+    float cy;
+    fetch(sample(nb, ng), cx, cy);
+    advance(nb, ng);
+    uint32_t ns = nb < a.n ? sample(nb, ng) : kNoSample;
+    float loss = 0;
+    uint32_t step = 0;
+    __syncthreads();
+
+    for (uint32_t b0 = 0; b0 < a.n; step++) {
+        const uint32_t bn = umin32(a.batch, a.n - b0);
+        const float inv_n = bn == a.batch ? a.inv_batch : a.inv_last;
+        const float2 co = a.coef[step];
+        float sw[4] = {0, 0, 0, 0}, se[4] = {0, 0, 0, 0};
+        for (uint32_t g0 = 0; g0 < bn; g0 += group) {
+            // next group's inputs, and the ids of the one after
+            float4 nx;
+            float ny;
+            fetch(ns, nx, ny);
+            if (nb < a.n) advance(nb, ng);
+            ns = nb < a.n ? sample(nb, ng) : kNoSample;
+
+            if (g0 + 16 * w < bn) {
+                EpochTile& T = S.tile[w];
+                const bf16x4 ax = pack4(cx.x, cx.y, cx.z, cx.w);
+                T.x[r][q] = ax;
+                // layer 1, samples along the registers (ha) and along the lanes (ht)
+                bf16x4 ha[4], ht[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const bf16x4 f = S.w1[t][lane];
+                    const f32x4 za = mfma16(ax, f, f32x4{0, 0, 0, 0}), zt = mfma16(f, ax, f32x4{0, 0, 0, 0});
+                    const float ba = S.b1[16 * t + r];
+                    const float4 bt = *(const float4*)&S.b1[16 * t + 4 * q];
+                    auto relu = [](float z) { return z > 0 ? z : 0.f; };
+                    ha[t] = pack4(relu(za[0] + ba), relu(za[1] + ba), relu(za[2] + ba), relu(za[3] + ba));
+                    ht[t] = pack4(relu(zt[0] + bt.x), relu(zt[1] + bt.y), relu(zt[2] + bt.z), relu(zt[3] + bt.w));
+                    T.h[t][lane] = ha[t];
+                }
+                // layer 2 in both layouts
+                f32x4 h2[4], h2t[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    h2[t] = h2t[t] = f32x4{0, 0, 0, 0};
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        const bf16x4 f = S.w2[k][t][lane];
+                        h2[t] = mfma16(ht[k], f, h2[t]);
+                        h2t[t] = mfma16(f, ht[k], h2t[t]);
+                    }
+                }
+                float part[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float ba = S.b2[16 * t + r], w3 = S.w3[16 * t + r];
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const float z = h2[t][i] + ba;
+                        h2[t][i] = z > 0 ? z : 0;
+                        part[i] += h2[t][i] * w3;
+                    }
+                }
+                // errors and dy of samples 4q + i (every lane of the row of 16)
+                float dy[4], sse = 0, gb3 = 0;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float y = add_ror<1>(add_ror<2>(add_ror<4>(add_ror<8>(part[i])))) + S.b3;
+                    const float yt = __shfl(cy, (int)(4 * q + i), kWave);
+                    const float e = g0 + 16 * w + 4 * q + i < bn ? y - yt : 0.f;
+                    // (mlp_train_kernel's contractions, spelt out)
+                    sse = __builtin_fmaf(e, e, sse);
+                    dy[i] = 2.0f * e * inv_n;
+                    gb3 = __builtin_fmaf(inv_n, 2.0f * e, gb3);
+                }
+                sse += __shfl_xor(sse, 32, kWave);
+                gb3 += __shfl_xor(gb3, 32, kWave);
+                sse += __shfl_xor(sse, 16, kWave);
+                gb3 += __shfl_xor(gb3, 16, kWave);
+                if (lane == 0) {
+                    T.gb3 = gb3;
+                    T.sse = sse;
+                }
+                float dyr = 0;  // dy of sample r
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const float d = __shfl(dy[i], (int)(16 * (r / 4)), kWave);
+                    dyr = (int)(r % 4) == i ? d : dyr;
+                }
+                // dh2 in both layouts; columns of dW3 and db2
+                float col[3][4];
+                bf16x4 gt[4];
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    const float w3 = S.w3[16 * t + r];
+                    const float4 w3t = *(const float4*)&S.w3[16 * t + 4 * q];
+                    const float4 b2t = *(const float4*)&S.b2[16 * t + 4 * q];
+                    float g[4], col3 = 0, colb = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        g[i] = h2[t][i] > 0 ? dy[i] * w3 : 0.f;
+                        col3 += h2[t][i] * dy[i];
+                        colb += g[i];
+                    }
+                    T.g[t][lane] = pack4(g[0], g[1], g[2], g[3]);
+                    col[2][t] = col3;
+                    col[1][t] = colb;
+                    gt[t] = pack4(h2t[t][0] + b2t.x > 0 ? dyr * w3t.x : 0.f, h2t[t][1] + b2t.y > 0 ? dyr * w3t.y : 0.f,
+                                  h2t[t][2] + b2t.z > 0 ? dyr * w3t.z : 0.f, h2t[t][3] + b2t.w > 0 ? dyr * w3t.w : 0.f);
+                }
+                // dh1 masked by layer 1's ReLU; columns of db1
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    f32x4 d1 = f32x4{0, 0, 0, 0};
+#pragma unroll
+                    for (int k = 0; k < 4; k++) d1 = mfma16(gt[k], S.w2t[t][k][lane], d1);
+                    float g[4], colb = 0;
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        g[i] = ha[t][i] > 0 ? d1[i] : 0.f;  // (a bf16 pattern of a value >= 0: positive as an integer, too)
+                        colb += g[i];
+                    }
+                    T.d[t][lane] = pack4(g[0], g[1], g[2], g[3]);
+                    col[0][t] = colb;
+                }
+                // column sums over the four q: (q0 + q1) + (q2 + q3).  Each
+                // step halves the columns a lane keeps: t = 2 (q % 2) + q / 2
+#pragma unroll
+                for (int k = 0; k < 3; k++) {
+                    const bool odd = q & 1, high = q & 2;
+                    const float c0 = odd ? col[k][2] : col[k][0], c1 = odd ? col[k][3] : col[k][1];
+                    const float o0 = odd ? col[k][0] : col[k][2], o1 = odd ? col[k][1] : col[k][3];
+                    const float s0 = c0 + __shfl_xor(o0, 16, kWave), s1 = c1 + __shfl_xor(o1, 16, kWave);
+                    const float v = (high ? s1 : s0) + __shfl_xor(high ? s0 : s1, 32, kWave);
+                    T.col[k][16 * (2 * (q & 1) + q / 2) + r] = v;
+                }
+            }
+            cx = nx;
+            cy = ny;
+            __syncthreads();
+            // the owners add the group's tiles in tile order
+            const uint32_t nt = umin32((bn - g0 + 15) / 16, kEpochTiles);
+            for (uint32_t k = 0; k < nt; k += 4) {  // (four tiles' operands in flight; past the last one, its own again)
+                bf16x4 h[4], g[4];
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++) {
+                    h[j] = S.tile[umin32(k + j, nt - 1)].h[wp][lane];
+                    g[j] = S.tile[umin32(k + j, nt - 1)].g[wt][lane];
+                }
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++) {
+                    const f32x4 d = mfma16(h[j], g[j], f32x4{0, 0, 0, 0});
+                    if (k + j < nt)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) sw[i] += d[i];
+                }
+            }
+            if (w < 4) {
+                for (uint32_t k = 0; k < nt; k += 4) {
+                    bf16x4 x[4], g[4];
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; j++) {
+                        const EpochTile& T = S.tile[umin32(k + j, nt - 1)];
+                        const uint16_t* xs = (const uint16_t*)&T.x[4 * q][0] + r;
+#pragma unroll
+                        for (int i = 0; i < 4; i++) x[j][i] = (short)xs[16 * i];
+                        g[j] = T.d[w][lane];
+                    }
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; j++) {
+                        const f32x4 d = mfma16(x[j], g[j], f32x4{0, 0, 0, 0});
+                        if (k + j < nt)
+#pragma unroll
+                            for (int i = 0; i < 4; i++) se[i] += d[i];
+                    }
+                }
+            } else if (w < 7) {
+#pragma unroll 4
+                for (uint32_t k = 0; k < nt; k++) se[0] += S.tile[k].col[w - 4][lane];
+            } else if (w == 7) {
+                for (uint32_t k = 0; k < nt; k++) {
+                    se[0] += S.tile[k].gb3;
+                    se[1] += S.tile[k].sse;
+                }
+            }
+            if (g0 + group < bn) __syncthreads();  // (the last group's barrier follows the new weights)
+        }
+        loss += se[1];  // (wave 7)
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            adam_update(sw[i], P[i], Mo[i], Vo[i], a.lr, a.b1, a.b2, a.eps, co.x, co.y);
+            if (i < ne) adam_update(se[i], E[i], EM[i], EV[i], a.lr, a.b1, a.b2, a.eps, co.x, co.y);
+        }
+        publish();
+        __syncthreads();
+        b0 = a.n - b0 > a.batch ? b0 + a.batch : a.n;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < 4; i++) {
+        a.params[pi + i * kH] = P[i];
+        a.m[pi + i * kH] = Mo[i];
+        a.v[pi + i * kH] = Vo[i];
+        if (i < ne) {
+            a.params[ei + i * kH] = E[i];
+            a.m[ei + i * kH] = EM[i];
+            a.v[ei + i * kH] = EV[i];
+        }
+    }
+    if (w == 7 && lane == 0) *a.loss = loss;
 }
 
 }  // namespace g2
@@ -751,6 +1110,9 @@ struct g2_mlp {
     float* partial = nullptr;  // per-wave partial gradients of one training launch
     uint64_t partial_waves = 0;
     uint32_t* idx = nullptr;
+    float2* coef = nullptr;    // Adam's step corrections of one epoch
+    uint64_t coef_cap = 0;
+    hipEvent_t copied = nullptr;  // an epoch's order has left the host
     uint64_t cap = 0;
     uint64_t step = 0;
     uint32_t num_cus = 256;
@@ -798,6 +1160,11 @@ static int mlp_train_launch(g2_mlp* M, MlpArgs a) {
     hipLaunchKernelGGL(mlp_reduce_kernel, dim3((kNParam + 1 + 255) / 256), dim3(256), 0, M->stream, M->partial,
                        (uint32_t)waves, a.grad, a.loss);
     return hipGetLastError() == hipSuccess ? G2_OK : G2_EHIP;
+}
+
+// Adam's corrections of step t: 1 / (1 - b1^t), 1 / (1 - b2^t)
+static float2 adam_coef(float b1, float b2, uint64_t t) {
+    return {1.f / (1.f - std::pow(b1, (float)t)), 1.f / (1.f - std::pow(b2, (float)t))};
 }
 
 extern "C" {
@@ -883,7 +1250,7 @@ int g2_mlp_create(g2_mlp** out, int device, uint64_t seed) {
     }
     hipDeviceProp_t p;
     if (hipGetDeviceProperties(&p, device) == hipSuccess) M->num_cus = p.multiProcessorCount;
-    if (hipMalloc(&M->params, kNParam * 4) || hipMalloc(&M->grad, kNParam * 4) || hipMalloc(&M->m, kNParam * 4) ||
+    if (hipEventCreateWithFlags(&M->copied, hipEventDisableTiming) || hipMalloc(&M->params, kNParam * 4) || hipMalloc(&M->grad, kNParam * 4) || hipMalloc(&M->m, kNParam * 4) ||
         hipMalloc(&M->v, kNParam * 4) || hipMalloc(&M->loss, 4)) {
         g2_mlp_destroy(M);
         return G2_EHIP;
@@ -911,8 +1278,9 @@ void g2_mlp_destroy(g2_mlp* M) {
     if (!M) return;
     (void)hipSetDevice(M->device);
     for (void* p : {(void*)M->params, (void*)M->grad, (void*)M->m, (void*)M->v, (void*)M->loss, (void*)M->x,
-                    (void*)M->y, (void*)M->out, (void*)M->idx, (void*)M->partial})
+                    (void*)M->y, (void*)M->out, (void*)M->idx, (void*)M->partial, (void*)M->coef})
         if (p) (void)hipFree(p);
+    if (M->copied) (void)hipEventDestroy(M->copied);
     if (M->stream) (void)hipStreamDestroy(M->stream);
     delete M;
 }
@@ -968,10 +1336,42 @@ int g2_mlp_train(g2_mlp* M, const float* x, const float* y, uint64_t n, uint32_t
     if (hipMemcpyAsync(M->x, x, n * kIn * 4, hipMemcpyHostToDevice, M->stream) ||
         hipMemcpyAsync(M->y, y, n * 4, hipMemcpyHostToDevice, M->stream))
         return G2_EHIP;
+    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     std::vector<uint32_t> perm(n);
     for (uint64_t i = 0; i < n; i++) perm[i] = (uint32_t)i;
+    const bool small = batch <= kEpochBatch && n < (1ull << 31);
+    const uint64_t steps = (n + batch - 1) / batch;
+    std::vector<float2> coef;
+    if (small && steps > M->coef_cap) {
+        if (M->coef) (void)hipFree(M->coef);
+        M->coef = nullptr;
+        M->coef_cap = 0;
+        if (hipMalloc(&M->coef, steps * sizeof(float2)) != hipSuccess) {
+            M->coef = nullptr;
+            return G2_EHIP;
+        }
+        M->coef_cap = steps;
+    }
     float last = 0;
     for (uint32_t ep = 0; ep < epochs; ep++) {
+        if (small) {
+            // one launch per epoch; the next epoch's order is shuffled while it
+            // runs, once this one's copy has left the host
+            if (ep && hipEventSynchronize(M->copied)) return G2_EHIP;
+            std::shuffle(perm.begin(), perm.end(), M->rng);
+            coef.resize(steps);
+            for (uint64_t s = 0; s < steps; s++) coef[s] = adam_coef(b1, b2, M->step + 1 + s);
+            if (hipMemcpyAsync(M->idx, perm.data(), n * 4, hipMemcpyHostToDevice, M->stream) ||
+                hipMemcpyAsync(M->coef, coef.data(), steps * sizeof(float2), hipMemcpyHostToDevice, M->stream) ||
+                hipEventRecord(M->copied, M->stream))
+                return G2_EHIP;
+            M->step += steps;
+            EpochArgs a{M->params, M->m, M->v, M->x, M->y, M->idx, M->coef, (uint32_t)n, batch, 1.f / batch,
+                        1.f / (n - (steps - 1) * batch), lr, b1, b2, eps, M->loss};
+            hipLaunchKernelGGL(mlp_epoch_kernel, dim3(1), dim3(1024), 0, M->stream, a);
+            if (hipGetLastError() != hipSuccess) return G2_EHIP;
+            continue;
+        }
         std::shuffle(perm.begin(), perm.end(), M->rng);
         if (hipMemcpyAsync(M->idx, perm.data(), n * 4, hipMemcpyHostToDevice, M->stream) ||
             hipMemsetAsync(M->loss, 0, 4, M->stream))
@@ -981,12 +1381,17 @@ int g2_mlp_train(g2_mlp* M, const float* x, const float* y, uint64_t n, uint32_t
             MlpArgs a{M->params, M->x, M->y, M->idx + b0, bn, 1.f / bn, M->grad, M->loss, nullptr, nullptr};
             if (mlp_train_launch(M, a)) return G2_EHIP;
             M->step++;
-            const float b1 = 0.9f, b2 = 0.999f;
-            AdamArgs ad{M->params, M->grad, M->m, M->v, lr, b1, b2, 1e-8f,
-                        1.f / (1.f - std::pow(b1, (float)M->step)), 1.f / (1.f - std::pow(b2, (float)M->step))};
+            const float2 co = adam_coef(b1, b2, M->step);
+            AdamArgs ad{M->params, M->grad, M->m, M->v, lr, b1, b2, eps, co.x, co.y};
             hipLaunchKernelGGL(adam_kernel, dim3(8), dim3(256), 0, M->stream, ad);
             if (hipGetLastError() != hipSuccess) return G2_EHIP;
         }
+        float sse = 0;
+        if (hipMemcpyAsync(&sse, M->loss, 4, hipMemcpyDeviceToHost, M->stream) || hipStreamSynchronize(M->stream))
+            return G2_EHIP;
+        last = sse / n;
+    }
+    if (small && epochs) {
         float sse = 0;
         if (hipMemcpyAsync(&sse, M->loss, 4, hipMemcpyDeviceToHost, M->stream) || hipStreamSynchronize(M->stream))
             return G2_EHIP;
