@@ -47,8 +47,8 @@
 //      position is a popcount over the words its order range leaves.
 // The roots go through passes, each taking the roots the previous one
 // deferred: one wave per root with the rows in the wave's LDS (|U| <= 149);
-// one workgroup per root with the rows in the workgroup's LDS (|U| <= 448, 700, 1039); one wave per root with the rows in
-// a global arena sized to the largest remaining root.
+// one workgroup per root with the rows in the workgroup's LDS (|U| <= 448, 700, 1039); several workgroups per root with the
+// rows in a global arena.
 #include <algorithm>
 #include <vector>
 
@@ -610,37 +610,35 @@ __device__ __forceinline__ void count_root(const LocalProgram& P, uint32_t m, co
     const uint32_t lane = lane_id();
     const uint32_t W = row_stride(m);
     if constexpr (CLQ && N > 4) {
-        if (queue) {
-            const uint32_t nw = (m + 63) >> 6;
-            uint32_t k = 0;
-            auto drain = [&](uint32_t nq) {
-                wave_sync();
-                if (lane < nq) {
-                    const uint32_t e = queue[lane];
-                    uint32_t off[N];
-                    off[1] = (e >> 16) * W;
-                    off[2] = (e & 0xffffu) * W;
-                    nodes++;
-                    clique_walk<N, 3>(rows, W, nw, off, e & 0xffffu, lane_total, nodes);
-                }
-                wave_sync();
-            };
-            for (uint32_t r1 = 0; r1 < m; r1++) {
-                for (uint32_t w = r1 >> 6; w < nw; w++) {
-                    const uint64_t cw = uniform(rows[r1 * W + w]);
-                    const uint32_t cnt = (uint32_t)__popcll(cw);
-                    if (k + cnt > kWave) {
-                        drain(k);
-                        k = 0;
-                    }
-                    if ((cw >> lane) & 1) queue[k + lanes_below(cw)] = (r1 << 16) | (w * 64 + lane);
-                    k += cnt;
-                }
+        const uint32_t nw = (m + 63) >> 6;
+        uint32_t k = 0;
+        auto drain = [&](uint32_t nq) {
+            wave_sync();
+            if (lane < nq) {
+                const uint32_t e = queue[lane];
+                uint32_t off[N];
+                off[1] = (e >> 16) * W;
+                off[2] = (e & 0xffffu) * W;
+                nodes++;
+                clique_walk<N, 3>(rows, W, nw, off, e & 0xffffu, lane_total, nodes);
             }
-            if (k) drain(k);
-            if (lane == 0) nodes += m;
-            return;
+            wave_sync();
+        };
+        for (uint32_t r1 = 0; r1 < m; r1++) {
+            for (uint32_t w = r1 >> 6; w < nw; w++) {
+                const uint64_t cw = uniform(rows[r1 * W + w]);
+                const uint32_t cnt = (uint32_t)__popcll(cw);
+                if (k + cnt > kWave) {
+                    drain(k);
+                    k = 0;
+                }
+                if ((cw >> lane) & 1) queue[k + lanes_below(cw)] = (r1 << 16) | (w * 64 + lane);
+                k += cnt;
+            }
         }
+        if (k) drain(k);
+        if (lane == 0) nodes += m;
+        return;
     }
     if constexpr (CLQ) {
         const uint32_t nw = (m + 63) >> 6;
@@ -657,6 +655,46 @@ __device__ __forceinline__ void count_root(const LocalProgram& P, uint32_t m, co
             nodes++;
             walk_from<N>(P, M, 2, rows, W, m, lane_total, nodes);
         }
+    }
+}
+
+// Matches of one position-1 candidate r1 on one wave: its position-2
+// candidates, 64 at a time in the queue, one per lane.
+template <int N>
+__device__ __forceinline__ void count_first(const LocalProgram& P, uint32_t r1, uint32_t m, uint32_t W, const uint64_t* rows,
+                                            uint32_t* queue, uint64_t& lane_total, uint64_t& nodes) {
+    const uint32_t lane = lane_id();
+    uint32_t M[N];
+    M[1] = r1;
+    if (lane == 0) nodes++;
+    uint32_t plo, phi;
+    cand_range(P, 2, M, m, &plo, &phi);
+    if (plo >= phi) return;
+    if constexpr (N == 3) {
+        for (uint32_t w = (plo >> 6) + lane; w <= (phi - 1) >> 6; w += kWave)
+            lane_total += __popcll(cand_word(P, 2, M, rows, W, plo, phi, w));
+    } else {
+        uint32_t k = 0;
+        auto drain_queue = [&](uint32_t nq) {
+            wave_sync();
+            if (lane < nq) {
+                M[2] = queue[lane];
+                nodes++;
+                walk_from<N>(P, M, 3, rows, W, m, lane_total, nodes);
+            }
+            wave_sync();
+        };
+        for (uint32_t w = plo >> 6; w <= (phi - 1) >> 6; w++) {
+            const uint64_t cw = cand_word(P, 2, M, rows, W, plo, phi, w);
+            const uint32_t cnt = (uint32_t)__popcll(cw);
+            if (k + cnt > kWave) {
+                drain_queue(k);
+                k = 0;
+            }
+            if ((cw >> lane) & 1) queue[k + lanes_below(cw)] = w * 64 + lane;
+            k += cnt;
+        }
+        if (k) drain_queue(k);
     }
 }
 
@@ -714,21 +752,6 @@ __device__ __forceinline__ void wave_root(const LocalArgs& a, uint64_t lo, uint3
     }
 }
 
-// One root whose rows lie in a global arena.
-template <int N, bool CLQ>
-__device__ __forceinline__ void arena_root(const LocalArgs& a, uint64_t lo, uint32_t m, uint64_t* rows, uint64_t& lane_total,
-                                           uint64_t& nodes) {
-    const uint32_t W = row_stride(m);
-    for (uint64_t i = lane_id(); i < (uint64_t)m * W; i += kWave) rows[i] = 0;
-    wave_sync();
-    for (uint32_t a0 = 0; a0 + 1 < m; a0 += kWave) {
-        uint32_t unused = 0;
-        build_chunk<CLQ ? 1 : 0>(a, a.ocols + lo, rows, m, W, a0, 0, unused);
-        wave_sync();  // (the chunk's atomics complete before the walk reads rows)
-    }
-    count_root<N, CLQ>(a.prog, m, rows, nullptr, lane_total, nodes);
-}
-
 // Pass 1: roots whose rows fit the wave's LDS (the others are passed over:
 // they are on the other passes' lists).  Roots are taken from the top rank
 // down: the roots with the largest local graphs sit in the upper middle of the
@@ -784,30 +807,6 @@ __global__ __launch_bounds__(256, 7) void gm_local_kernel(LocalArgs a) {
                 wave_root<N, CLQ>(a, clo, cm, lds[wid], lane_total, nodes);
             }
         }
-    }
-    const uint64_t tot = wave_sum(lane_total);
-    const uint64_t nd = wave_sum(nodes);
-    if (lane == 0) {
-        if (tot) atomicAdd(&a.ctr[LCTR_COUNT], (unsigned long long)tot);
-        if (nd) atomicAdd(&a.ctr[LCTR_NODES], (unsigned long long)nd);
-    }
-}
-
-// Last pass: the roots too large for a workgroup's LDS, rows in per-wave
-// global arenas of scratch_words (the largest root's need).
-template <int N, bool CLQ>
-__global__ __launch_bounds__(256, 4) void gm_local_arena_kernel(LocalArgs a) {
-    const uint32_t lane = lane_id();
-    const uint64_t gwave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave;
-    uint64_t* ws = a.scratch + gwave * a.scratch_words;
-    uint64_t lane_total = 0, nodes = 0;
-    while (true) {
-        const uint64_t t = fetch_task(&a.ctr[LCTR_NEXT + a.pass]);
-        if (t >= a.ntasks) break;
-        const uint32_t x = uniform(a.list[t]);
-        const uint64_t lo = uniform(a.orp[x]);
-        const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
-        arena_root<N, CLQ>(a, lo, m, ws, lane_total, nodes);
     }
     const uint64_t tot = wave_sum(lane_total);
     const uint64_t nd = wave_sum(nodes);
@@ -955,45 +954,132 @@ __global__ __launch_bounds__(BT, block_waves(N, CLQ, BU)) void gm_local_block_ke
             if (tid == 0) nodes += m;
             continue;
         }
-        uint32_t M[N];
         while (true) {
             __builtin_amdgcn_wave_barrier();
             uint32_t r1 = 0;
             if (lane == 0) r1 = atomicAdd(&s_next, 1u);
             r1 = uniform(r1);
             if (r1 >= m) break;
-            M[1] = r1;
+            count_first<N>(P, r1, m, W, rows, queue[wid], lane_total, nodes);
+        }
+    }
+    const uint64_t tot = wave_sum(lane_total);
+    const uint64_t nd = wave_sum(nodes);
+    if (lane == 0) {
+        if (tot) atomicAdd(&a.ctr[LCTR_COUNT], (unsigned long long)tot);
+        if (nd) atomicAdd(&a.ctr[LCTR_NODES], (unsigned long long)nd);
+    }
+}
+
+// Last pass: the roots too large for a workgroup's LDS, rows in global arenas of
+// scratch_words each (the largest root's need).  Such a root is the launch's
+// critical path: one wave per root held R-MAT 22's 4-cliques for 17.8 ms of
+// 51.5 where the draw has a single root of 1,049 members, which takes 0.06 ms
+// here (passes on LDS rows end at 1,039 members).  A root is
+// spread over gridDim.x workgroups in each of two launches, the arenas cleared
+// before: they build its rows (members dealt over all their waves; each
+// workgroup has the hash index over U, or, beyond kWideU members, searches U
+// itself), then count it (position-1 candidates dealt over their waves).
+constexpr int kWideThreads = 512, kWideCountThreads = 256;
+constexpr uint32_t kWideU = 8190;
+static_assert(kWideU * 4 <= kMember4, "members fit an entry");
+
+template <bool CLQ>
+__global__ __launch_bounds__(kWideThreads) void gm_local_wide_build_kernel(LocalArgs a) {
+    __shared__ __align__(16) uint16_t slot[kSlots];
+    __shared__ uint16_t next[kWideU];
+    __shared__ uint32_t U[kWideU + 1];
+    const HashIndex<kSlots, kWideU> H{slot, next, U};
+    const uint32_t x = uniform(a.list[blockIdx.y]);
+    const uint64_t lo = uniform(a.orp[x]);
+    const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - lo);
+    const uint32_t W = row_stride(m);
+    uint64_t* rows = a.scratch + blockIdx.y * a.scratch_words;
+    const uint32_t waves = gridDim.x * (kWideThreads / kWave);
+    const uint32_t first = uniform(blockIdx.x * (kWideThreads / kWave) + threadIdx.x / kWave);
+    if (m <= kWideU) {
+        H.clear(threadIdx.x, kWideThreads);
+        __syncthreads();
+        for (uint32_t i = threadIdx.x; i < m; i += kWideThreads) H.put(i, a.ocols[lo + i]);
+        __syncthreads();
+        for (uint64_t i0 = first; i0 + 1 < m; i0 += (uint64_t)waves * kWave)
+            build_rows<kVecs>(a, H, m, lo, (uint32_t)i0, waves, kRevFactor, [&](uint32_t ia, uint32_t ib, uint32_t) {
+                set_row_bit(rows, (uint64_t)ia * W + (ib >> 6), ib);
+                if constexpr (!CLQ) set_row_bit(rows, (uint64_t)ib * W + (ia >> 6), ia);
+            });
+    } else {
+        for (uint64_t a0 = (uint64_t)first * kWave; a0 + 1 < m; a0 += (uint64_t)waves * kWave) {
+            uint32_t unused = 0;
+            build_chunk<CLQ ? 1 : 0>(a, a.ocols + lo, rows, m, W, (uint32_t)a0, 0, unused);
+        }
+    }
+}
+
+template <int N, bool CLQ>
+__global__ __launch_bounds__(kWideCountThreads) void gm_local_wide_count_kernel(LocalArgs a) {
+    __shared__ uint32_t queues[kWideCountThreads / kWave][kWave];
+    const uint32_t lane = lane_id();
+    const uint32_t wid = uniform(threadIdx.x / kWave);
+    uint32_t* queue = queues[wid];
+    const uint32_t x = uniform(a.list[blockIdx.y]);
+    const uint32_t m = (uint32_t)(uniform(a.orp[x + 1]) - uniform(a.orp[x]));
+    const uint32_t W = row_stride(m), nw = (m + 63) >> 6;
+    const uint64_t* rows = a.scratch + blockIdx.y * a.scratch_words;
+    const uint32_t waves = gridDim.x * (kWideCountThreads / kWave);
+    uint64_t lane_total = 0, nodes = 0;
+    for (uint64_t r = (uint64_t)blockIdx.x * (kWideCountThreads / kWave) + wid; r < m; r += waves) {
+        const uint32_t r1 = (uint32_t)r;
+        if constexpr (!CLQ) {
+            count_first<N>(a.prog, r1, m, W, rows, queue, lane_total, nodes);
+        } else if constexpr (N == 3) {
+            for (uint32_t w = (r1 >> 6) + lane; w < nw; w += kWave) lane_total += __popcll(rows[(uint64_t)r1 * W + w]);
             if (lane == 0) nodes++;
-            uint32_t plo, phi;
-            cand_range(P, 2, M, m, &plo, &phi);
-            if (plo >= phi) continue;
-            if constexpr (N == 3) {
-                for (uint32_t w = (plo >> 6) + lane; w <= (phi - 1) >> 6; w += kWave)
-                    lane_total += __popcll(cand_word(P, 2, M, rows, W, plo, phi, w));
-            } else {
-                // position-2 candidates of r1, 64 at a time
-                uint32_t k = 0;
-                auto drain_queue = [&](uint32_t nq) {
-                    wave_sync();
-                    if (lane < nq) {
-                        M[2] = queue[wid][lane];
-                        nodes++;
-                        walk_from<N>(P, M, 3, rows, W, m, lane_total, nodes);
+        } else {
+            if (lane == 0) nodes++;
+            const uint32_t base = r1 * W;
+            uint32_t k = 0;
+            auto drain_queue = [&](uint32_t nq) {
+                wave_sync();
+                if (lane < nq) {
+                    const uint32_t r2 = queue[lane];
+                    if constexpr (N == 4) {
+                        // four words of both rows in flight (past the last one, that one again, uncounted)
+                        uint32_t c = 0;
+                        for (uint32_t w = r2 >> 6; w < nw; w += 4) {
+                            uint64_t y[4];
+#pragma unroll
+                            for (uint32_t j = 0; j < 4; j++) {
+                                const uint32_t at = umin32(w + j, nw - 1);
+                                y[j] = rows[base + at] & rows[r2 * W + at];
+                            }
+#pragma unroll
+                            for (uint32_t j = 0; j < 4; j++) c += w + j < nw ? (uint32_t)__popcll(y[j]) : 0u;
+                        }
+                        lane_total += c;
+                    } else {
+                        uint32_t off[N];
+                        off[1] = base;
+                        off[2] = r2 * W;
+                        clique_walk<N, 3>(rows, W, nw, off, r2, lane_total, nodes);
                     }
-                    wave_sync();
-                };
-                for (uint32_t w = plo >> 6; w <= (phi - 1) >> 6; w++) {
-                    const uint64_t cw = cand_word(P, 2, M, rows, W, plo, phi, w);
+                }
+                if (lane == 0) nodes += nq;
+                wave_sync();
+            };
+            for (uint32_t w0 = (r1 >> 6) & ~63u; w0 < nw; w0 += kWave) {
+                const uint64_t own = w0 + lane < nw ? rows[base + w0 + lane] : 0;
+                for (uint32_t w = w0; w < umin32(w0 + kWave, nw); w++) {
+                    const uint64_t cw = read_lane(own, w - w0);
                     const uint32_t cnt = (uint32_t)__popcll(cw);
                     if (k + cnt > kWave) {
                         drain_queue(k);
                         k = 0;
                     }
-                    if ((cw >> lane) & 1) queue[wid][k + lanes_below(cw)] = w * 64 + lane;
+                    if ((cw >> lane) & 1) queue[k + lanes_below(cw)] = w * 64 + lane;
                     k += cnt;
                 }
-                if (k) drain_queue(k);
             }
+            if (k) drain_queue(k);
         }
     }
     const uint64_t tot = wave_sum(lane_total);
@@ -1551,10 +1637,11 @@ void gm_local_compile(g2_ctx* c, const g2_plan* p) {
     c->local_ok = true;
 }
 
-enum class LocalPass { Wave, Group1, Group2, Group3, Arena };
+enum class LocalPass { Wave, Group1, Group2, Group3, WideBuild, WideCount };
 
 template <int N, bool CLQ>
 static void launch_local(LocalPass pass, uint64_t blocks, uint32_t bw, hipStream_t s, const LocalArgs& a) {
+    // (the last pass: `blocks` workgroups for each of its roots)
     if constexpr (N > 2) {
         switch (pass) {
             case LocalPass::Group1:
@@ -1569,8 +1656,12 @@ static void launch_local(LocalPass pass, uint64_t blocks, uint32_t bw, hipStream
                 hipLaunchKernelGGL((gm_local_block_kernel<N, CLQ, kB3Threads, kB3RowWords, kB3U>), dim3(blocks),
                                    dim3(kB3Threads), 0, s, a);
                 return;
-            case LocalPass::Arena:
-                hipLaunchKernelGGL((gm_local_arena_kernel<N, CLQ>), dim3(blocks), dim3(bw * kWave), 0, s, a);
+            case LocalPass::WideBuild:
+                hipLaunchKernelGGL((gm_local_wide_build_kernel<CLQ>), dim3(blocks, (unsigned)a.ntasks), dim3(kWideThreads), 0, s, a);
+                return;
+            case LocalPass::WideCount:
+                hipLaunchKernelGGL((gm_local_wide_count_kernel<N, CLQ>), dim3(blocks, (unsigned)a.ntasks),
+                                   dim3(kWideCountThreads), 0, s, a);
                 return;
             default:
                 break;
@@ -1615,8 +1706,7 @@ static int pass_roots(g2_ctx* c, const uint64_t* orp, const uint32_t* rank, uint
 }
 
 // Passes over the roots: rows in a wave's LDS; in three sizes of workgroup LDS;
-// in per-wave global arenas sized to the largest
-// root left.  Which roots a pass takes is known before the first one starts,
+// in global arenas sized to the largest root.  Which roots a pass takes is known before the first one starts,
 // so the passes are enqueued back to back and waited for once.
 int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     if (c->nv + 1 > 0x7fffffffull) return set_err(c, G2_EINVAL, "local-bitmap matching supports fewer than 2^31-1 vertices");
@@ -1654,12 +1744,13 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
         roots[k] = c->pass_count[k];
         roots[0] -= roots[k];
     }
-    // last pass: per-wave global arenas
-    uint64_t bwaves = std::min<uint64_t>(std::max<uint32_t>(c->tune.big_waves, 1), roots[kPasses - 1]);
-    if (bwaves) {
-        while (bwaves > 1 && c->budget && c->used - c->big_scratch.bytes + bwaves * c->pass_need * 8 > c->budget) bwaves /= 2;
-        bwaves = (bwaves + bw - 1) / bw * bw;
-        if ((rc = ensure(c, c->big_scratch, bwaves * c->pass_need * 8, "large-root arenas"))) return rc;
+    // last pass: a global arena for each of its roots, for as many at a time as
+    // the budget allows
+    uint64_t arenas = std::min<uint64_t>(std::max<uint32_t>(c->tune.big_waves, 1), roots[kPasses - 1]);
+    if (arenas) {
+        arenas = std::min<uint64_t>(arenas, 65535);  // (one grid row each)
+        while (arenas > 1 && c->budget && c->used - c->big_scratch.bytes + arenas * c->pass_need * 8 > c->budget) arenas /= 2;
+        if ((rc = ensure(c, c->big_scratch, arenas * c->pass_need * 8, "large-root arenas"))) return rc;
     }
     if ((e = hipMemsetAsync(ctr, 0, LCTR_N * 8, c->stream))) return hip_err(c, e, "memset counters");
     LocalArgs a{};
@@ -1690,7 +1781,7 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
         {LocalPass::Group1, (uint64_t)c->num_cus * kB1PerCu},
         {LocalPass::Group2, (uint64_t)c->num_cus * kB2PerCu},
         {LocalPass::Group3, (uint64_t)c->num_cus * (tri ? 2 : kB3PerCu)},
-        {LocalPass::Arena, bwaves / bw}};
+        {LocalPass::WideBuild, 0}};
     int pass_ev[kPasses] = {-1, -1, -1, -1, -1};
     for (int k = 0; k < kPasses; k++) {
         if (k && !roots[k]) continue;
@@ -1704,11 +1795,25 @@ int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
             a.ntasks = roots[k];
             list += roots[k];
         }
-        a.scratch = (uint64_t*)c->big_scratch.ptr;
-        a.scratch_words = c->pass_need;
-        // (a workgroup takes one root at a time; a wave of the others up to a run)
-        const uint64_t blocks = k == kPasses - 1 ? shape[k].most : std::min<uint64_t>(shape[k].most, std::max<uint64_t>(a.ntasks, 1));
-        if ((e = launch(shape[k].pass, blocks))) return hip_err(c, e, "local launch");
+        if (k < kPasses - 1) {
+            // (a workgroup takes one root at a time; a wave of the first pass up to a run)
+            if ((e = launch(shape[k].pass, std::min<uint64_t>(shape[k].most, std::max<uint64_t>(a.ntasks, 1)))))
+                return hip_err(c, e, "local launch");
+        } else {
+            a.scratch = (uint64_t*)c->big_scratch.ptr;
+            a.scratch_words = c->pass_need;
+            for (uint64_t done = 0; done < roots[k]; done += a.ntasks, a.list += a.ntasks) {
+                a.ntasks = std::min<uint64_t>(arenas, roots[k] - done);
+                if ((e = hipMemsetAsync(a.scratch, 0, a.ntasks * a.scratch_words * 8, c->stream)))
+                    return hip_err(c, e, "memset arenas");
+                // workgroups per root: enough to fill the device, each at least a few members
+                const uint64_t members = c->pass_need / row_stride(1040) + 1;
+                for (const auto& w : {std::make_pair(LocalPass::WideBuild, 2u), std::make_pair(LocalPass::WideCount, 8u)}) {
+                    const uint64_t fill = ((uint64_t)c->num_cus * w.second + a.ntasks - 1) / a.ntasks;
+                    if ((e = launch(w.first, std::min<uint64_t>(fill, members / 8 + 1)))) return hip_err(c, e, "local launch");
+                }
+            }
+        }
         pass_ev[k] = nev;
         if ((rc = mark())) return rc;
     }
