@@ -263,6 +263,8 @@ __device__ inline bool wait_record(const MceArgs& a, uint32_t gwave) {
 }
 
 constexpr int kMaxBlockWaves = 4;  // __launch_bounds__(256)
+constexpr uint32_t kSubtreeP = 2;      // fewest P members of a subtree that is moved to registers
+constexpr uint32_t kSubtreeRec = 2 * kWave;  // longest record put together for a frame of such a subtree
 constexpr int kScoreWords = 2;     // candidate words scored per round (arena path)
 constexpr int kLdsArena = 896;     // u64 words of LDS per wave for the walk of a medium root
 constexpr uint32_t kWideX = 256;   // largest |X'| of the register walk over several words (384 and 512 spill more and gain nothing)
@@ -374,37 +376,36 @@ __device__ inline uint64_t small_root(const MceArgs& a, SmallLds& L, uint32_t si
 // rowP (position k over P0) and, for k < p0, rowX (P0 member k over X).  Also
 // used by larger roots whose rows over X' (the X0 members with a neighbour in
 // P0) and P0 fit one word each and |X'| + p0 <= 64.
-__device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s, uint32_t d, uint64_t rowP, uint64_t rowX,
-                                      uint32_t part, uint32_t parts, const uint64_t* rec, RingLook& look,
-                                      uint64_t& cliques, uint64_t& hcount, uint64_t& hbig) {
+//
+// P, XP, XX and Q are the start node (depth `base`), fresh if it has still to
+// be counted and its pivot chosen; `before` are the task's nodes so far, `every`
+// the nodes between looks for idle waves (0: never);
+// give(to, depth, P, XP, Q, XX) hands a frame to waiting wave `to`.
+template <class Give>
+__device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t s, uint32_t d, uint64_t rowP, uint64_t rowX,
+                                                  uint32_t part, uint32_t parts, uint64_t P, uint64_t XP, uint64_t XX,
+                                                  uint64_t Q, uint32_t base, bool fresh, uint32_t every, uint64_t before,
+                                                  RingLook& look, Give give, uint64_t& cliques, uint64_t& hcount,
+                                                  uint64_t& hbig) {
     const uint32_t lane = lane_id();
-    const uint32_t p0 = d - s;
-    // ---- depth-first walk (depth relative to `base`, the start node's depth) ----
-    walk_begins(look);
-    uint64_t P = ones(p0), XP = 0, XX = ones(s), Q = 0;
-    uint32_t base = 0;
-    bool fresh = true;
-    if (rec) {
-        const unsigned long long* r = (const unsigned long long*)rec;
-        const uint64_t w = lane < 6 ? ld_dev(r + lane) : 0;
-        base = (uint32_t)read_lane(w, 1);
-        P = read_lane(w, 2);
-        XP = read_lane(w, 3);
-        Q = read_lane(w, 4);
-        XX = read_lane(w, 5);
-        fresh = false;
-    }
     uint64_t fP = 0, fXP = 0, fXX = 0, fQ = 0;  // frame of depth == lane
-    uint32_t depth = 0, child = 0, since = 0;
-    uint64_t nodes = 0;
+    uint32_t depth = 0, child = 0;
+    uint64_t nodes = 0, looked = 0;  // looked: nodes at the last look for idle waves
+    auto clique = [&](uint32_t sz) {  // a maximal clique of sz vertices
+        cliques++;
+        hcount += (lane == sz);
+        hbig += (lane + kWave == sz);
+        // (larger ones only below a frame of a root with more than 64 later neighbours)
+        if (sz >= 2 * kWave && lane == 0) atomicAdd(&a.hist[umin32(sz, a.hist_len - 1)], 1ull);
+    };
     while (true) {
         bool descend = false;
         if (fresh) {
             if (base + depth > 0 || part == 0) nodes++;
             // a task that has walked kDonateFrom x donate_every nodes looks for
             // idle waves every donate_every nodes
-            if (a.donate_every && ++since >= a.donate_every && nodes >= (uint64_t)kDonateFrom * a.donate_every) {
-                since = 0;
+            if (every && nodes - looked >= every && before + nodes >= (uint64_t)kDonateFrom * every) {
+                looked = nodes;
                 // hand the upper half of the shallowest frame's untried children
                 // to an idle wave (not the root frame of a split root: its
                 // children are dealt by part)
@@ -419,22 +420,12 @@ __device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s,
                     // already account for those siblings, which come first
                     const uint32_t nq = __popcll(fq);
                     const uint64_t keep = nq >= 2 ? lowest_bits(fq, nq - nq / 2) : 0;
-                    const uint64_t w = lane == 0 ? (uint64_t)si : lane == 1 ? (uint64_t)(base + i)
-                                     : lane == 2 ? (fp & ~keep) : lane == 3 ? (fxp | keep)
-                                     : lane == 4 ? (fq & ~keep) : fxx;
-                    record_made(a);
-                    if (lane < 6) st_dev((unsigned long long*)&a.area[(uint64_t)to * kRecWords + lane], w);
-                    record_send(a, to);
+                    give(to, base + i, fp & ~keep, fxp | keep, fq & ~keep, fxx);
                     fQ = lane == i ? keep : fQ;
                 }
             }
             if (P == 0) {
-                if (XP == 0 && XX == 0) {  // maximal clique, |R| = base + depth + 1
-                    cliques++;
-                    const uint32_t sz = base + depth + 1;
-                    if (sz < kWave) hcount += (lane == sz);
-                    else hbig += (lane == sz - kWave);
-                }
+                if (XP == 0 && XX == 0) clique(base + depth + 1);
             } else {
                 const uint64_t PX = P | XP;
                 const bool cand = lane < s ? ((XX >> lane) & 1) : (lane < d && ((PX >> (lane - s)) & 1));
@@ -451,15 +442,34 @@ __device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s,
             P &= ~m;
             XP |= m;
             if (base + depth == 0 && (child++ % parts) != part) continue;  // another part's child
+            const uint64_t qrow = read_lane(rowP, s + j), xrow = read_lane(rowX, j);
+            const uint64_t cP = P & qrow;
+            if ((cP & (cP - 1)) == 0) {
+                // A child with at most one vertex to add is settled here, without
+                // its frame and pivot: a leaf is maximal if nothing is left in X,
+                // and of one vertex k the pivot rule leaves the branch to k only if
+                // no X member is joined to it, which makes that branch a maximal
+                // clique.  (Most nodes are such; 800k social 23.5 -> 20.6 ms.)
+                nodes++;
+                uint64_t left = (XP & qrow) | (XX & xrow);
+                uint32_t sz = base + depth + 2;
+                if (cP) {
+                    const uint32_t k = __builtin_ctzll(cP);
+                    left = (XP & qrow & read_lane(rowP, s + k)) | (XX & xrow & read_lane(rowX, k));
+                    nodes += left == 0;
+                    sz++;
+                }
+                if (left == 0) clique(sz);
+                continue;
+            }
             const bool mine = lane == depth;
             fP = mine ? P : fP;
             fXP = mine ? XP : fXP;
             fXX = mine ? XX : fXX;
             fQ = mine ? Q : fQ;
-            const uint64_t qrow = read_lane(rowP, s + j);
-            P &= qrow;
+            P = cP;
             XP &= qrow;
-            XX &= read_lane(rowX, j);
+            XX &= xrow;
             Q = 0;
             depth++;
             fresh = true;
@@ -475,6 +485,35 @@ __device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s,
         }
     }
     return nodes;
+}
+
+
+// The register walk of a whole root, or of a record of it.
+__device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s, uint32_t d, uint64_t rowP, uint64_t rowX,
+                                      uint32_t part, uint32_t parts, const uint64_t* rec, RingLook& look,
+                                      uint64_t& cliques, uint64_t& hcount, uint64_t& hbig) {
+    const uint32_t lane = lane_id();
+    walk_begins(look);
+    uint64_t P = ones(d - s), XP = 0, XX = ones(s), Q = 0;
+    uint32_t base = 0;
+    if (rec) {
+        const unsigned long long* r = (const unsigned long long*)rec;
+        const uint64_t w = lane < 6 ? ld_dev(r + lane) : 0;
+        base = (uint32_t)read_lane(w, 1);
+        P = read_lane(w, 2);
+        XP = read_lane(w, 3);
+        Q = read_lane(w, 4);
+        XX = read_lane(w, 5);
+    }
+    auto give = [&](uint32_t to, uint32_t depth, uint64_t gP, uint64_t gXP, uint64_t gQ, uint64_t gXX) {
+        const uint64_t w = lane == 0 ? (uint64_t)si : lane == 1 ? (uint64_t)depth : lane == 2 ? gP : lane == 3 ? gXP
+                         : lane == 4 ? gQ : gXX;
+        record_made(a);
+        if (lane < 6) st_dev((unsigned long long*)&a.area[(uint64_t)to * kRecWords + lane], w);
+        record_send(a, to);
+    };
+    return register_walk(a, s, d, rowP, rowX, part, parts, P, XP, XX, Q, base, !rec, a.donate_every, 0, look, give, cliques,
+                         hcount, hbig);
 }
 
 // The register walk of a root with |P0| <= 64 and |X'| <= 64 R: lane j holds
@@ -512,14 +551,19 @@ __device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uin
     uint64_t fP = 0, fXP = 0, fQ = 0, fXX[R];  // frame of depth == lane
 #pragma unroll
     for (int r = 0; r < R; r++) fXX[r] = 0;
-    uint32_t depth = 0, child = 0, since = 0;
-    uint64_t nodes = 0;
+    uint32_t depth = 0, child = 0;
+    uint64_t nodes = 0, looked = 0;
+    auto clique = [&](uint32_t sz) {  // a maximal clique of sz <= 65 vertices
+        cliques++;
+        hcount += (lane == sz);
+        hbig += (lane + kWave == sz);
+    };
     while (true) {
         if (fresh) {
             if (base + depth > 0 || part == 0) nodes++;
-            if (a.donate_every && ++since >= a.donate_every && nodes >= (uint64_t)kDonateFrom * a.donate_every) {
-                // as in small_walk
-                since = 0;
+            if (a.donate_every && nodes - looked >= a.donate_every && nodes >= (uint64_t)kDonateFrom * a.donate_every) {
+                // as in register_walk
+                looked = nodes;
                 const uint32_t first = (base == 0 && parts > 1) ? 1u : 0u;
                 const uint64_t open = ballot(lane < depth && lane >= first && fQ != 0);
                 const uint32_t to = open ? ring_take(a, look) : ~0u;
@@ -545,12 +589,7 @@ __device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uin
                 uint64_t x = XP;
 #pragma unroll
                 for (int r = 0; r < R; r++) x |= XX[r];
-                if (x == 0) {  // maximal clique, |R| = base + depth + 1
-                    cliques++;
-                    const uint32_t sz = base + depth + 1;
-                    if (sz < kWave) hcount += (lane == sz);
-                    else hbig += (lane == sz - kWave);
-                }
+                if (x == 0) clique(base + depth + 1);
             } else {
                 uint32_t key = (((P | XP) >> lane) & 1) ? ((uint32_t)__popcll(rowPP & P) << 10) | (64u * R + lane) : 0u;
 #pragma unroll
@@ -574,6 +613,29 @@ __device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uin
             P &= ~m;
             XP |= m;
             if (base + depth == 0 && (child++ % parts) != part) continue;  // another part's child
+            const uint64_t qrow = read_lane(rowPP, j), cP = P & qrow;
+            uint64_t cX[R];
+#pragma unroll
+            for (int r = 0; r < R; r++) cX[r] = XX[r] & read_lane(rowX[r], j);
+            if ((cP & (cP - 1)) == 0) {  // at most one vertex to add: as in register_walk
+                nodes++;
+                uint64_t left = XP & qrow;
+                uint32_t sz = base + depth + 2;
+                if (cP) {
+                    const uint32_t k = __builtin_ctzll(cP);
+                    left &= read_lane(rowPP, k);
+#pragma unroll
+                    for (int r = 0; r < R; r++) cX[r] &= read_lane(rowX[r], k);
+                    sz++;
+                }
+#pragma unroll
+                for (int r = 0; r < R; r++) left |= cX[r];
+                if (left == 0) {
+                    nodes += cP != 0;
+                    clique(sz);
+                }
+                continue;
+            }
             const bool mine = lane == depth;
             fP = mine ? P : fP;
             fXP = mine ? XP : fXP;
@@ -581,10 +643,9 @@ __device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uin
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 fXX[r] = mine ? XX[r] : fXX[r];
-                XX[r] &= read_lane(rowX[r], j);
+                XX[r] = cX[r];
             }
-            const uint64_t qrow = read_lane(rowPP, j);
-            P &= qrow;
+            P = cP;
             XP &= qrow;
             Q = 0;
             depth++;
@@ -1030,18 +1091,93 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
         }
         uint64_t depth = 0;  // relative to base
         uint32_t child = 0;  // first-level children passed so far
-        uint32_t since = 0;  // nodes since the last look for idle waves
+        uint64_t looked = 0;  // nodes at the last look for idle waves
         while (true) {
             uint64_t* F = frame(depth);
             uint64_t* XX = F + 3 * W;
             bool descend = false;
             // the root node belongs to part 0 of a split root
             const bool own = base + depth > 0 || part == 0;
+            if (!ACCOUNT && fresh && depth && WXE <= kWave) {
+                // A subtree whose P, XP and XX have at most 64 members in all is
+                // walked in registers: its members are listed in position order
+                // (X', then P0), lane k takes member k's row over the listed P0
+                // members, and the rows over X' are those rows' columns.  A
+                // deeper level's sets are small even where the root's rows take
+                // several words, and a node costs a third there.  Same tree, pivots and
+                // child order.  100k Chung-Lu 3.8 -> 1.75 ms, 800k social 28.8 -> 23.5
+                // (24.5 and 26.8 from 4 and 8 P members on instead of 2).
+                uint64_t* const XXf = F + 3 * W;
+                const uint64_t xxw = lane < WXE ? XXf[lane] : 0, pxw = pw | xpw;
+                const uint32_t many = wave_sum32((uint32_t)__popcll(pw) << 16 | (uint32_t)(__popcll(pxw) + __popcll(xxw)));
+                if ((many & 0xffffu) <= kWave && (many >> 16) >= kSubtreeP) {
+                    uint32_t n = 0, sx = 0;
+                    for (uint64_t nz = ballot(xxw != 0); nz; nz &= nz - 1) {
+                        const uint32_t t = __builtin_ctzll(nz);
+                        const uint64_t word = read_lane(xxw, t);
+                        if ((word >> lane) & 1) SL.pref[n + lanes_below(word)] = t * 64 + lane;
+                        n += __popcll(word);
+                    }
+                    sx = n;
+                    for (uint64_t nz = ballot(pxw != 0); nz; nz &= nz - 1) {
+                        const uint32_t t = __builtin_ctzll(nz);
+                        const uint64_t word = read_lane(pxw, t);
+                        if ((word >> lane) & 1) SL.pref[n + lanes_below(word)] = t * 64 + lane;
+                        n += __popcll(word);
+                    }
+                    wave_sync();
+                    const uint32_t at = lane < n ? SL.pref[lane] : 0;  // the member's position in X' or P0
+                    const uint64_t* row = aP + ((lane < sx ? 0 : sE) + at) * W;
+                    uint64_t rowP = 0, rowX = 0;
+                    uint32_t k = 0;
+                    for (uint64_t nz = ballot(pxw != 0); nz; nz &= nz - 1) {
+                        const uint32_t t = __builtin_ctzll(nz);
+                        const uint64_t bits = lane < n ? row[t] : 0;
+                        for (uint64_t word = read_lane(pxw, t); word; word &= word - 1, k++) {
+                            const uint64_t bit = (bits >> __builtin_ctzll(word)) & 1;
+                            rowP |= bit << k;
+                            const uint64_t col = ballot(bit != 0) & ones(sx);
+                            rowX = lane == k ? col : rowX;
+                        }
+                    }
+                    const uint64_t pword = __shfl(pw, (int)(at >> 6), kWave);  // (all lanes active)
+                    const bool inP = lane >= sx && lane < n && ((pword >> (at & 63u)) & 1);
+                    const uint64_t subP = ballot(inP) >> sx, subXP = ones(n - sx) & ~subP;
+                    auto give = [&](uint32_t to, uint32_t dep, uint64_t gP, uint64_t gXP, uint64_t gQ, uint64_t gXX) {
+                        // the record's words over X' and P0, put together in the small path's row area
+                        uint64_t* R = SL.adjP;  // (kSubtreeRec words: adjP and adjX)
+                        wave_sync();
+                        for (uint32_t i = lane; i < FWE; i += kWave) R[i] = 0;
+                        wave_sync();
+                        const uint32_t b = at & 63u, wd = at >> 6, p = lane - sx;
+                        if (lane < sx) {
+                            if ((gXX >> lane) & 1) atomicOr((unsigned long long*)&R[3 * W + wd], 1ull << b);
+                        } else if (lane < n) {
+                            if ((gP >> p) & 1) atomicOr((unsigned long long*)&R[wd], 1ull << b);
+                            if ((gXP >> p) & 1) atomicOr((unsigned long long*)&R[W + wd], 1ull << b);
+                            if ((gQ >> p) & 1) atomicOr((unsigned long long*)&R[2 * W + wd], 1ull << b);
+                        }
+                        wave_sync();
+                        record_made(a);
+                        unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * kRecWords;
+                        for (uint32_t i = lane; i < FWE; i += kWave) st_dev(out + 2 + i, R[i]);
+                        if (lane < 2) st_dev(out + lane, lane == 0 ? (uint64_t)si : (uint64_t)dep);
+                        record_send(a, to);
+                    };
+                    const uint64_t sub = register_walk(a, sx, n, rowP, rowX, 0, 1, subP, subXP, ones(sx), 0,
+                                                       (uint32_t)(base + depth), true, FWE <= kSubtreeRec ? a.donate_every : 0u,
+                                                       root_nodes, look, give,
+                                                       small_cliques, small_hist, small_big);
+                    root_nodes += sub;
+                    fresh = false;
+                    qw = 0;
+                }
+            }
             if (fresh) {
                 if (own) root_nodes++;
-                if (!ACCOUNT && a.donate_every && ++since >= a.donate_every &&
+                if (!ACCOUNT && a.donate_every && root_nodes - looked >= a.donate_every &&
                     root_nodes >= (uint64_t)kDonateFrom * a.donate_every && 2 + FWE <= kRecWords) {
-                    since = 0;
+                    looked = root_nodes;
                     // hand the upper half of the shallowest ancestor frame's untried
                     // children to an idle wave (not the root frame of a split root)
                     for (uint64_t i = (base == 0 && parts > 1) ? 1 : 0; i < depth; i++) {
@@ -1221,19 +1357,41 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                     xpw |= m;
                 }
                 if (base + depth == 0 && (child++ % parts) != part) continue;  // another part's child
+                const uint64_t r = lane < W ? aP[(sE + j) * W + lane] : 0;
+                const uint64_t* xrow = aX + j * WXE;
+                const uint64_t some = ballot((pw & r) != 0);
+                if (!ACCOUNT && WXE <= kWave && (some & (some - 1)) == 0) {
+                    const uint32_t wk = some ? __builtin_ctzll(some) : 0u;
+                    const uint64_t cP = some ? read_lane(pw & r, wk) : 0;
+                    if ((cP & (cP - 1)) == 0) {  // at most one vertex to add: as in register_walk
+                        uint64_t left = xpw & r, lx = lane < WXE ? XX[lane] & xrow[lane] : 0;
+                        uint64_t sz = base + depth + 2;
+                        if (cP) {
+                            const uint64_t k = (uint64_t)wk * 64 + __builtin_ctzll(cP);
+                            left &= lane < W ? aP[(sE + k) * W + lane] : 0;
+                            lx &= lane < WXE ? aX[k * WXE + lane] : 0;
+                            sz++;
+                        }
+                        root_nodes++;
+                        if (ballot((left | lx) != 0) == 0) {
+                            root_nodes += cP != 0;
+                            if (lane == 0) {
+                                my_cliques++;
+                                if (sz < 64) atomicAdd(&lhist[sz], 1ull);
+                                else atomicAdd(&a.hist[sz < a.hist_len ? sz : a.hist_len - 1], 1ull);
+                            }
+                        }
+                        continue;
+                    }
+                }
                 if (lane < W) {
                     F[lane] = pw;
                     F[W + lane] = xpw;
                     F[2 * W + lane] = qw;
-                }
-                const uint64_t* qrow = aP + (sE + j) * W;
-                if (lane < W) {
-                    const uint64_t r = qrow[lane];
                     pw &= r;
                     xpw &= r;
                 }
                 qw = 0;
-                const uint64_t* xrow = aX + j * WXE;
                 uint64_t* XXc = frame(depth + 1) + 3 * W;
                 for (uint64_t i = lane; i < WXE; i += kWave) XXc[i] = XX[i] & xrow[i];
                 depth++;
