@@ -31,6 +31,7 @@
 // Roots whose bitsets exceed the per-wave arena are deferred to a second pass
 // with a larger arena (never dropped).
 #include <algorithm>
+#include <type_traits>
 
 #include <hipcub/hipcub.hpp>
 
@@ -81,7 +82,12 @@ struct MceArgs {
 constexpr uint32_t kRings = 16;
 constexpr uint64_t kDqStride = 16;       // u64 words of one 128-byte line
 constexpr uint32_t kRecWords = 1024;     // longest record; a wider root's frames are not handed on
-constexpr uint32_t kDonateFrom = 8;      // a task looks for idle waves from this many x donate_every nodes on
+constexpr uint32_t kRecRows = 16;         // first row word of a record that takes its rows along
+constexpr uint64_t kRegRecord = 1ull << 32;  // kind of a register_walk record (wide_walk<R>: R << 32; none: rows rebuilt)
+// A task looks for idle waves from this many x donate_every nodes on.  Fewer hand
+// on more and smaller frames than the waves' mailboxes serve: R-MAT 11 / R-MAT 10
+// 0.71 / 0.42 ms with 8, 1.1 / 0.36 with 3, 1.75 / 0.34 with 1.
+constexpr uint32_t kDonateFrom = 8;
 enum { MAIL_NONE = 0, MAIL_RECORD, MAIL_END };
 
 // u64 words of the per-root arena: adjP (d*W) + adjX (p0*WX) + (p0+1) frames
@@ -101,10 +107,14 @@ __device__ inline void arena_sync() { wave_sync(); }
 __device__ inline uint64_t degree_of(const uint64_t* __restrict__ rp, uint32_t u) { return rp[u + 1] - rp[u]; }
 
 
-// Work donation.  A record is [source index, absolute depth, P (W words),
-// XP (W), Q (W), XX (WX)]: a frame whose untried children Q the taker walks
-// exactly as the donor would have (same P/XP progression, same order), so
-// the search tree and every count stay the same.
+// Work donation.  A record is [source index, absolute depth and kind, P (W
+// words), XP (W), Q (W), XX (WX)]: a frame whose untried children Q the taker
+// walks exactly as the donor would have (same P/XP progression, same order), so
+// the search tree and every count stay the same.  Frames of a register walk
+// take their rows along (1 to 5 KB), so that a taker starts within microseconds;
+// the taker of any other frame builds the root's bitsets again.
+// (With every taker rebuilding, 2 x 45 us a generation, R-MAT 11 took 2.2 ms,
+// 0.71 so; R-MAT 9 0.46 and 0.24.)
 //
 // A wave without work registers in the ring of its group (16 rings) and waits
 // on a mailbox line of its own; a donor takes one registered wave off a ring,
@@ -176,10 +186,11 @@ struct RingLook {
     uint64_t from;         // clock from which its frames may be handed on
 };
 __device__ inline RingLook ring_start(uint32_t gwave) { return RingLook{gwave % kRings, 0, 0, 0}; }
-// A taker builds the root's bitsets again, so a task hands nothing on before
-// it has walked for half as long as its own build took.  Wall ms of R-MAT 11 /
-// R-MAT 9 / 5k-vertex Chung-Lu: 2.54 / 0.51 / 0.48 without this rule, 2.55 /
-// 0.53 / 0.39 with it, 3.04 / 0.46 / 0.33 with the whole of the build's time.
+// The taker of a frame without rows builds the root's bitsets again, so a task
+// hands nothing on before it has walked for half as long as its own build took
+// (a record's rows are a build of a microsecond).  With an eighth of that time and
+// three looks' nodes, R-MAT 11 / 5k-vertex Chung-Lu took 1.31 / 0.28 ms for 0.71 /
+// 0.31: more and smaller frames were handed on.
 __device__ inline void walk_begins(RingLook& k) {
     const uint64_t now = clock64();
     k.from = now + (now - k.begin) / 2;
@@ -264,7 +275,6 @@ __device__ inline bool wait_record(const MceArgs& a, uint32_t gwave) {
 
 constexpr int kMaxBlockWaves = 4;  // __launch_bounds__(256)
 constexpr uint32_t kSubtreeP = 2;      // fewest P members of a subtree that is moved to registers
-constexpr uint32_t kSubtreeRec = 2 * kWave;  // longest record put together for a frame of such a subtree
 constexpr int kScoreWords = 2;     // candidate words scored per round (arena path)
 constexpr int kLdsArena = 896;     // u64 words of LDS per wave for the walk of a medium root
 constexpr uint32_t kWideX = 256;   // largest |X'| of the register walk over several words (384 and 512 spill more and gain nothing)
@@ -298,17 +308,23 @@ __device__ inline uint32_t lds_lower_bound(const uint32_t* A, uint32_t lo, uint3
 // are those of the arena path, so every count is unchanged.  Clique sizes are
 // counted per lane (lane = size, sizes 64 and 65 in hbig at lanes 0 and 1) and
 // flushed once per wave.
-//
-// With rec != nullptr the walk resumes a donated frame (W = WX = 1 here):
-// it starts at that node with its untried children, one level above which
-// the walk ends.
-__device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s, uint32_t d, uint64_t rowP, uint64_t rowX,
-                                      uint32_t part, uint32_t parts, const uint64_t* rec, RingLook& look,
-                                      uint64_t& cliques, uint64_t& hcount, uint64_t& hbig);
+__device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t si, uint32_t s, uint32_t d, uint64_t rowP,
+                                                  uint64_t rowX, uint32_t part, uint32_t parts, uint64_t P, uint64_t XP,
+                                                  uint64_t XX, uint64_t Q, uint32_t base, bool fresh, uint64_t before,
+                                                  RingLook& look, uint64_t& cliques, uint64_t& hcount, uint64_t& hbig);
+
+// the walk of a whole root (or its part)
+__device__ __forceinline__ uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s, uint32_t d, uint64_t rowP,
+                                               uint64_t rowX, uint32_t part, uint32_t parts, RingLook& look,
+                                               uint64_t& cliques, uint64_t& hcount, uint64_t& hbig) {
+    walk_begins(look);
+    return register_walk(a, si, s, d, rowP, rowX, part, parts, ones(d - s), 0, ones(s), 0, 0, true, 0, look, cliques,
+                         hcount, hbig);
+}
 
 __device__ inline uint64_t small_root(const MceArgs& a, SmallLds& L, uint32_t si, uint32_t v, uint64_t lo, uint32_t d,
-                                      uint32_t s, uint32_t part, uint32_t parts, const uint64_t* rec, RingLook& look,
-                                      uint64_t& cliques, uint64_t& hcount, uint64_t& hbig) {
+                                      uint32_t s, uint32_t part, uint32_t parts, RingLook& look, uint64_t& cliques,
+                                      uint64_t& hcount, uint64_t& hbig) {
     const uint32_t lane = lane_id();
     const uint32_t p0 = d - s;
     // ---- neighbourhood bitsets in LDS ----
@@ -369,7 +385,7 @@ __device__ inline uint64_t small_root(const MceArgs& a, SmallLds& L, uint32_t si
         }
     }
     wave_sync();
-    return small_walk(a, si, s, d, L.adjP[lane], L.adjX[lane], part, parts, rec, look, cliques, hcount, hbig);
+    return small_walk(a, si, s, d, L.adjP[lane], L.adjX[lane], part, parts, look, cliques, hcount, hbig);
 }
 
 // The register walk of a root whose rows are in registers: lane k holds row
@@ -377,16 +393,14 @@ __device__ inline uint64_t small_root(const MceArgs& a, SmallLds& L, uint32_t si
 // used by larger roots whose rows over X' (the X0 members with a neighbour in
 // P0) and P0 fit one word each and |X'| + p0 <= 64.
 //
-// P, XP, XX and Q are the start node (depth `base`), fresh if it has still to
-// be counted and its pivot chosen; `before` are the task's nodes so far, `every`
-// the nodes between looks for idle waves (0: never);
-// give(to, depth, P, XP, Q, XX) hands a frame to waiting wave `to`.
-template <class Give>
-__device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t s, uint32_t d, uint64_t rowP, uint64_t rowX,
-                                                  uint32_t part, uint32_t parts, uint64_t P, uint64_t XP, uint64_t XX,
-                                                  uint64_t Q, uint32_t base, bool fresh, uint32_t every, uint64_t before,
-                                                  RingLook& look, Give give, uint64_t& cliques, uint64_t& hcount,
-                                                  uint64_t& hbig) {
+// P, XP, XX and Q are the start node (depth `base`; the walk ends one level
+// above it), fresh if it has still to be counted and its pivot chosen; `before`
+// are the task's nodes so far.  A frame handed on takes its rows along
+// (kRegRecord): the taker starts at once, whatever the root was.
+__device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t si, uint32_t s, uint32_t d, uint64_t rowP,
+                                                  uint64_t rowX, uint32_t part, uint32_t parts, uint64_t P, uint64_t XP,
+                                                  uint64_t XX, uint64_t Q, uint32_t base, bool fresh, uint64_t before,
+                                                  RingLook& look, uint64_t& cliques, uint64_t& hcount, uint64_t& hbig) {
     const uint32_t lane = lane_id();
     uint64_t fP = 0, fXP = 0, fXX = 0, fQ = 0;  // frame of depth == lane
     uint32_t depth = 0, child = 0;
@@ -404,7 +418,8 @@ __device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t s, 
             if (base + depth > 0 || part == 0) nodes++;
             // a task that has walked kDonateFrom x donate_every nodes looks for
             // idle waves every donate_every nodes
-            if (every && nodes - looked >= every && before + nodes >= (uint64_t)kDonateFrom * every) {
+            if (a.donate_every && nodes - looked >= a.donate_every &&
+                before + nodes >= (uint64_t)kDonateFrom * a.donate_every) {
                 looked = nodes;
                 // hand the upper half of the shallowest frame's untried children
                 // to an idle wave (not the root frame of a split root: its
@@ -420,7 +435,15 @@ __device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t s, 
                     // already account for those siblings, which come first
                     const uint32_t nq = __popcll(fq);
                     const uint64_t keep = nq >= 2 ? lowest_bits(fq, nq - nq / 2) : 0;
-                    give(to, base + i, fp & ~keep, fxp | keep, fq & ~keep, fxx);
+                    const uint64_t w = lane == 0 ? (uint64_t)si : lane == 1 ? kRegRecord | (base + i)
+                                     : lane == 2 ? (fp & ~keep) : lane == 3 ? (fxp | keep) : lane == 4 ? (fq & ~keep)
+                                     : lane == 5 ? fxx : lane == 6 ? (uint64_t)s : (uint64_t)d;
+                    record_made(a);
+                    unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * kRecWords;
+                    if (lane < 8) st_dev(out + lane, w);
+                    st_dev(out + kRecRows + lane, rowP);
+                    st_dev(out + kRecRows + kWave + lane, rowX);
+                    record_send(a, to);
                     fQ = lane == i ? keep : fQ;
                 }
             }
@@ -488,34 +511,6 @@ __device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t s, 
 }
 
 
-// The register walk of a whole root, or of a record of it.
-__device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s, uint32_t d, uint64_t rowP, uint64_t rowX,
-                                      uint32_t part, uint32_t parts, const uint64_t* rec, RingLook& look,
-                                      uint64_t& cliques, uint64_t& hcount, uint64_t& hbig) {
-    const uint32_t lane = lane_id();
-    walk_begins(look);
-    uint64_t P = ones(d - s), XP = 0, XX = ones(s), Q = 0;
-    uint32_t base = 0;
-    if (rec) {
-        const unsigned long long* r = (const unsigned long long*)rec;
-        const uint64_t w = lane < 6 ? ld_dev(r + lane) : 0;
-        base = (uint32_t)read_lane(w, 1);
-        P = read_lane(w, 2);
-        XP = read_lane(w, 3);
-        Q = read_lane(w, 4);
-        XX = read_lane(w, 5);
-    }
-    auto give = [&](uint32_t to, uint32_t depth, uint64_t gP, uint64_t gXP, uint64_t gQ, uint64_t gXX) {
-        const uint64_t w = lane == 0 ? (uint64_t)si : lane == 1 ? (uint64_t)depth : lane == 2 ? gP : lane == 3 ? gXP
-                         : lane == 4 ? gQ : gXX;
-        record_made(a);
-        if (lane < 6) st_dev((unsigned long long*)&a.area[(uint64_t)to * kRecWords + lane], w);
-        record_send(a, to);
-    };
-    return register_walk(a, s, d, rowP, rowX, part, parts, P, XP, XX, Q, base, !rec, a.donate_every, 0, look, give, cliques,
-                         hcount, hbig);
-}
-
 // The register walk of a root with |P0| <= 64 and |X'| <= 64 R: lane j holds
 // P0 member j's row over P0 (rowPP) and its rows over X' (rowX, word r = X'
 // positions 64 r ..), lane l the rows over P0 of X' members l, l + 64, ..
@@ -523,31 +518,15 @@ __device__ inline uint64_t small_walk(const MceArgs& a, uint32_t si, uint32_t s,
 // stack is spread over the lanes as in small_walk, so a node costs no memory:
 // 0.6 us where the arena path's frames and rows in LDS took 1.4 (R-MAT 11, the
 // root with 53 later neighbours of 178).  The tree, the pivot rule (positions:
-// X', then P0) and the child order are the arena path's; so is a record, W = 1
-// and wx words of XX.
+// X', then P0) and the child order are the arena path's.  A record (kind R)
+// takes the rows along.
 template <int R>
-__device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uint32_t s2, uint32_t p0, uint64_t rowPP,
-                                              const uint64_t* rowXP, const uint64_t* rowX, uint32_t wx, uint32_t part,
-                                              uint32_t parts, const uint64_t* rec, RingLook& look, uint64_t& cliques,
-                                              uint64_t& hcount, uint64_t& hbig) {
+__device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uint64_t rowPP, const uint64_t* rowXP,
+                                              const uint64_t* rowX, uint32_t part, uint32_t parts, uint64_t P, uint64_t XP,
+                                              uint64_t Q, uint64_t* XX, uint32_t base, bool fresh, RingLook& look,
+                                              uint64_t& cliques, uint64_t& hcount, uint64_t& hbig) {
     const uint32_t lane = lane_id();
     walk_begins(look);
-    uint64_t P = ones(p0), XP = 0, Q = 0, XX[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) XX[r] = s2 > 64u * r ? ones(s2 - 64 * r) : 0;
-    uint32_t base = 0;
-    bool fresh = true;
-    if (rec) {
-        const unsigned long long* d = (const unsigned long long*)rec;
-        const uint64_t w = lane < 5 + wx ? ld_dev(d + lane) : 0;
-        base = (uint32_t)read_lane(w, 1);
-        P = read_lane(w, 2);
-        XP = read_lane(w, 3);
-        Q = read_lane(w, 4);
-#pragma unroll
-        for (int r = 0; r < R; r++) XX[r] = read_lane(w, 5 + r);
-        fresh = false;
-    }
     uint64_t fP = 0, fXP = 0, fQ = 0, fXX[R];  // frame of depth == lane
 #pragma unroll
     for (int r = 0; r < R; r++) fXX[r] = 0;
@@ -572,7 +551,7 @@ __device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uin
                     const uint64_t fp = read_lane(fP, i), fxp = read_lane(fXP, i), fq = read_lane(fQ, i);
                     const uint32_t nq = __popcll(fq);
                     const uint64_t keep = nq >= 2 ? lowest_bits(fq, nq - nq / 2) : 0;
-                    uint64_t w = lane == 0 ? (uint64_t)si : lane == 1 ? (uint64_t)(base + i)
+                    uint64_t w = lane == 0 ? (uint64_t)si : lane == 1 ? ((uint64_t)R << 32 | (base + i))
                                : lane == 2 ? (fp & ~keep) : lane == 3 ? (fxp | keep) : (fq & ~keep);
 #pragma unroll
                     for (int r = 0; r < R; r++) {
@@ -580,7 +559,14 @@ __device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uin
                         w = lane == 5u + r ? fx : w;
                     }
                     record_made(a);
-                    if (lane < 5 + wx) st_dev((unsigned long long*)&a.area[(uint64_t)to * kRecWords + lane], w);
+                    unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * kRecWords;
+                    if (lane < 5 + R) st_dev(out + lane, w);
+                    st_dev(out + kRecRows + lane, rowPP);
+#pragma unroll
+                    for (int r = 0; r < R; r++) {
+                        st_dev(out + kRecRows + (1 + r) * kWave + lane, rowXP[r]);
+                        st_dev(out + kRecRows + (1 + R + r) * kWave + lane, rowX[r]);
+                    }
                     record_send(a, to);
                     fQ = lane == i ? keep : fQ;
                 }
@@ -690,12 +676,45 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
         const uint32_t si = (uint32_t)code;
         const uint32_t part = (uint32_t)(code >> 32) & 0xffffu;
         const uint32_t parts = (uint32_t)(code >> 48) ? (uint32_t)(code >> 48) : 1u;
+        look.begin = clock64();
+        auto walked = [&](uint64_t nodes) {
+            my_nodes += nodes;
+            if (a.per_root && lane == 0 && nodes) atomicAdd(&a.per_root[si], (unsigned long long)nodes);
+            t_end = wall_clock64();
+        };
+        if (!ACCOUNT && rec) {  // a frame that brings its rows
+            const unsigned long long* in = (const unsigned long long*)rec;
+            const uint64_t w = lane < kRecRows ? ld_dev(in + lane) : 0;
+            const uint32_t base = (uint32_t)read_lane(w, 1), kind = (uint32_t)(read_lane(w, 1) >> 32);
+            const uint64_t P = read_lane(w, 2), XP = read_lane(w, 3), Q = read_lane(w, 4);
+            auto wide = [&](auto words) {
+                constexpr int R = decltype(words)::value;
+                uint64_t rowXP[R], rowX[R], XX[R];
+                const uint64_t rowPP = ld_dev(in + kRecRows + lane);
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    XX[r] = read_lane(w, 5 + r);
+                    rowXP[r] = ld_dev(in + kRecRows + (1 + r) * kWave + lane);
+                    rowX[r] = ld_dev(in + kRecRows + (1 + R + r) * kWave + lane);
+                }
+                walked(wide_walk<R>(a, si, rowPP, rowXP, rowX, 0, 1, P, XP, Q, XX, base, false, look, small_cliques,
+                                    small_hist, small_big));
+            };
+            if (kind == (uint32_t)(kRegRecord >> 32)) {
+                const uint64_t rowP = ld_dev(in + kRecRows + lane), rowX = ld_dev(in + kRecRows + kWave + lane);
+                walk_begins(look);
+                walked(register_walk(a, si, (uint32_t)read_lane(w, 6), (uint32_t)read_lane(w, 7), rowP, rowX, 0, 1, P, XP,
+                                     read_lane(w, 5), Q, base, false, 0, look, small_cliques, small_hist, small_big));
+                return;
+            }
+            if (kind == 2) return wide(std::integral_constant<int, 2>());
+            if (kind == kWideX / 64) return wide(std::integral_constant<int, kWideX / 64>());
+        }
         const uint32_t v = uniform(a.src[si]);
         const uint64_t lo = uniform(a.rp[v]);
         const uint64_t d = uniform(a.rp[v + 1]) - lo;
         const uint32_t* __restrict__ C = a.cols + lo;
         uint64_t root_nodes = 0;
-        look.begin = clock64();
 
         if (d == 0) return;  // no subgraph is generated for an isolated root
         const uint64_t s = uniform(lower_bound(C, 0, d, v));
@@ -709,11 +728,8 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
             return;
         }
         if (!ACCOUNT && d <= a.small_max) {
-            root_nodes = small_root(a, SL, si, v, lo, (uint32_t)d, (uint32_t)s, part, parts, rec, look, small_cliques,
-                                    small_hist, small_big);
-            my_nodes += root_nodes;
-            if (a.per_root && lane == 0 && root_nodes) atomicAdd(&a.per_root[si], (unsigned long long)root_nodes);
-            t_end = wall_clock64();
+            walked(small_root(a, SL, si, v, lo, (uint32_t)d, (uint32_t)s, part, parts, look, small_cliques, small_hist,
+                              small_big));
             return;
         }
         const uint64_t W = (p0 + 63) / 64, WX = (s + 63) / 64, FW = 3 * W + WX;
@@ -1004,16 +1020,15 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                 wave_sync();
 #pragma unroll
                 for (uint32_t r = 0; r < kWideX / 64; r++) rowX[r] = lane < p0 && r < WX2 ? SA[lane * WX2 + r] : 0;
-                const uint32_t wx = (uint32_t)WX2, sx = (uint32_t)s2, pp = (uint32_t)p0;
-                if (wx <= 2)
-                    root_nodes = wide_walk<2>(a, si, sx, pp, rowPP, rowXP, rowX, wx, part, parts, rec, look, small_cliques,
-                                              small_hist, small_big);
+                uint64_t XX[kWideX / 64];
+#pragma unroll
+                for (uint32_t r = 0; r < kWideX / 64; r++) XX[r] = s2 > 64 * r ? ones(s2 - 64 * r) : 0;
+                if (WX2 <= 2)
+                    walked(wide_walk<2>(a, si, rowPP, rowXP, rowX, part, parts, ones(p0), 0, 0, XX, 0, true, look,
+                                        small_cliques, small_hist, small_big));
                 else
-                    root_nodes = wide_walk<kWideX / 64>(a, si, sx, pp, rowPP, rowXP, rowX, wx, part, parts, rec, look,
-                                                        small_cliques, small_hist, small_big);
-                my_nodes += root_nodes;
-                if (a.per_root && lane == 0 && root_nodes) atomicAdd(&a.per_root[si], (unsigned long long)root_nodes);
-                t_end = wall_clock64();
+                    walked(wide_walk<kWideX / 64>(a, si, rowPP, rowXP, rowX, part, parts, ones(p0), 0, 0, XX, 0, true, look,
+                                                  small_cliques, small_hist, small_big));
                 return;
             }
             const uint64_t rows2 = (s2 + p0) * W + p0 * WX2;
@@ -1058,11 +1073,8 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
         if (!ACCOUNT && DL > 0 && W == 1 && WXE == 1 && sE + p0 <= kWave) {
             const uint64_t rowP = lane < sE + p0 ? aP[lane] : 0;
             const uint64_t rowX = lane < p0 ? aX[lane] : 0;
-            root_nodes = small_walk(a, si, (uint32_t)sE, (uint32_t)(sE + p0), rowP, rowX, part, parts, rec, look,
-                                    small_cliques, small_hist, small_big);
-            my_nodes += root_nodes;
-            if (a.per_root && lane == 0 && root_nodes) atomicAdd(&a.per_root[si], (unsigned long long)root_nodes);
-            t_end = wall_clock64();
+            walked(small_walk(a, si, (uint32_t)sE, (uint32_t)(sE + p0), rowP, rowX, part, parts, look, small_cliques,
+                              small_hist, small_big));
             return;
         }
         // frame of depth dep: the first DL in LDS, the rest in the global arena
@@ -1143,31 +1155,9 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                     const uint64_t pword = __shfl(pw, (int)(at >> 6), kWave);  // (all lanes active)
                     const bool inP = lane >= sx && lane < n && ((pword >> (at & 63u)) & 1);
                     const uint64_t subP = ballot(inP) >> sx, subXP = ones(n - sx) & ~subP;
-                    auto give = [&](uint32_t to, uint32_t dep, uint64_t gP, uint64_t gXP, uint64_t gQ, uint64_t gXX) {
-                        // the record's words over X' and P0, put together in the small path's row area
-                        uint64_t* R = SL.adjP;  // (kSubtreeRec words: adjP and adjX)
-                        wave_sync();
-                        for (uint32_t i = lane; i < FWE; i += kWave) R[i] = 0;
-                        wave_sync();
-                        const uint32_t b = at & 63u, wd = at >> 6, p = lane - sx;
-                        if (lane < sx) {
-                            if ((gXX >> lane) & 1) atomicOr((unsigned long long*)&R[3 * W + wd], 1ull << b);
-                        } else if (lane < n) {
-                            if ((gP >> p) & 1) atomicOr((unsigned long long*)&R[wd], 1ull << b);
-                            if ((gXP >> p) & 1) atomicOr((unsigned long long*)&R[W + wd], 1ull << b);
-                            if ((gQ >> p) & 1) atomicOr((unsigned long long*)&R[2 * W + wd], 1ull << b);
-                        }
-                        wave_sync();
-                        record_made(a);
-                        unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * kRecWords;
-                        for (uint32_t i = lane; i < FWE; i += kWave) st_dev(out + 2 + i, R[i]);
-                        if (lane < 2) st_dev(out + lane, lane == 0 ? (uint64_t)si : (uint64_t)dep);
-                        record_send(a, to);
-                    };
-                    const uint64_t sub = register_walk(a, sx, n, rowP, rowX, 0, 1, subP, subXP, ones(sx), 0,
-                                                       (uint32_t)(base + depth), true, FWE <= kSubtreeRec ? a.donate_every : 0u,
-                                                       root_nodes, look, give,
-                                                       small_cliques, small_hist, small_big);
+                    const uint64_t sub = register_walk(a, si, sx, n, rowP, rowX, 0, 1, subP, subXP, ones(sx), 0,
+                                                       (uint32_t)(base + depth), true, root_nodes, look, small_cliques,
+                                                       small_hist, small_big);
                     root_nodes += sub;
                     fresh = false;
                     qw = 0;
@@ -1409,8 +1399,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                 }
             }
         }
-        my_nodes += root_nodes;
-        if (a.per_root && lane == 0 && root_nodes) atomicAdd(&a.per_root[si], (unsigned long long)root_nodes);
+        walked(root_nodes);
     };
 
     // root tasks, then (with donation) records of other waves' frames
