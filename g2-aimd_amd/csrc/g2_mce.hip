@@ -282,6 +282,57 @@ constexpr int kMinLdsFrames = 16; // frames that must fit next to the rows for t
 constexpr int kBuildItems = 4;    // neighbourhood-build items per lane in flight (C in LDS)
 constexpr uint32_t kPB = 255;      // value buckets over a root's P0 part in the build (C in LDS)
 
+// Row windows of members k0 + lane, k0 + 64 + lane, .. of C: N(c) within
+// [v + 1, C[d-1]] (c in X0) or [c + 1, C[d-1]] (c in P0), whole rows up to
+// kWholeRow entries.  Both ends of all of a lane's windows are searched in
+// lockstep, so even a short row's window costs less than the entries outside it,
+// each of which is looked up: 100k / 30k Chung-Lu 1.29 / 0.82 ms with rows up to 64
+// entries streamed whole, 1.16 / 0.66 up to 24, 1.09 / 0.60 up to 8 and to 3.
+constexpr uint32_t kBuildChunks = 4;
+constexpr uint32_t kWholeRow = 8;
+template <uint32_t CH>
+__device__ __forceinline__ void build_windows(const uint64_t* __restrict__ rp, const uint32_t* __restrict__ cols,
+                                              const uint32_t* C, uint64_t k0, uint64_t d, uint64_t s, uint32_t v,
+                                              uint64_t* first, uint32_t* count) {
+    const uint32_t lane = lane_id(), above = C[d - 1] + 1;
+    uint32_t x[CH], n[CH], lo[CH], hi[CH], most = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < CH; q++) {
+        const uint64_t k = k0 + q * kWave + lane;
+        const bool on = k < d;
+        const uint32_t c = C[on ? k : 0];
+        x[q] = k < s ? v + 1 : c + 1;
+        first[q] = on ? rp[c] : 0;
+        count[q] = on ? (uint32_t)(rp[c + 1] - first[q]) : 0u;
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < CH; q++) {
+        n[q] = count[q] > kWholeRow ? count[q] : 0u;
+        lo[q] = hi[q] = 0;
+        most = umax32(most, n[q]);
+    }
+    uint32_t step = 1;
+    while (step <= most / 2) step *= 2;
+    for (step = most ? step : 0; step; step >>= 1) {  // lo, hi = entries below x, below `above`
+        uint32_t a[CH], b[CH];
+#pragma unroll
+        for (uint32_t q = 0; q < CH; q++) {
+            a[q] = step <= n[q] - lo[q] ? cols[first[q] + lo[q] + step - 1] : ~0u;
+            b[q] = step <= n[q] - hi[q] ? cols[first[q] + hi[q] + step - 1] : ~0u;
+        }
+#pragma unroll
+        for (uint32_t q = 0; q < CH; q++) {
+            lo[q] += a[q] < x[q] ? step : 0u;
+            hi[q] += b[q] < above ? step : 0u;
+        }
+    }
+#pragma unroll
+    for (uint32_t q = 0; q < CH; q++) {
+        first[q] += lo[q];
+        count[q] = n[q] ? hi[q] - lo[q] : count[q];
+    }
+}
+
 // LDS of one wave for the register-resident path
 struct SmallLds {
     uint32_t C[kWave];         // the root's neighbourhood, sorted
@@ -335,20 +386,13 @@ __device__ inline uint64_t small_root(const MceArgs& a, SmallLds& L, uint32_t si
     // Oriented build: every edge inside C that touches P0 is found in the
     // later part of its lower end's row.  Member k = lane (vertex c) streams
     // N(c) within [v+1, C[d-1]] (c in X0) or [c+1, C[d-1]] (c in P0) and looks
-    // each entry up among C's P0 part; a row of at most 64 entries is streamed
-    // whole (entries outside the range miss, and a P0 pair found from both
-    // ends sets the same bits twice).
-    uint32_t len = 0;
-    if (lane < d) {
-        const uint32_t c = L.C[lane];
-        uint64_t e0 = a.rp[c], e1 = a.rp[c + 1];
-        if (e1 - e0 > kWave) {
-            e0 = lower_bound(a.cols, e0, e1, lane < s ? v + 1 : c + 1);
-            e1 = lower_bound(a.cols, e0, e1, L.C[d - 1] + 1);
-        }
-        L.start[lane] = e0;
-        len = (uint32_t)(e1 - e0);
-    }
+    // each entry up among C's P0 part (entries outside the range miss, and a
+    // P0 pair found from both ends sets the same bits twice).
+    uint64_t first;
+    uint32_t len;
+    build_windows<1>(a.rp, a.cols, L.C, 0, d, s, v, &first, &len);
+    if (lane >= d) len = 0;
+    L.start[lane] = first;
     uint32_t incl = len;
 #pragma unroll
     for (int o = 1; o < kWave; o <<= 1) {
@@ -772,8 +816,8 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
             // streams N(c) within [lo, C[d-1]], lo = v+1 for c in X0 (partners
             // in P0) and c+1 for c in P0 (later partners), and looks each entry
             // up among C's P0 part in LDS.  These later-neighbour parts are
-            // short in degeneracy order.  A row of at most 64 entries is
-            // streamed whole: entries outside the range miss, and a P0 pair
+            // short in degeneracy order.  A row of at most kWholeRow entries
+            // is streamed whole: entries outside the range miss, and a P0 pair
             // found from both ends sets the same bits twice.
             uint32_t hb_p = 1;  // highest power of two <= p0
             while ((uint64_t)hb_p * 2 <= p0) hb_p *= 2;
@@ -802,20 +846,20 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                 big = (uint32_t)wave_max((uint64_t)big);
                 while (hb_b * 2 <= big) hb_b *= 2;
             }
+            uint64_t first[kBuildChunks];  // the members' row windows, a lane's searches in lockstep
+            uint32_t count[kBuildChunks];
             for (uint64_t k0 = 0; k0 < d; k0 += kWave) {
-                const uint32_t nk = (uint32_t)umin64(kWave, d - k0);
-                uint32_t len = 0;
-                if (lane < nk) {  // (a row of at most 64 entries is streamed whole)
-                    const uint64_t k = k0 + lane;
-                    const uint32_t c = Cb[k];
-                    uint64_t e0 = a.rp[c], e1 = a.rp[c + 1];
-                    if (e1 - e0 > kWave) {
-                        e0 = lower_bound(a.cols, e0, e1, k < s ? v + 1 : c + 1);
-                        e1 = lower_bound(a.cols, e0, e1, Cb[d - 1] + 1);
-                    }
-                    SL.start[lane] = e0;
-                    len = (uint32_t)(e1 - e0);
+                const uint32_t nk = (uint32_t)umin64(kWave, d - k0), at = (uint32_t)(k0 / kWave) % kBuildChunks;
+                if (at == 0) build_windows<kBuildChunks>(a.rp, a.cols, Cb, k0, d, s, v, first, count);
+                uint64_t e0 = first[0];
+                uint32_t len = count[0];
+#pragma unroll
+                for (uint32_t q = 1; q < kBuildChunks; q++) {
+                    e0 = at == q ? first[q] : e0;
+                    len = at == q ? count[q] : len;
                 }
+                if (lane >= nk) len = 0;
+                SL.start[lane] = e0;
                 uint32_t incl = len;
 #pragma unroll
                 for (int o = 1; o < kWave; o <<= 1) {
