@@ -279,6 +279,7 @@ constexpr int kScoreWords = 2;     // candidate words scored per round (arena pa
 constexpr int kLdsArena = 896;     // u64 words of LDS per wave for the walk of a medium root
 constexpr uint32_t kWideX = 256;   // largest |X'| of the register walk over several words (384 and 512 spill more and gain nothing)
 constexpr int kMinLdsFrames = 16; // frames that must fit next to the rows for the LDS layout
+constexpr int kSmallItems = 2;    // and for a root of degree <= 64 (one after the other: 8.0 ms for the 660k such roots of 800k social, 7.1 so)
 constexpr int kBuildItems = 4;    // neighbourhood-build items per lane in flight (C in LDS)
 constexpr uint32_t kPB = 255;      // value buckets over a root's P0 part in the build (C in LDS)
 
@@ -331,6 +332,21 @@ __device__ __forceinline__ void build_windows(const uint64_t* __restrict__ rp, c
         first[q] += lo[q];
         count[q] = n[q] ? hi[q] - lo[q] : count[q];
     }
+}
+
+// entries of the sorted C[0, d) below v, 64 splitters a step: a dependent load
+// or two where halving waits for log2 d of them
+__device__ __forceinline__ uint64_t wave_rank(const uint32_t* __restrict__ C, uint64_t d, uint32_t v) {
+    const uint32_t lane = lane_id();
+    uint64_t lo = 0, n = d;  // the answer lies in [lo, lo + n]
+    while (n) {
+        const uint64_t step = (n + kWave - 1) / kWave, at = lo + (lane + 1) * step - 1;
+        const uint64_t below = ballot(at < lo + n && C[umin64(at, d - 1)] < v);
+        const uint64_t c = (uint64_t)__popcll(below) * step;  // (the lanes below are the first ones)
+        lo += c;
+        n = step > 1 ? umin64(step - 1, n - c) : 0;
+    }
+    return lo;
 }
 
 // LDS of one wave for the register-resident path
@@ -404,27 +420,54 @@ __device__ inline uint64_t small_root(const MceArgs& a, SmallLds& L, uint32_t si
     uint32_t hb_p = 1;  // highest power of two <= p0
     while (hb_p * 2 <= p0) hb_p *= 2;
     wave_sync();
-    for (uint32_t f = lane; f < T; f += kWave) {
-        // member k whose streamed slice holds entry f (last k with pref[k] <= f)
-        uint32_t lo2 = 0, hi2 = d;
-        while (hi2 - lo2 > 1) {
-            const uint32_t mid = (lo2 + hi2) >> 1;
-            if (L.pref[mid] <= f) lo2 = mid; else hi2 = mid;
+    for (uint32_t f0 = 0; f0 < T; f0 += kSmallItems * kWave) {
+        // member k whose streamed slice holds entry f (last k with pref[k] <= f),
+        // searched between the round's first and last
+        const uint32_t flast = umin32(f0 + kSmallItems * kWave, T) - 1;
+        const uint32_t o0 = __popcll(ballot(lane < d && incl - len <= f0)) - 1;
+        const uint32_t o1 = __popcll(ballot(lane < d && incl - len <= flast)) - 1;
+        uint32_t k[kSmallItems], w[kSmallItems], pos[kSmallItems];
+        uint32_t hb_o = o1 > o0 ? 32u >> (__builtin_clz(o1 - o0) - 26) : 0u;
+#pragma unroll
+        for (int q = 0; q < kSmallItems; q++) {
+            k[q] = o0;
+            pos[q] = s;
         }
-        const uint32_t k = lo2;
-        const uint32_t w = a.cols[L.start[k] + (f - L.pref[k])];
-        uint32_t pos = s;  // first P0 position with C >= w, fixed halving steps
-        for (uint32_t step = hb_p; step >= 1; step >>= 1)
-            if (pos + step <= d && L.C[pos + step - 1] < w) pos += step;
-        if (pos < d && L.C[pos] == w && pos != k) {
-            const uint32_t j2 = pos - s;
-            if (k < s) {  // X0 member k, P0 member j2
-                atomicOr((unsigned long long*)&L.adjX[j2], 1ull << k);
-                atomicOr((unsigned long long*)&L.adjP[k], 1ull << j2);
-            } else {      // P0 members j1, j2
-                const uint32_t j1 = k - s;
-                atomicOr((unsigned long long*)&L.adjP[s + j1], 1ull << j2);
-                atomicOr((unsigned long long*)&L.adjP[s + j2], 1ull << j1);
+        for (uint32_t step = hb_o; step >= 1; step >>= 1) {
+#pragma unroll
+            for (int q = 0; q < kSmallItems; q++) {
+                const uint32_t c = k[q] + step;
+                const uint32_t pc = L.pref[umin32(c, o1)];
+                k[q] = (c <= o1 && pc <= f0 + q * kWave + lane) ? c : k[q];
+            }
+        }
+        // (an item past T reads the root's first entry and never hits)
+#pragma unroll
+        for (int q = 0; q < kSmallItems; q++) {
+            const uint32_t f = f0 + q * kWave + lane;
+            w[q] = a.cols[f < T ? L.start[k[q]] + (f - L.pref[k[q]]) : lo];
+        }
+        for (uint32_t step = hb_p; step >= 1; step >>= 1) {  // first P0 position with C >= w
+#pragma unroll
+            for (int q = 0; q < kSmallItems; q++) {
+                const uint32_t c = pos[q] + step;
+                const uint32_t cv = L.C[umin32(c, d) - 1];
+                pos[q] = (c <= d && cv < w[q]) ? c : pos[q];
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < kSmallItems; q++) {
+            const uint32_t cv = L.C[umin32(pos[q], d - 1)];
+            if (f0 + q * kWave + lane < T && pos[q] < d && cv == w[q] && pos[q] != k[q]) {
+                const uint32_t j2 = pos[q] - s;
+                if (k[q] < s) {  // X0 member k, P0 member j2
+                    atomicOr((unsigned long long*)&L.adjX[j2], 1ull << k[q]);
+                    atomicOr((unsigned long long*)&L.adjP[k[q]], 1ull << j2);
+                } else {         // P0 members j1, j2
+                    const uint32_t j1 = k[q] - s;
+                    atomicOr((unsigned long long*)&L.adjP[s + j1], 1ull << j2);
+                    atomicOr((unsigned long long*)&L.adjP[s + j2], 1ull << j1);
+                }
             }
         }
     }
@@ -761,7 +804,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
         uint64_t root_nodes = 0;
 
         if (d == 0) return;  // no subgraph is generated for an isolated root
-        const uint64_t s = uniform(lower_bound(C, 0, d, v));
+        const uint64_t s = wave_rank(C, d, v);
         const uint64_t p0 = d - s;
         if (p0 == 0) {  // root node with empty P and non-empty X: one node, no clique (never donated)
             if (part == 0) {
