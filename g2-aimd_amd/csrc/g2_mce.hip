@@ -1205,49 +1205,82 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                 // deeper level's sets are small even where the root's rows take
                 // several words, and a node costs a third there.  Same tree, pivots and
                 // child order.  100k Chung-Lu 3.8 -> 1.75 ms, 800k social 28.8 -> 23.5
-                // (24.5 and 26.8 from 4 and 8 P members on instead of 2).
+                // (24.5 and 26.8 from 4 and 8 P members on instead of 2).  Up to 128
+                // members are listed, those of X that have no neighbour in P left out
+                // first: 30k Chung-Lu 0.60 -> 0.49 ms.
                 uint64_t* const XXf = F + 3 * W;
                 const uint64_t xxw = lane < WXE ? XXf[lane] : 0, pxw = pw | xpw;
                 const uint32_t many = wave_sum32((uint32_t)__popcll(pw) << 16 | (uint32_t)(__popcll(pxw) + __popcll(xxw)));
-                if ((many & 0xffffu) <= kWave && (many >> 16) >= kSubtreeP) {
+                if ((many & 0xffffu) <= 2 * kWave && (many >> 16) >= kSubtreeP) {
+                    uint16_t* const list = reinterpret_cast<uint16_t*>(SL.pref);  // (positions below 4096)
                     uint32_t n = 0, sx = 0;
                     for (uint64_t nz = ballot(xxw != 0); nz; nz &= nz - 1) {
                         const uint32_t t = __builtin_ctzll(nz);
                         const uint64_t word = read_lane(xxw, t);
-                        if ((word >> lane) & 1) SL.pref[n + lanes_below(word)] = t * 64 + lane;
+                        if ((word >> lane) & 1) list[n + lanes_below(word)] = (uint16_t)(t * 64 + lane);
                         n += __popcll(word);
                     }
                     sx = n;
                     for (uint64_t nz = ballot(pxw != 0); nz; nz &= nz - 1) {
                         const uint32_t t = __builtin_ctzll(nz);
                         const uint64_t word = read_lane(pxw, t);
-                        if ((word >> lane) & 1) SL.pref[n + lanes_below(word)] = t * 64 + lane;
+                        if ((word >> lane) & 1) list[n + lanes_below(word)] = (uint16_t)(t * 64 + lane);
                         n += __popcll(word);
                     }
                     wave_sync();
-                    const uint32_t at = lane < n ? SL.pref[lane] : 0;  // the member's position in X' or P0
-                    const uint64_t* row = aP + ((lane < sx ? 0 : sE) + at) * W;
-                    uint64_t rowP = 0, rowX = 0;
-                    uint32_t k = 0;
-                    for (uint64_t nz = ballot(pxw != 0); nz; nz &= nz - 1) {
-                        const uint32_t t = __builtin_ctzll(nz);
-                        const uint64_t bits = lane < n ? row[t] : 0;
-                        for (uint64_t word = read_lane(pxw, t); word; word &= word - 1, k++) {
-                            const uint64_t bit = (bits >> __builtin_ctzll(word)) & 1;
-                            rowP |= bit << k;
-                            const uint64_t col = ballot(bit != 0) & ones(sx);
-                            rowX = lane == k ? col : rowX;
+                    if (n > kWave) {
+                        // members of X and XP without a neighbour in P leave (they can
+                        // neither be the pivot nor survive into a child's X)
+                        uint32_t at2[2];
+                        uint64_t left[2];
+#pragma unroll
+                        for (uint32_t h = 0; h < 2; h++) {
+                            const uint32_t i = h * kWave + lane;
+                            at2[h] = i < n ? list[i] : 0u;
+                            const uint64_t* r2 = aP + ((i < sx ? 0 : sE) + at2[h]) * W;
+                            uint64_t any = 0;
+                            for (uint64_t nz = ballot(pw != 0); nz; nz &= nz - 1) {
+                                const uint32_t t = __builtin_ctzll(nz);
+                                any |= (i < n ? r2[t] : 0) & read_lane(pw, t);
+                            }
+                            const uint64_t pword = __shfl(pw, (int)(at2[h] >> 6), kWave);
+                            left[h] = ballot(i < n && (any != 0 || (i >= sx && ((pword >> (at2[h] & 63u)) & 1))));
                         }
+                        const uint32_t n0 = __popcll(left[0]);
+                        n = n0 + __popcll(left[1]);
+                        sx = __popcll(left[0] & ones(umin32(sx, kWave))) + __popcll(left[1] & ones(sx > kWave ? sx - kWave : 0));
+                        wave_sync();
+                        if ((left[0] >> lane) & 1) list[lanes_below(left[0])] = (uint16_t)at2[0];
+                        if ((left[1] >> lane) & 1) list[n0 + lanes_below(left[1])] = (uint16_t)at2[1];
+                        wave_sync();
                     }
-                    const uint64_t pword = __shfl(pw, (int)(at >> 6), kWave);  // (all lanes active)
-                    const bool inP = lane >= sx && lane < n && ((pword >> (at & 63u)) & 1);
-                    const uint64_t subP = ballot(inP) >> sx, subXP = ones(n - sx) & ~subP;
-                    const uint64_t sub = register_walk(a, si, sx, n, rowP, rowX, 0, 1, subP, subXP, ones(sx), 0,
-                                                       (uint32_t)(base + depth), true, root_nodes, look, small_cliques,
-                                                       small_hist, small_big);
-                    root_nodes += sub;
-                    fresh = false;
-                    qw = 0;
+                    if (n <= kWave) {
+                        const uint32_t at = lane < n ? list[lane] : 0;  // the member's position in X' or P0
+                        const uint64_t* row = aP + ((lane < sx ? 0 : sE) + at) * W;
+                        uint64_t rowP = 0, rowX = 0;
+                        uint32_t k = 0;
+                        for (uint64_t nz = ballot(pxw != 0); nz; nz &= nz - 1) {
+                            const uint32_t t = __builtin_ctzll(nz);
+                            const uint64_t bits = lane < n ? row[t] : 0;
+                            for (; sx + k < n; k++) {
+                                const uint32_t pos = read_lane(at, sx + k);
+                                if (pos >> 6 != t) break;
+                                const uint64_t bit = (bits >> (pos & 63u)) & 1;
+                                rowP |= bit << k;
+                                const uint64_t col = ballot(bit != 0) & ones(sx);
+                                rowX = lane == k ? col : rowX;
+                            }
+                        }
+                        const uint64_t pword = __shfl(pw, (int)(at >> 6), kWave);  // (all lanes active)
+                        const bool inP = lane >= sx && lane < n && ((pword >> (at & 63u)) & 1);
+                        const uint64_t subP = ballot(inP) >> sx, subXP = ones(n - sx) & ~subP;
+                        const uint64_t sub = register_walk(a, si, sx, n, rowP, rowX, 0, 1, subP, subXP, ones(sx), 0,
+                                                           (uint32_t)(base + depth), true, root_nodes, look, small_cliques,
+                                                           small_hist, small_big);
+                        root_nodes += sub;
+                        fresh = false;
+                        qw = 0;
+                    }
                 }
             }
             if (fresh) {
