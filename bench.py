@@ -561,9 +561,9 @@ def main():
     assert acc["count"] == cnt and acc["stats"]["local_bitmap"] == 1
     pbytes = acc["stats"]["local_pass_bytes"]
     pms = np.mean(np.array(pass_ms), axis=0)
-    names = ["gm_local_kernel<4> (rows in the wave's LDS)", "gm_local_block_kernel<4,256,...>",
-             "gm_local_block_kernel<4,512,...>", "gm_local_block_kernel<4,1024,...>",
-             "gm_local_kernel<4> (rows in global arenas)"]
+    names = ["gm_local_kernel<4> (rows in the wave's LDS)", "gm_local_block_kernel<4,512,...> (|U| <= 448)",
+             "gm_local_block_kernel<4,1024,...> (|U| <= 700)", "gm_local_block_kernel<4,1024,...> (|U| <= 1039)",
+             "gm_local_wide kernels (rows in global arenas)"]
     passes = [{"kernel": names[k], "ms": float(pms[k]), "alg_bytes": int(pbytes[k]),
                "achieved_GBs": pbytes[k] / (pms[k] / 1e3) / 1e9 if pms[k] > 0 else None,
                "roots": int(acc["stats"]["local_pass_roots"][k])} for k in range(5)]

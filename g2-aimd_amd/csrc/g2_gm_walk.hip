@@ -25,9 +25,9 @@
 // windows that any wave takes from one of 16 counters.  Against one candidate
 // at a time with scalar searches and a whole root (or caller's window) per
 // wave, per call on one MI355X:
-//   4 vertices, 5 edges, per-root counts, 100k-vertex Chung-Lu   58.6 -> 1.9 ms
-//   5 vertices, 8 edges, R-MAT 9 (512 vertices, 6k edges)         475 -> 1.6 ms
-//   48 random patterns of 3-5 vertices in one launch, R-MAT 7     308 -> 0.9 ms
+//   4 vertices, 5 edges, per-root counts, 100k-vertex Chung-Lu   58.6 -> 1.6 ms
+//   5 vertices, 8 edges, R-MAT 9 (512 vertices, 6k edges)         475 -> 1.4 ms
+//   48 random patterns of 3-5 vertices in one launch, R-MAT 7     308 -> 0.85 ms
 #include <algorithm>
 #include <vector>
 
