@@ -21,10 +21,11 @@
 //     built from the later parts of the members' rows (each edge inside C
 //     found at its lower end), short in degeneracy order;
 //   * a node is (P, XP) in P0 space (one 64-bit word per lane, lane i holds
-//     word i) plus XX in X0 space (a stack frame).  Roots of degree <= 64 keep
-//     everything in registers; larger ones keep the rows over X' (the X0
-//     members with a P0 neighbour) and the shallow frames in the wave's LDS
-//     when they fit, else in the wave's global arena;
+//     word i) plus XX in X0 space (a stack frame).  Roots of degree <= 64,
+//     those with up to 64 later and 256 earlier neighbours that matter, and
+//     subtrees of any root that small keep everything in registers; the others
+//     keep the rows over X' (the X0 members with a P0 neighbour) and the
+//     shallow frames in the wave's LDS when they fit, else in its global arena;
 //   * pivot scoring gives each candidate to one lane and reduces the key
 //     (score << 32 | position) with a 64-bit wave max: max score, then the
 //     largest position == the reference's "last maximum" rule.
