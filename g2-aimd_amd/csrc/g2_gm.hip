@@ -464,7 +464,7 @@ int gm_run(g2_ctx* c, uint32_t flags, uint64_t* count, uint64_t* per_root, g2_st
     const uint32_t bw = std::min<uint32_t>(c->tune.block_waves, kGmMaxBlockWaves);
     uint64_t nblocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, account ? WK_GM : WK_WALK) / bw);
     const uint64_t cap = std::max<uint64_t>(c->max_degree, 64);
-    const uint64_t per_wave = cap * 2 * c->prog.n * 4;
+    const uint64_t per_wave = cap * (account ? 2 * c->prog.n : walk_lists(c->prog.n)) * 4;
     // shrink the grid until the arenas fit the budget
     nblocks = fit_arenas(c, nblocks, bw * per_wave);
     int rc;

@@ -395,12 +395,14 @@ __device__ inline bool budget_charge(const NodeBudget& nb, uint32_t q, uint64_t&
 
 // One root task: source vertex v0, entries [w0, w1) of `cols` (within its
 // row) as position-1 candidates, and of the position-2 candidates those with
-// index mod parts == part.  The wave's lists live in `ws` (L(id) at id*cap,
-// S(id) at (levels+id)*cap).  `nodes` counts the candidates of positions
-// 1 .. n-2 (BUDGET: those not charged yet).  Returns false when the query's
-// node budget ran out (BUDGET only).
+// index mod parts == part.  The wave's lists of `cap` entries each are L(1) ..
+// L(levels-2), then S(2) .. S(levels-1), for plans of up to `levels` positions
+// (walk_lists): L(id) at ws + id*cap (ws lies one list before the arena), S(id) at
+// ws + (behind+id)*cap, behind = levels-3.  `nodes` counts the candidates of
+// positions 1 .. n-2 (BUDGET: those not charged yet).  Returns false when the
+// query's node budget ran out (BUDGET only).
 template <bool BUDGET>
-__device__ bool walk_root(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t* ws, uint32_t levels, uint32_t v0,
+__device__ bool walk_root(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t* ws, uint32_t behind, uint32_t v0,
                           uint64_t w0, uint64_t w1, uint32_t part, uint32_t parts, uint64_t& lane_total,
                           uint64_t& nodes, const NodeBudget& nb, uint32_t q) {
     const uint32_t lane = lane_id();
@@ -408,6 +410,7 @@ __device__ bool walk_root(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t
     const uint64_t cap = a.cap;
     const uint32_t* __restrict__ cols = a.cols;
     auto LIST = [&](uint32_t id) { return ws + (uint64_t)id * cap; };
+    auto SLIST = [&](uint32_t id) { return LIST(behind + id); };
     wave_sync();  // (the previous task's reads of L are done)
     {
         const GmWalkStep& st = P.step[1];
@@ -464,12 +467,12 @@ __device__ bool walk_root(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t
                 wave_sync();
                 const Range rg = walk_range(L, st.npc, st.pcop, st.pcpos);
                 len = walk_collect<false, false>(L, cols, cols + best0, 0, len, rg, st.npre - 1, nullptr, 0, 0, st.npneq, st.pneq,
-                                          false, 0, LIST(levels + id), top, &off);
+                                          false, 0, SLIST(id), top, &off);
                 if (off != kNotInLds) top += len;
             }
             if (off == kNotInLds && len && (st.prev || id + 1 == n) && len <= kWalkPool - top) {
                 wave_sync();
-                const uint32_t* p = st.npre > 1 ? LIST(levels + id) : cols + best0;
+                const uint32_t* p = st.npre > 1 ? SLIST(id) : cols + best0;
                 for (uint32_t i = lane; i < len; i += kWave) L.pool[top + i] = p[i];
                 off = top;
                 top += len;
@@ -487,7 +490,7 @@ __device__ bool walk_root(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t
     auto source = [&](uint32_t id) -> const uint32_t* {
         const GmWalkStep& st = P.step[id];
         if (st.alias) return LIST(id - 1);
-        return st.npre == 1 ? cols + uniform(L.sst[id]) : LIST(levels + id);
+        return st.npre == 1 ? cols + uniform(L.sst[id]) : SLIST(id);
     };
     prepare(2);
     uint32_t id = 1;
@@ -579,7 +582,7 @@ __device__ inline uint64_t walk_tasks(const GmArgs& a, uint64_t* nheavy) {
 
 // Task t of plan P on this wave; false when the query's node budget ran out.
 template <bool BUDGET>
-__device__ __forceinline__ bool walk_task(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t* ws, uint32_t levels,
+__device__ __forceinline__ bool walk_task(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t* ws, uint32_t behind,
                                           uint64_t t, uint64_t nheavy, uint64_t& lane_total, uint64_t& nodes,
                                           const NodeBudget& nb, uint32_t q) {
     const bool heavy = t < nheavy;
@@ -596,7 +599,7 @@ __device__ __forceinline__ bool walk_task(const GmArgs& a, const GmWalk& P, Walk
         if (!heavy && e1 - e0 > a.heavy_min) continue;
         const uint64_t w0 = e0 + win.first, w1 = heavy ? w0 + win.len : e1;
         const uint64_t before = lane_total;
-        if (!walk_root<BUDGET>(a, P, L, ws, levels, v0, w0, w1, win.part, win.parts, lane_total, nodes, nb, q))
+        if (!walk_root<BUDGET>(a, P, L, ws, behind, v0, w0, w1, win.part, win.parts, lane_total, nodes, nb, q))
             return false;
         if (a.per_root) {
             const uint64_t mine = wave_sum(lane_total - before);
@@ -612,7 +615,7 @@ __global__ __launch_bounds__(256, 5) void walk_kernel(GmArgs a, GmWalk P) {
     const uint32_t wib = threadIdx.x / kWave;
     WalkLds& L = lds[wib];
     const uint64_t gwave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + wib;
-    uint32_t* ws = a.scratch + gwave * a.cap * (2 * P.n);
+    uint32_t* ws = a.scratch + gwave * a.cap * walk_lists(P.n) - a.cap;
     uint64_t lane_total = 0, nodes = 0, nheavy;
     const NodeBudget nb{nullptr, nullptr, 0};
     const uint64_t total = walk_tasks(a, &nheavy);
@@ -620,7 +623,7 @@ __global__ __launch_bounds__(256, 5) void walk_kernel(GmArgs a, GmWalk P) {
     while (true) {
         const uint64_t t = queue_next(a.ctr + GCTR_QUEUE, queue, total);
         if (t == kNoTask) break;
-        walk_task<false>(a, P, L, ws, P.n, t, nheavy, lane_total, nodes, nb, 0);
+        walk_task<false>(a, P, L, ws, P.n - 3, t, nheavy, lane_total, nodes, nb, 0);
     }
     const uint64_t tot = wave_sum(lane_total);
     if (lane == 0) {
@@ -647,7 +650,7 @@ __global__ __launch_bounds__(256, 5) void walk_batch_kernel(GmArgs a, GmBatchArg
     const uint32_t wib = threadIdx.x / kWave;
     WalkLds& L = lds[wib];
     const uint64_t gwave = (uint64_t)blockIdx.x * (blockDim.x / kWave) + wib;
-    uint32_t* ws = a.scratch + gwave * a.cap * (2 * b.levels);
+    uint32_t* ws = a.scratch + gwave * a.cap * walk_lists(b.levels) - a.cap;
     uint64_t nheavy;
     const uint64_t per_q = walk_tasks(a, &nheavy), total = (uint64_t)b.nq * per_q;
     uint32_t queue = (uint32_t)(gwave % kQueues);
@@ -665,7 +668,7 @@ __global__ __launch_bounds__(256, 5) void walk_batch_kernel(GmArgs a, GmBatchArg
         if (lane == 0) over = __hip_atomic_load(&b.nb.qflag[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (uniform(over)) continue;
         uint64_t lane_total = 0;
-        walk_task<true>(a, b.progs[q], L, ws, b.levels, u, nheavy, lane_total, nodes, b.nb, q);
+        walk_task<true>(a, b.progs[q], L, ws, b.levels - 3, u, nheavy, lane_total, nodes, b.nb, q);
         const uint64_t tot = wave_sum(lane_total);
         if (lane == 0 && tot) atomicAdd(&b.qcount[q], (unsigned long long)tot);
     }
@@ -900,7 +903,7 @@ int gm_run_batch(g2_ctx* c, const g2_plan* plans, uint32_t nq, const g2_batch* c
     const uint32_t bw = std::min<uint32_t>(c->tune.block_waves, kGmMaxBlockWaves);
     uint64_t nblocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * wpc / bw);
     const uint64_t cap = std::max<uint64_t>(c->max_degree, 64);
-    const uint64_t per_wave = cap * 2 * levels * 4;
+    const uint64_t per_wave = cap * walk_lists(levels) * 4;
     nblocks = fit_arenas(c, nblocks, bw * per_wave);
     if ((rc = ensure(c, c->counters, GCTR_N * 8, "counters"))) return rc;
     if ((rc = ensure(c, c->scratch, nblocks * bw * per_wave, "wave arenas"))) return rc;

@@ -194,6 +194,13 @@ int walk_split(g2_ctx* c, GmArgs& a, uint32_t n, uint32_t nq, uint32_t chunk);
 uint32_t walk_run(uint64_t ns, uint64_t waves);
 // the counting walk over `blocks` workgroups of block_waves waves
 hipError_t walk_launch(const GmArgs& a, const GmWalk& walk, uint64_t blocks, uint32_t block_waves, hipStream_t s);
+// lists in a wave's arena for plans of up to n positions: the candidates of
+// positions 1 .. n-2 (the last position's are counted, not stored; the one
+// position of an edge may need its list), and what positions 2 .. n-1 take from
+// the rows before the previous position.  20 waves per CU of these take less
+// than 16 with two lists for every position did (R-MAT 22, 4 positions: 13.4
+// GB, 21.4; 26.7 for 20 waves).
+__host__ __device__ inline uint32_t walk_lists(uint32_t n) { return n > 2 ? 2 * (n - 2) : 1; }
 // the largest grid (at most nblocks) whose wave arenas fit the budget
 uint64_t fit_arenas(g2_ctx* c, uint64_t nblocks, uint64_t per_block);
 void gm_local_compile(g2_ctx* c, const g2_plan* p);

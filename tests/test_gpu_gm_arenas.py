@@ -1,0 +1,39 @@
+"""Device memory of the counting walk's wave arenas.  Counts are whole numbers:
+equal to the oracle's, no tolerance."""
+import importlib
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def star(g2, d, chords, seed):
+    """a hub joined to d vertices with a few edges among them"""
+    rng = np.random.default_rng(seed)
+    a, b = rng.integers(1, d + 1, (2, chords))
+    src = np.concatenate((np.zeros(d, np.int64), a))
+    dst = np.concatenate((np.arange(1, d + 1), b))
+    keep = src != dst
+    return g2.Graph.from_edges(src[keep].astype(np.uint32), dst[keep].astype(np.uint32), d + 1)
+
+
+@pytest.mark.parametrize("d,q", [(9000, 0), (9000, 2), (5000, 7)])
+def test_arenas_hold_the_stored_lists(g2, orc, d, q):
+    """patterns of 3, 4 and 5 positions: no more memory than 16 waves per CU
+    with two lists of the largest degree for every position (and 16 MB for the
+    view, the windows and the counters)"""
+    print("case: walk arenas", d, q, flush=True)
+    g = star(g2, d, 300, 5)
+    p = g2.plan_for_preset(q)
+    ref = orc.gm(g, orc.OrcPlan.from_buffer_copy(bytes(p)), per_root=True)
+    cus = importlib.import_module("g2-aimd_amd.device").device_info()["num_cus"]
+    with g2.Executor(device=0) as ex:
+        ex.transfer(g)
+        ex.set_plan(p)
+        got = ex.run_gm(per_root=True, canonical=True)
+        solo = got["stats"]["device_bytes"]
+        batch = ex.run_gm_batch([p])
+    assert got["count"] == ref["count"] == batch["counts"][0]
+    assert np.array_equal(got["per_root_count"], ref["per_root_count"])
+    assert solo <= cus * 16 * d * 2 * p.n * 4 + (16 << 20)
