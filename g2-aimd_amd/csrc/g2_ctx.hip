@@ -80,11 +80,19 @@ int hip_err(g2_ctx* c, hipError_t e, const char* what) {
     return set_err(c, G2_EHIP, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+static void release(g2_ctx* c, DevBuf& b) {
+    if (b.ptr) (void)hipFree(b.ptr);
+    c->used -= b.bytes;
+    b.ptr = nullptr;
+    b.bytes = 0;
+}
+
 int ensure(g2_ctx* c, DevBuf& b, uint64_t bytes, const char* what) {
     if (bytes <= b.bytes) return G2_OK;
     bytes = (bytes + 255) & ~255ull;
-    const uint64_t after = c->used - b.bytes + bytes;
-    if (c->budget && after > c->budget)
+    DevBuf& w = c->windows;
+    if (c->budget && c->used - b.bytes + bytes > c->budget && &b != &w) release(c, w);
+    if (c->budget && c->used - b.bytes + bytes > c->budget)
         return set_err(c, G2_EBUDGET, std::string(what) + ": needs " + std::to_string(bytes) +
                                           " B, budget left " + std::to_string(c->budget - (c->used - b.bytes)));
     if (b.ptr) {
@@ -95,17 +103,22 @@ int ensure(g2_ctx* c, DevBuf& b, uint64_t bytes, const char* what) {
         b.bytes = 0;
     }
     hipError_t e = hipMalloc(&b.ptr, bytes);
-    if (e != hipSuccess) return hip_err(c, e, what);
+    if (e != hipSuccess && &b != &w && w.ptr) {
+        release(c, w);
+        e = hipMalloc(&b.ptr, bytes);
+    }
+    if (e != hipSuccess) {
+        b.ptr = nullptr;
+        (void)hipGetLastError();  // (reported here, not by the next launch)
+        return hip_err(c, e, what);
+    }
     b.bytes = bytes;
     c->used += bytes;
     return G2_OK;
 }
 
-static void release(g2_ctx* c, DevBuf& b) {
-    if (b.ptr) (void)hipFree(b.ptr);
-    c->used -= b.bytes;
-    b.ptr = nullptr;
-    b.bytes = 0;
+void windows_release(g2_ctx* c) {
+    if (c->budget) release(c, c->windows);
 }
 
 static void apply_tuning_defaults(g2_ctx* c) {
@@ -187,7 +200,7 @@ void g2_destroy(g2_ctx* c) {
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     for (DevBuf* b : {&c->rp, &c->cols, &c->src, &c->gm_task_off, &c->counters, &c->scratch,
-                      &c->big_scratch, &c->list, &c->per_root, &c->order, &c->deg, &c->big_list2, &c->spans,
+                      &c->big_scratch, &c->list, &c->windows, &c->per_root, &c->order, &c->deg, &c->big_list2, &c->spans,
                       &c->batch_progs, &c->batch_q, &c->donate, &c->taskbuild, &c->orient, &c->roots})
         release(c, *b);
     if (c->spill) (void)hipHostFree(c->spill);
@@ -234,6 +247,7 @@ int g2_upload_view(g2_ctx* c, const uint64_t* rp, uint64_t nv, const uint32_t* c
         if (chunk && d > chunk) w = (d + chunk - 1) / chunk;
         task_off[i + 1] = task_off[i] + w;
     }
+    windows_release(c);
     // The budget is checked for every view buffer before any is replaced, so
     // a refused upload leaves the previous view intact.
     struct Need { DevBuf* b; uint64_t bytes; const char* what; };
@@ -297,6 +311,7 @@ int g2_upload_view(g2_ctx* c, const uint64_t* rp, uint64_t nv, const uint32_t* c
     c->h_gm_task_off.swap(task_off);
     c->h_src_deg.swap(src_deg);
     c->src_deg_sum = deg_sum;
+    c->walk_parts = 0;
     c->batch_tasks_valid = false;
     c->view_ok = true;
     return G2_OK;

@@ -465,27 +465,30 @@ int gm_run(g2_ctx* c, uint32_t flags, uint64_t* count, uint64_t* per_root, g2_st
     uint64_t nblocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, account ? WK_GM : WK_WALK) / bw);
     const uint64_t cap = std::max<uint64_t>(c->max_degree, 64);
     const uint64_t per_wave = cap * (account ? 2 * c->prog.n : walk_lists(c->prog.n)) * 4;
-    // shrink the grid until the arenas fit the budget
-    nblocks = fit_arenas(c, nblocks, bw * per_wave);
     int rc;
     if ((rc = ensure(c, c->counters, GCTR_N * 8, "counters"))) return rc;
-    if ((rc = ensure(c, c->scratch, nblocks * bw * per_wave, "wave arenas"))) return rc;
-    if (per_root && (rc = ensure(c, c->per_root, std::max<uint64_t>(c->ns, 1) * 8, "per-root counts"))) return rc;
     hipError_t e;
     auto* ctr = (unsigned long long*)c->counters.ptr;
     if ((e = hipMemsetAsync(ctr, 0, GCTR_N * 8, c->stream))) return hip_err(c, e, "memset counters");
-    if (per_root && (e = hipMemsetAsync(c->per_root.ptr, 0, c->ns * 8, c->stream))) return hip_err(c, e, "memset per-root");
     GmArgs a{};
     a.rp = (const uint64_t*)c->rp.ptr;
     a.cols = (const uint32_t*)c->cols.ptr;
     a.src = (const uint32_t*)c->src.ptr;
-    a.task_off = (const uint64_t*)c->gm_task_off.ptr;
     a.ns = c->ns;
+    a.ctr = ctr;
+    WalkRule rule{};
+    if (account) windows_release(c);
+    else if ((rc = walk_reserve(c, a, c->walk.n, 1, c->gm_task_chunk, &rule))) return rc;
+    // shrink the grid until the arenas fit the budget
+    nblocks = fit_arenas(c, nblocks, bw * per_wave);
+    if ((rc = ensure(c, c->scratch, nblocks * bw * per_wave, "wave arenas"))) return rc;
+    if (per_root && (rc = ensure(c, c->per_root, std::max<uint64_t>(c->ns, 1) * 8, "per-root counts"))) return rc;
+    if (per_root && (e = hipMemsetAsync(c->per_root.ptr, 0, c->ns * 8, c->stream))) return hip_err(c, e, "memset per-root");
+    a.task_off = (const uint64_t*)c->gm_task_off.ptr;
     a.ntasks = c->h_gm_task_off.empty() ? 0 : c->h_gm_task_off.back();
     a.chunk = c->gm_task_chunk;
     a.scratch = (uint32_t*)c->scratch.ptr;
     a.cap = cap;
-    a.ctr = ctr;
     a.per_root = per_root ? (unsigned long long*)c->per_root.ptr : nullptr;
     if ((e = hipEventRecord(c->ev[0], c->stream))) return hip_err(c, e, "event");
     if (account) {
@@ -493,7 +496,7 @@ int gm_run(g2_ctx* c, uint32_t flags, uint64_t* count, uint64_t* per_root, g2_st
         if ((e = hipGetLastError())) return hip_err(c, e, "gm launch");
     } else {
         a.run = walk_run(c->ns, nblocks * bw);
-        if ((rc = walk_split(c, a, c->walk.n, 1, c->gm_task_chunk))) return rc;
+        if ((rc = walk_list(c, a, rule))) return rc;
         if ((e = walk_launch(a, c->walk, nblocks, bw, c->stream))) return hip_err(c, e, "gm launch");
     }
     if ((e = hipEventRecord(c->ev[1], c->stream))) return hip_err(c, e, "event");

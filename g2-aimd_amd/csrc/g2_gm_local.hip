@@ -1710,6 +1710,7 @@ static int pass_roots(g2_ctx* c, const uint64_t* orp, const uint32_t* rank, uint
 // so the passes are enqueued back to back and waited for once.
 int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     if (c->nv + 1 > 0x7fffffffull) return set_err(c, G2_EINVAL, "local-bitmap matching supports fewer than 2^31-1 vertices");
+    windows_release(c);
     const uint32_t bw = std::min<uint32_t>(c->tune.block_waves, kLocalBlockWaves);
     const uint64_t nblocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, WK_GM_LOCAL) / bw);
     // roots: every rank of a whole-graph view, else the ranks of the sources

@@ -686,18 +686,11 @@ __global__ __launch_bounds__(256) void walk_batch_init_kernel(NodeBudget nb, uns
     nb.qflag[q] = ntasks > nb.limit ? 1u : 0u;
 }
 
-// The windows of the sources whose row is longer than heavy_min.  Windows of
-// one entry (part_deg > 0) are dealt out further, in parts of the position-2
-// candidates, by the smaller of the two degrees.  A wave takes `per` sources,
-// lists their windows as one sequence over its lanes, and reserves their places
-// with one atomic (64 windows at a time where they are dealt out): source by
-// source, an atomic's round trip for each, the 100k-vertex Chung-Lu graph's
-// list took 385 us of a call of 1.85 ms, now 1.60.
-struct WalkRule {
-    uint64_t work, least, most;  // window length: work / row length, within [least, most]
-    uint32_t part_deg;           // entries of the smaller row per part (0: whole windows)
-    uint32_t per;                // sources per wave, at most 64
-};
+// The windows of the sources whose row is longer than heavy_min.  A wave takes
+// `per` sources, lists their windows as one sequence over its lanes, and reserves
+// their places with one atomic (64 windows at a time where they are dealt out):
+// source by source, an atomic's round trip for each, the 100k-vertex Chung-Lu
+// graph's list took 385 us of a call of 1.85 ms, now 1.60.
 __global__ __launch_bounds__(256) void walk_split_kernel(GmArgs a, WalkWindow* heavy, WalkRule rule) {
     const uint32_t lane = lane_id();
     const uint64_t nw = (uint64_t)gridDim.x * blockDim.x / kWave;
@@ -746,7 +739,7 @@ __global__ __launch_bounds__(256) void walk_split_kernel(GmArgs a, WalkWindow* h
             if (rule.part_deg) {
                 if (parts) {
                     const uint32_t u = a.cols[ek + j];
-                    parts = (uint32_t)umin64(kWalkParts, 1 + umin64(dk, a.rp[u + 1] - a.rp[u]) / rule.part_deg);
+                    parts = (uint32_t)umin64(rule.parts, 1 + umin64(dk, a.rp[u + 1] - a.rp[u]) / rule.part_deg);
                 }
                 const uint64_t sum = before(parts);
                 at = reserve(read_lane(sum, kWave - 1)) + sum - parts;
@@ -799,7 +792,7 @@ GmWalk walk_program(const GmProgram& g) {
 }
 
 // Windows of the long root rows, listed on the device (a.heavy stays null
-// where no row is long, or the budget cannot hold the list).  chunk: the
+// where no row is long, or the list does not fit).  chunk: the
 // caller's window length, 0 = by rule.  The rule: a window is one wave's
 // serial work.  With 3 positions a window is one flattened count, so it only
 // has to fill the lanes.  With 4, every entry is a list and a count of its own
@@ -809,17 +802,38 @@ GmWalk walk_program(const GmProgram& g) {
 // with the row's length in; 4-cycles of 5k vertices: 3.4 ms with 8, 0.8).  With
 // 5 or more it is a walk of lists: single entries, dealt out further where two
 // hubs meet (the 8-edge pattern on R-MAT 9: 6.7 ms undealt, 1.7 dealt, 1.4 and
-// 2.5 with a part per 16 and 64 entries, which reverse on flatter graphs).  The
-// list stays under 2^21 windows (2^18 where they are dealt
-// out) plus one per long row.
-int walk_split(g2_ctx* c, GmArgs& a, uint32_t n, uint32_t nq, uint32_t chunk) {
+// 2.5 with a part per 16 and 64 entries, which reverse on flatter graphs).
+//   The list stays under 2^22 windows plus one per long row (76 MB; 134 with a
+// caller's windows of single entries): windows, the caller's too, are at least the
+// sources' row entries / 2^21 long.  Dealt out, it stays under kWalkDealt (268 MB),
+// for which the most parts are halved: at 4 instead of 8 an 8-edge pattern takes
+// 36.3 ms for 32.4 on the 100k-vertex Chung-Lu graph (a 6-edge one 6.5 for 7.3), so
+// only where the list would not fit.  From 2^22 row entries on nothing is dealt
+// out.  How many parts the windows have at most follows from the sources' degrees,
+// once per view (94 MB for that graph; 8 parts for every window 286).  Counted on
+// the device, call by call, they took 0.35 ms of 3.8 (6 edges, 50k vertices); up to
+// 466k row entries room for 8 parts of every window is taken instead (67 MB).
+constexpr uint64_t kWalkDealt = 1ull << 24, kWalkDealtPlain = 1ull << 22;
+// the most windows of one entry that the view's long rows have, dealt out in up
+// to `most` parts each
+static uint64_t dealt_windows(g2_ctx* c, uint64_t min_row, uint32_t most) {
+    uint64_t n = 0;
+    for (uint64_t d : c->h_src_deg)
+        if (d > min_row) n += d * std::min<uint64_t>(most, 1 + d / kWalkPartDeg);
+    return n;
+}
+static uint64_t split_blocks(g2_ctx* c) {
+    return std::max<uint64_t>(1, std::min<uint64_t>((c->ns + 3) / 4, (uint64_t)c->num_cus * 8));
+}
+int walk_reserve(g2_ctx* c, GmArgs& a, uint32_t n, uint32_t nq, uint32_t chunk, WalkRule* out) {
     a.heavy = nullptr;
     a.heavy_min = ~0ull;
-    WalkRule rule{0, chunk, chunk, 0, 1};
-    uint64_t min_row = chunk;
+    const uint64_t shortest = std::max<uint64_t>(c->src_deg_sum >> 21, chunk);
+    WalkRule rule{0, shortest, shortest, 0, kWalkParts, 1, 0};
+    uint64_t min_row = shortest;
+    *out = rule;
     if (!chunk) {
         const uint64_t waves = (uint64_t)c->num_cus * waves_per_cu(c, WK_WALK);
-        rule.least = c->src_deg_sum >> 21;
         if (n <= 3) rule.least = std::max<uint64_t>(rule.least, 64);
         rule.least = rule.most = std::max<uint64_t>(rule.least, 1);
         if (n == 4) {
@@ -829,20 +843,48 @@ int walk_split(g2_ctx* c, GmArgs& a, uint32_t n, uint32_t nq, uint32_t chunk) {
         min_row = n <= 3 ? 2 * rule.most : 8 * rule.most;
         if (n >= 5 && rule.most == 1) rule.part_deg = kWalkPartDeg;
     }
-    if (c->max_degree <= min_row) return G2_OK;
-    a.heavy_min = min_row;
-    const uint64_t cap = (c->src_deg_sum / rule.least + c->src_deg_sum / min_row + 1) * (rule.part_deg ? kWalkParts : 1u);
-    int rc;
-    if ((rc = ensure(c, c->list, cap * sizeof(WalkWindow), "root windows"))) {
-        a.heavy_min = ~0ull;
-        return rc == G2_EBUDGET ? G2_OK : rc;
+    if (c->max_degree <= min_row) {
+        windows_release(c);
+        return G2_OK;
     }
-    const uint64_t blocks = std::max<uint64_t>(1, std::min<uint64_t>((c->ns + 3) / 4, (uint64_t)c->num_cus * 8));
+    const uint64_t blocks = split_blocks(c);
     rule.per = (uint32_t)std::min<uint64_t>(kWave, (c->ns + blocks * 4 - 1) / (blocks * 4));
-    hipLaunchKernelGGL(walk_split_kernel, dim3(blocks), dim3(256), 0, c->stream, a, (WalkWindow*)c->list.ptr, rule);
+    uint64_t windows = c->src_deg_sum / rule.least + c->src_deg_sum / min_row + 1;
+    a.heavy_min = min_row;
+    if (rule.part_deg && windows * kWalkParts <= kWalkDealtPlain) {
+        windows *= kWalkParts;
+    } else if (rule.part_deg) {
+        if (!c->walk_parts) {  // (min_row is the same for every plan that deals windows out)
+            c->walk_parts = kWalkParts;
+            while ((c->walk_dealt = dealt_windows(c, min_row, c->walk_parts)) > kWalkDealt && c->walk_parts > 1)
+                c->walk_parts /= 2;
+        }
+        rule.parts = c->walk_parts;
+        if (rule.parts > 1) windows = c->walk_dealt;
+        else rule.part_deg = 0;
+    }
+    const uint64_t bytes = windows * sizeof(WalkWindow);
+    if (c->windows.bytes / 2 > bytes) windows_release(c);
+    if (ensure(c, c->windows, bytes, "root windows") == G2_OK) {
+        rule.bytes = bytes;
+    } else {  // (without a list the rows are walked whole)
+        a.heavy_min = ~0ull;
+        c->err.clear();
+    }
+    *out = rule;
+    return G2_OK;
+}
+
+int walk_list(g2_ctx* c, GmArgs& a, const WalkRule& rule) {
+    if (!rule.bytes || c->windows.bytes < rule.bytes) {  // (given back for the arenas)
+        a.heavy_min = ~0ull;
+        return G2_OK;
+    }
+    hipLaunchKernelGGL(walk_split_kernel, dim3(split_blocks(c)), dim3(256), 0, c->stream, a,
+                       (WalkWindow*)c->windows.ptr, rule);
     hipError_t e = hipGetLastError();
     if (e) return hip_err(c, e, "root windows launch");
-    a.heavy = (const WalkWindow*)c->list.ptr;
+    a.heavy = (const WalkWindow*)c->windows.ptr;
     return G2_OK;
 }
 
@@ -904,34 +946,36 @@ int gm_run_batch(g2_ctx* c, const g2_plan* plans, uint32_t nq, const g2_batch* c
     uint64_t nblocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * wpc / bw);
     const uint64_t cap = std::max<uint64_t>(c->max_degree, 64);
     const uint64_t per_wave = cap * walk_lists(levels) * 4;
-    nblocks = fit_arenas(c, nblocks, bw * per_wave);
     if ((rc = ensure(c, c->counters, GCTR_N * 8, "counters"))) return rc;
-    if ((rc = ensure(c, c->scratch, nblocks * bw * per_wave, "wave arenas"))) return rc;
-    if ((rc = ensure(c, c->batch_progs, (uint64_t)nq * sizeof(GmWalk), "batch programs"))) return rc;
-    // per query: order u32, count u64, nodes u64, flag u32
-    const uint64_t qbytes = (uint64_t)nq * 24;
-    if ((rc = ensure(c, c->batch_q, qbytes, "batch query state"))) return rc;
     auto* ctr = (unsigned long long*)c->counters.ptr;
-    auto* qcount = (unsigned long long*)c->batch_q.ptr;
-    auto* qn = qcount + nq;
-    auto* qord = (uint32_t*)(qn + nq);
-    auto* qflag = qord + nq;
     hipError_t e;
-    if ((e = hipMemcpyAsync(c->batch_progs.ptr, progs.data(), (uint64_t)nq * sizeof(GmWalk), hipMemcpyHostToDevice,
-                            c->stream)))
-        return hip_err(c, e, "H2D batch programs");
-    if ((e = hipMemcpyAsync(qord, order.data(), (uint64_t)nq * 4, hipMemcpyHostToDevice, c->stream)))
-        return hip_err(c, e, "H2D query order");
     if ((e = hipMemsetAsync(ctr, 0, GCTR_N * 8, c->stream))) return hip_err(c, e, "memset counters");
     GmArgs a{};
     a.rp = (const uint64_t*)c->rp.ptr;
     a.cols = (const uint32_t*)c->cols.ptr;
     a.src = (const uint32_t*)c->src.ptr;
     a.ns = c->ns;
+    a.ctr = ctr;
+    WalkRule rule;
+    if ((rc = walk_reserve(c, a, levels, nq, cfg->window, &rule))) return rc;
+    nblocks = fit_arenas(c, nblocks, bw * per_wave);
+    if ((rc = ensure(c, c->scratch, nblocks * bw * per_wave, "wave arenas"))) return rc;
+    if ((rc = ensure(c, c->batch_progs, (uint64_t)nq * sizeof(GmWalk), "batch programs"))) return rc;
+    // per query: order u32, count u64, nodes u64, flag u32
+    const uint64_t qbytes = (uint64_t)nq * 24;
+    if ((rc = ensure(c, c->batch_q, qbytes, "batch query state"))) return rc;
+    auto* qcount = (unsigned long long*)c->batch_q.ptr;
+    auto* qn = qcount + nq;
+    auto* qord = (uint32_t*)(qn + nq);
+    auto* qflag = qord + nq;
+    if ((e = hipMemcpyAsync(c->batch_progs.ptr, progs.data(), (uint64_t)nq * sizeof(GmWalk), hipMemcpyHostToDevice,
+                            c->stream)))
+        return hip_err(c, e, "H2D batch programs");
+    if ((e = hipMemcpyAsync(qord, order.data(), (uint64_t)nq * 4, hipMemcpyHostToDevice, c->stream)))
+        return hip_err(c, e, "H2D query order");
     a.run = std::max<uint32_t>(cfg->roots_per_task, 1);
     a.scratch = (uint32_t*)c->scratch.ptr;
     a.cap = cap;
-    a.ctr = ctr;
     a.per_root = nullptr;
     GmBatchArgs b{};
     b.progs = (const GmWalk*)c->batch_progs.ptr;
@@ -942,7 +986,7 @@ int gm_run_batch(g2_ctx* c, const g2_plan* plans, uint32_t nq, const g2_batch* c
     b.nb = NodeBudget{qn, qflag, cfg->node_budget ? cfg->node_budget : ~0ull};
     hipLaunchKernelGGL(walk_batch_init_kernel, dim3((nq + 255) / 256), dim3(256), 0, c->stream, b.nb, qcount, nq, ntasks);
     if ((e = hipEventRecord(c->ev[0], c->stream))) return hip_err(c, e, "event");
-    if ((rc = walk_split(c, a, levels, nq, cfg->window))) return rc;
+    if ((rc = walk_list(c, a, rule))) return rc;
     hipLaunchKernelGGL(walk_batch_kernel, dim3(nblocks), dim3(bw * kWave), 0, c->stream, a, b);
     if ((e = hipGetLastError())) return hip_err(c, e, "batch launch");
     if ((e = hipEventRecord(c->ev[1], c->stream))) return hip_err(c, e, "event");

@@ -71,6 +71,16 @@ struct WalkWindow {
     uint16_t part, parts;
 };
 
+// How the rows longer than GmArgs::heavy_min are cut into windows.  Windows of
+// one entry (part_deg > 0) are dealt out further, in parts of the position-2
+// candidates, by the smaller of the two degrees.
+struct WalkRule {
+    uint64_t work, least, most;  // window length: work / row length, within [least, most]
+    uint32_t part_deg, parts;    // entries of the smaller row per part (0: whole windows), most parts
+    uint32_t per;                // sources per wave, at most 64
+    uint64_t bytes;              // room the list needs (0: no list)
+};
+
 struct GmArgs {
     const uint64_t* __restrict__ rp;
     const uint32_t* __restrict__ cols;
@@ -131,6 +141,8 @@ struct g2_ctx {
     g2::DevBuf scratch;           // per-wave arenas
     g2::DevBuf big_scratch;
     g2::DevBuf list;              // deferred roots
+    g2::DevBuf windows;           // matching: windows of the long root rows, of the current run only:
+                                  // given back when another buffer does not fit (ensure)
     g2::DevBuf per_root;
     g2::DevBuf order;
     g2::DevBuf spans;
@@ -157,6 +169,8 @@ struct g2_ctx {
     // batched matching
     std::vector<uint64_t> h_src_deg;  // host copy: degree of every source
     uint64_t src_deg_sum = 0;
+    uint32_t walk_parts = 0;          // most parts of a window of the view (0: not chosen yet)
+    uint64_t walk_dealt = 0;          // and the windows there are with them, at most
     uint32_t batch_window = 0;        // root tasks of the last batch window
     uint64_t batch_ntasks = 0;
     bool batch_tasks_valid = false;
@@ -176,8 +190,13 @@ inline uint32_t waves_per_cu(const g2_ctx* c, WaveKind k) {
     return c->tune.waves_per_cu ? c->tune.waves_per_cu : (uint32_t)k;
 }
 int hip_err(g2_ctx* c, hipError_t e, const char* what);
-// make sure buf holds at least `bytes`; charged against the budget
+// make sure buf holds at least `bytes`; charged against the budget.  Where they
+// do not fit, the window list gives way (a matching run without it walks the
+// rows whole, and between runs it holds nothing).
 int ensure(g2_ctx* c, DevBuf& buf, uint64_t bytes, const char* what);
+// under a budget, give the window list back: for what sizes itself by the
+// budget that is left, and needs no list
+void windows_release(g2_ctx* c);
 
 int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, uint64_t* hist,
             uint32_t hist_len, uint64_t* per_root_nodes, g2_stats* st);
@@ -186,9 +205,12 @@ int gm_compile(g2_ctx* c, const g2_plan* p);
 // plan tables re-indexed by position; G2_EINVAL with *why naming the first broken table
 int gm_program(const g2_plan* p, GmProgram* out, const char** why);
 GmWalk walk_program(const GmProgram& g);
-// list the windows of the long root rows into a, for nq plans of up to n
-// positions (chunk: window length, 0 = by rule)
-int walk_split(g2_ctx* c, GmArgs& a, uint32_t n, uint32_t nq, uint32_t chunk);
+// choose the windows of the long root rows for nq plans of up to n positions
+// (chunk: window length, 0 = by rule) and make room for their list; rows are
+// walked whole where there is none.  a.ctr is cleared.
+int walk_reserve(g2_ctx* c, GmArgs& a, uint32_t n, uint32_t nq, uint32_t chunk, WalkRule* rule);
+// list them into a, once the run's other buffers are there
+int walk_list(g2_ctx* c, GmArgs& a, const WalkRule& rule);
 // sources per task of the counting walk: blocks of up to 16 where every wave
 // still gets several (short rows cost little more than their fetch)
 uint32_t walk_run(uint64_t ns, uint64_t waves);

@@ -1975,6 +1975,7 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
     const uint32_t bw = std::min<uint32_t>(c->tune.block_waves, kMaxBlockWaves);
     uint64_t nblocks = std::max<uint64_t>(1, (uint64_t)c->num_cus * waves_per_cu(c, WK_MCE) / bw);
     const uint64_t sw = c->tune.wave_scratch_words;
+    windows_release(c);
     // under a budget the grid shrinks until its wave arenas fit what the
     // budget leaves (fewer resident waves, same result)
     if (c->budget) {
