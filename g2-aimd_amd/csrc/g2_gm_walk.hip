@@ -495,12 +495,13 @@ __device__ bool walk_root(const GmArgs& a, const GmWalk& P, WalkLds& L, uint32_t
     prepare(2);
     uint32_t id = 1;
     while (true) {
+        // (here, so that a walk that never gets to its last position is charged too)
+        if (BUDGET && nodes >= kBudgetBlock && budget_charge(nb, q, nodes)) return false;
         const uint32_t len = uniform(L.len[id]), loff = uniform(L.loff[id]);
         const uint32_t nx = id + 1;
         const GmWalkStep& st = P.step[nx];
         const uint32_t sn = uniform(L.slen[nx]), soff = uniform(L.soff[nx]);
         if (nx + 1 == n) {
-            if (BUDGET && nodes >= kBudgetBlock && budget_charge(nb, q, nodes)) return false;
             const bool raw = st.npre == 1 && !st.alias;
             if (soff != kNotInLds) lane_total += walk_last<true>(a, L, st, LIST(id), loff, len, nullptr, soff, sn, raw);
             else if (!st.npre || sn) lane_total += walk_last<false>(a, L, st, LIST(id), loff, len, source(nx), 0, sn, raw);
