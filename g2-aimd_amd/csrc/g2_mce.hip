@@ -2009,25 +2009,44 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
         first = sched->begin;
         ntasks = sched->end;
     }
-    // work donation: tallies, rings and mailboxes (cleared before a launch), then a record area per wave
+    // work donation: tallies, rings and mailboxes (cleared before a launch), then
+    // a record area per wave, for launches of up to donation_waves waves
     const uint32_t every = account ? 0u : (c->tune.mce_donate_every == 0xffffffffu ? 0u : c->tune.mce_donate_every);
-    uint32_t ring_size = 64;
-    while ((uint64_t)ring_size * kRings < nwaves + kRings) ring_size *= 2;
-    const uint64_t done_bytes = kDqStride * 8, rings_bytes = kRings * kDqStride * 8,
-                   ring_bytes = (uint64_t)kRings * ring_size * 4, mail_bytes = nwaves * kDqStride * 8;
-    const uint64_t clear_bytes = done_bytes + rings_bytes + ring_bytes + mail_bytes;
-    if ((rc = ensure(c, c->donate, clear_bytes + nwaves * kRecWords * 8, "work donation"))) return rc;
+    MceArgs a{};
+    uint64_t donation_waves = 0, clear_bytes = 0;
+    const uint64_t done_bytes = kDqStride * 8, rings_bytes = kRings * kDqStride * 8;
+    auto ring_size = [](uint64_t waves) {
+        uint32_t n = 64;
+        while ((uint64_t)n * kRings < waves + kRings) n *= 2;
+        return n;
+    };
+    auto donation_clear = [&](uint64_t waves) {
+        return done_bytes + rings_bytes + (uint64_t)kRings * ring_size(waves) * 4 + waves * kDqStride * 8;
+    };
+    auto donation_bytes = [&](uint64_t waves) { return donation_clear(waves) + waves * kRecWords * 8; };
+    auto place_donation = [&](uint64_t waves) -> int {
+        if (int r = ensure(c, c->donate, donation_bytes(waves), "work donation")) return r;
+        char* dq = (char*)c->donate.ptr;
+        donation_waves = waves;
+        clear_bytes = donation_clear(waves);
+        a.done = (unsigned long long*)dq;
+        a.rings = (unsigned int*)(dq + done_bytes);
+        a.ring = (unsigned int*)(dq + done_bytes + rings_bytes);
+        a.ring_mask = ring_size(waves) - 1;
+        a.mail = (unsigned long long*)(dq + clear_bytes - waves * kDqStride * 8);
+        a.area = (uint64_t*)(dq + clear_bytes);
+        return G2_OK;
+    };
+    if ((rc = place_donation(nwaves))) return rc;
     // the one buffer that grows with the number of root tasks comes last, so
     // that a smaller range of roots fits where the whole view did not
     if ((rc = ensure(c, c->list, std::max<uint64_t>(ntasks - first, 1) * 8, "deferred roots"))) return rc;
-    char* dq = (char*)c->donate.ptr;
-    auto reset_donation = [&]() -> hipError_t { return every ? hipMemsetAsync(dq, 0, clear_bytes, c->stream) : hipSuccess; };
+    auto reset_donation = [&]() -> hipError_t { return every ? hipMemsetAsync(c->donate.ptr, 0, clear_bytes, c->stream) : hipSuccess; };
     hipError_t e;
     auto* ctr = (unsigned long long*)c->counters.ptr;
     if ((e = hipMemsetAsync(ctr, 0, clear_words * 8, c->stream))) return hip_err(c, e, "memset counters");
     if (per_root_nodes && (e = hipMemsetAsync(c->per_root.ptr, 0, c->ns * 8, c->stream))) return hip_err(c, e, "memset per-root");
 
-    MceArgs a{};
     a.rp = (const uint64_t*)c->rp.ptr;
     a.cols = (const uint32_t*)c->cols.ptr;
     a.src = (const uint32_t*)c->src.ptr;
@@ -2050,12 +2069,6 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
     // 800k 39.6 -> 30.7).  A run without donation keeps the source order, the
     // reference's, as the plain form the others are measured against.
     a.backwards = every && !(sched && sched->order);
-    a.done = (unsigned long long*)dq;
-    a.rings = (unsigned int*)(dq + done_bytes);
-    a.ring = (unsigned int*)(dq + done_bytes + rings_bytes);
-    a.ring_mask = ring_size - 1;
-    a.mail = (unsigned long long*)(dq + done_bytes + rings_bytes + ring_bytes);
-    a.area = (uint64_t*)(dq + clear_bytes);
     a.nwaves = (uint32_t)nwaves;
     a.donate_every = every;
 
@@ -2092,8 +2105,25 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
         // many waves as the budget holds (whole workgroups of bw waves, or
         // one smaller workgroup)
         const uint64_t need = h_ctr[CTR_MAXNEED];
-        uint64_t bwaves = std::min<uint64_t>(c->tune.big_waves, nbig);
-        while (bwaves > 1 && c->budget && c->used - c->big_scratch.bytes + bwaves * need * 8 > c->budget) bwaves /= 2;
+        const uint64_t most = std::min<uint64_t>(std::max<uint32_t>(c->tune.big_waves, 1), nbig);
+        // A budget or a tuning may have left the first pass with fewer waves than
+        // this one takes; every wave of this one, too, needs its mailbox and record
+        // area (no more waves than there is room for them)
+        auto with_donation = [&](uint64_t waves, uint64_t* fit) -> int {
+            *fit = waves;
+            if (!every || waves <= donation_waves || place_donation(waves) == G2_OK) return G2_OK;
+            c->err.clear();
+            *fit = nwaves;
+            return place_donation(nwaves);
+        };
+        uint64_t bwaves = most;
+        auto after = [&]() {  // device memory held with that many waves
+            const uint64_t more = every && bwaves > donation_waves ? donation_bytes(bwaves) + 256 : 0;
+            return c->used - c->big_scratch.bytes + bwaves * need * 8 +
+                   (more > c->donate.bytes ? more - c->donate.bytes : 0);
+        };
+        while (bwaves > 1 && c->budget && after() > c->budget) bwaves /= 2;
+        if ((rc = with_donation(bwaves, &bwaves))) return rc;
         big_bw = (uint32_t)std::min<uint64_t>(bw, bwaves);
         bwaves = bwaves / big_bw * big_bw;
         uint64_t* arenas = nullptr;
@@ -2107,7 +2137,7 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
             // only for budgets far below the roots' needs; the result is the
             // same.  The reference's host spill is dumpToHost / loadFromHost
             // (app_BK/BK.h:357-398, system/subgraph_container.h:213-216).
-            bwaves = std::min<uint64_t>(std::max<uint32_t>(c->tune.big_waves, 1), nbig);
+            if ((rc = with_donation(most, &bwaves))) return rc;
             big_bw = (uint32_t)std::min<uint64_t>(bw, bwaves);
             bwaves = bwaves / big_bw * big_bw;
             if ((rc = host_spill(c, bwaves * need * 8))) return rc;
