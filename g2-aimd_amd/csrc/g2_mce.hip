@@ -75,14 +75,20 @@ struct MceArgs {
     uint32_t ring_mask;
     unsigned long long* done;            // units of work done: roots and records, less records made
     unsigned long long* mail;            // per wave, a line each: MAIL_*
-    uint64_t* area;                      // per wave: kRecWords record words
+    uint64_t* area;                      // per wave: rec_words record words
+    uint64_t rec_words;
     uint32_t nwaves;
     uint32_t donate_every;               // nodes between looks for idle waves (0 = never donate)
 };
 
 constexpr uint32_t kRings = 16;
 constexpr uint64_t kDqStride = 16;       // u64 words of one 128-byte line
-constexpr uint32_t kRecWords = 1024;     // longest record; a wider root's frames are not handed on
+// Longest record, and the least of a launch's rec_words.  Frames of the default
+// arenas' roots fit it (one of 1,023 words needs more than 65,142 earlier
+// neighbours, hence an arena beyond 2^16 words).  The large-root pass has fewer
+// waves and divides the same areas among them: 16,384 words for 256, or about a
+// million earlier neighbours.  A frame wider than that is not handed on.
+constexpr uint32_t kRecWords = 1024;
 constexpr uint32_t kRecRows = 16;         // first row word of a record that takes its rows along
 constexpr uint64_t kRegRecord = 1ull << 32;  // kind of a register_walk record (wide_walk<R>: R << 32; none: rows rebuilt)
 // A task looks for idle waves from this many x donate_every nodes on.  Fewer hand
@@ -527,7 +533,7 @@ __device__ __forceinline__ uint64_t register_walk(const MceArgs& a, uint32_t si,
                                      : lane == 2 ? (fp & ~keep) : lane == 3 ? (fxp | keep) : lane == 4 ? (fq & ~keep)
                                      : lane == 5 ? fxx : lane == 6 ? (uint64_t)s : (uint64_t)d;
                     record_made(a);
-                    unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * kRecWords;
+                    unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * a.rec_words;
                     if (lane < 8) st_dev(out + lane, w);
                     st_dev(out + kRecRows + lane, rowP);
                     st_dev(out + kRecRows + kWave + lane, rowX);
@@ -647,7 +653,7 @@ __device__ __forceinline__ uint64_t wide_walk(const MceArgs& a, uint32_t si, uin
                         w = lane == 5u + r ? fx : w;
                     }
                     record_made(a);
-                    unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * kRecWords;
+                    unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * a.rec_words;
                     if (lane < 5 + R) st_dev(out + lane, w);
                     st_dev(out + kRecRows + lane, rowPP);
 #pragma unroll
@@ -1287,7 +1293,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
             if (fresh) {
                 if (own) root_nodes++;
                 if (!ACCOUNT && a.donate_every && root_nodes - looked >= a.donate_every &&
-                    root_nodes >= (uint64_t)kDonateFrom * a.donate_every && 2 + FWE <= kRecWords) {
+                    root_nodes >= (uint64_t)kDonateFrom * a.donate_every && 2 + FWE <= a.rec_words) {
                     looked = root_nodes;
                     // hand the upper half of the shallowest ancestor frame's untried
                     // children to an idle wave (not the root frame of a split root)
@@ -1310,7 +1316,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                         const uint32_t mine = keep_all > before ? min(cnt, keep_all - before) : 0u;
                         const uint64_t keepw = lowest_bits(qword, mine);
                         record_made(a);
-                        unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * kRecWords;
+                        unsigned long long* out = (unsigned long long*)a.area + (uint64_t)to * a.rec_words;
                         if (lane < W) {
                             st_dev(out + 2 + lane, Fi[lane] & ~keepw);
                             st_dev(out + 2 + W + lane, Fi[W + lane] | keepw);
@@ -1550,7 +1556,7 @@ __global__ __launch_bounds__(256, 4) void mce_kernel(MceArgs a) {
                     const uint32_t n = uniform(s_roots);
                     if (n || !total) units_done(a, n, total);
                 }
-                rec = a.area + gwave * kRecWords;
+                rec = a.area + gwave * a.rec_words;
             }
         } else {
             units_done(a, 1, total);
@@ -2034,6 +2040,7 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
         a.ring = (unsigned int*)(dq + done_bytes + rings_bytes);
         a.ring_mask = ring_size(waves) - 1;
         a.mail = (unsigned long long*)(dq + clear_bytes - waves * kDqStride * 8);
+        a.rec_words = kRecWords;
         a.area = (uint64_t*)(dq + clear_bytes);
         return G2_OK;
     };
@@ -2155,6 +2162,7 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
         a.big_list = nullptr;
         a.wave_span = nullptr;
         a.nwaves = (uint32_t)bwaves;
+        if (every) a.rec_words = donation_waves * kRecWords / bwaves;  // (wider roots, wider frames)
         a.backwards = 0;
         if ((e = hipMemsetAsync(a.queues, 0, kQueues * kQueueStride * 8, c->stream))) return hip_err(c, e, "memset next");
         if ((e = reset_donation())) return hip_err(c, e, "work donation reset");
