@@ -27,6 +27,11 @@ __global__ __launch_bounds__(256) void degree_kernel(const uint64_t* __restrict_
 // workgroup's, so that a hub is no serial tail.  A source that cannot raise the
 // maximum is left out, and a row is left at its first rowless neighbour.
 constexpr uint64_t kLongRow = 2048;
+// The host checks the rows itself up to this many entries of the sources: the
+// launch and the copy back are 14 us.  Uploads of a third of the vertices (R-MAT
+// 9, 11, 12, Chung-Lu of 10k and 20k vertices; 3k, 15k, 32k, 66k, 132k entries): 50,
+// 55, 62, 97, 185 us with the check here, 63, 66, 71, 92, 155 on the device.
+constexpr uint64_t kHostClosed = 1ull << 15;
 template <uint32_t STEP>
 __device__ __forceinline__ bool any_rowless(const uint32_t* __restrict__ cols, const uint32_t* deg, uint64_t lo,
                                             uint64_t hi, uint32_t at) {
@@ -247,6 +252,21 @@ int g2_upload_view(g2_ctx* c, const uint64_t* rp, uint64_t nv, const uint32_t* c
         if (chunk && d > chunk) w = (d + chunk - 1) / chunk;
         task_off[i + 1] = task_off[i] + w;
     }
+    // whole-graph view: every vertex is a source, in id order
+    bool all = ns == nv;
+    for (uint64_t i = 0; all && i < ns; i++) all = src[i] == i;
+    // closedness of the sources' rows, where it matters
+    const bool dev_closed = !all && deg_sum > kHostClosed;
+    uint32_t unclosed = 0;
+    for (uint64_t i = 0; !all && !dev_closed && i < ns; i++) {
+        if (src_deg[i] <= unclosed) continue;
+        const uint64_t lo = rp[src[i]], hi = rp[src[i] + 1];
+        for (uint64_t j = lo; j < hi; j++)
+            if (rp[cols[j] + 1] == rp[cols[j]]) {
+                unclosed = (uint32_t)(hi - lo);
+                break;
+            }
+    }
     windows_release(c);
     // The budget is checked for every view buffer before any is replaced, so
     // a refused upload leaves the previous view intact.
@@ -282,21 +302,17 @@ int g2_upload_view(g2_ctx* c, const uint64_t* rp, uint64_t nv, const uint32_t* c
     if ((e = hipMemcpyAsync(c->rp.ptr, rp, (nv + 1) * 8, hipMemcpyHostToDevice, c->stream))) return fail(hip_err(c, e, "H2D row_ptrs"));
     if (ne && (e = hipMemcpyAsync(c->cols.ptr, cols, ne * 4, hipMemcpyHostToDevice, c->stream))) return fail(hip_err(c, e, "H2D cols"));
     if (ns && (e = hipMemcpyAsync(c->src.ptr, src, ns * 4, hipMemcpyHostToDevice, c->stream))) return fail(hip_err(c, e, "H2D sources"));
-    // whole-graph view: every vertex is a source, in id order
-    bool all = ns == nv;
-    for (uint64_t i = 0; all && i < ns; i++) all = src[i] == i;
-    // degrees, and the closedness of the sources' rows where it matters (the
-    // view's host arrays were checked above, so every gather is in range)
+    // degrees, and the closedness of the sources' rows (the view's host arrays
+    // were checked above, so every gather is in range)
     uint32_t* const deg = (uint32_t*)c->deg.ptr;
     hipLaunchKernelGGL(degree_kernel, dim3((unsigned)std::min<uint64_t>(nv / 256 + 1, 8192)), dim3(256), 0, c->stream,
                        (const uint64_t*)c->rp.ptr, nv, deg);
-    if (!all && ns && ne)
+    if (dev_closed)
         hipLaunchKernelGGL(unclosed_kernel, dim3((unsigned)std::min<uint64_t>((ns + 3) / 4, (uint64_t)c->num_cus * 8)),
                            dim3(256), 0, c->stream, (const uint64_t*)c->rp.ptr, (const uint32_t*)c->cols.ptr,
                            (const uint32_t*)c->src.ptr, ns, nv, deg);
     if ((e = hipGetLastError())) return fail(hip_err(c, e, "degree kernels"));
-    uint32_t unclosed = 0;
-    if ((e = hipMemcpyAsync(&unclosed, deg + nv, 4, hipMemcpyDeviceToHost, c->stream)))
+    if (dev_closed && (e = hipMemcpyAsync(&unclosed, deg + nv, 4, hipMemcpyDeviceToHost, c->stream)))
         return fail(hip_err(c, e, "D2H unclosed degree"));
     if ((e = hipMemcpyAsync(c->gm_task_off.ptr, task_off.data(), (ns + 1) * 8, hipMemcpyHostToDevice, c->stream)))
         return fail(hip_err(c, e, "H2D task offsets"));
