@@ -76,7 +76,7 @@ struct MceArgs {
     unsigned long long* done;            // units of work done: roots and records, less records made
     unsigned long long* mail;            // per wave, a line each: MAIL_*
     uint64_t* area;                      // per wave: rec_words record words
-    uint64_t rec_words;
+    uint32_t rec_words;
     uint32_t nwaves;
     uint32_t donate_every;               // nodes between looks for idle waves (0 = never donate)
 };
@@ -2162,7 +2162,7 @@ int mce_run(g2_ctx* c, const g2_sched* sched, uint32_t flags, uint64_t* total, u
         a.big_list = nullptr;
         a.wave_span = nullptr;
         a.nwaves = (uint32_t)bwaves;
-        if (every) a.rec_words = donation_waves * kRecWords / bwaves;  // (wider roots, wider frames)
+        if (every) a.rec_words = (uint32_t)(donation_waves * kRecWords / bwaves);  // (wider roots, wider frames)
         a.backwards = 0;
         if ((e = hipMemsetAsync(a.queues, 0, kQueues * kQueueStride * 8, c->stream))) return hip_err(c, e, "memset next");
         if ((e = reset_donation())) return hip_err(c, e, "work donation reset");
