@@ -70,7 +70,7 @@ struct MceArgs {
     uint32_t backwards;                  // take the tasks from the last one down
     // work donation: a wave that sees idle waves hands one of them its
     // shallowest open frame (its untried children)
-    unsigned int* rings;                 // kRings lines: waves registered, waves taken, the difference
+    unsigned int* rings;                 // kRings lines: waves registered, waves taken, waves waiting
     unsigned int* ring;                  // kRings x (ring_mask + 1): wave id + 1, 0 = empty
     uint32_t ring_mask;
     unsigned long long* done;            // units of work done: roots and records, less records made
@@ -188,7 +188,7 @@ __device__ inline unsigned int* ring_place(const MceArgs& a, uint32_t r, unsigne
 // wait.
 struct RingLook {
     uint32_t r;            // ring looked at (wave-uniform)
-    unsigned int waiting;  // registered waves there at the last look
+    unsigned int waiting;  // waves waiting there at the last look (as an int: less than 0 between a donor's two steps)
     uint64_t begin;        // clock at the task's start
     uint64_t from;         // clock from which its frames may be handed on
 };
@@ -203,27 +203,28 @@ __device__ inline void walk_begins(RingLook& k) {
     k.from = now + (now - k.begin) / 2;
 }
 
-// a registered wave of the ring seen non-empty at the last look, taken off it; ~0 when there is none
+// a registered wave of the ring seen non-empty at the last look, taken off it; ~0
+// when there is none.  A donor first takes one of the waiting waves off their
+// count (and puts it back where there was none), then a place: two atomics that
+// each succeed, however many donors there are.  With the places' counter compared
+// and swapped in a loop, the donors of a ring failed on one another: 5 ms a
+// hand-over on R-MAT 13 (376,000 of them), 511 to 1209 ms where it now takes 8.8;
+// R-MAT 12 4.4 and 1.0.
 __device__ inline uint32_t ring_take(const MceArgs& a, RingLook& k) {
     uint32_t got = ~0u;
-    if (uniform(k.waiting) != 0 && (uint64_t)clock64() >= k.from) {
+    if ((int)uniform(k.waiting) > 0 && (uint64_t)clock64() >= k.from) {
         __builtin_amdgcn_wave_barrier();
         uint32_t w = ~0u;
         if (lane_id() == 0) {
             unsigned int* line = ring_line(a, k.r);
-            unsigned int out = ld_dev32(line + 1);
-            while (out != ld_dev32(line)) {
-                const unsigned int prev = atomicCAS(line + 1, out, out + 1);
-                if (prev == out) {
-                    unsigned int* place = ring_place(a, k.r, out);
-                    unsigned int id;
-                    while ((id = ld_dev32(place)) == 0) __builtin_amdgcn_s_sleep(1);  // (being written)
-                    st_dev32(place, 0);
-                    atomicSub(line + 2, 1u);
-                    w = id - 1;
-                    break;
-                }
-                out = prev;
+            if ((int)atomicSub(line + 2, 1u) > 0) {
+                unsigned int* place = ring_place(a, k.r, atomicAdd(line + 1, 1u));
+                unsigned int id;
+                while ((id = ld_dev32(place)) == 0) __builtin_amdgcn_s_sleep(1);  // (being written)
+                st_dev32(place, 0);
+                w = id - 1;
+            } else {
+                atomicAdd(line + 2, 1u);
             }
         }
         got = uniform(w);
