@@ -92,8 +92,9 @@ constexpr uint32_t kRecWords = 1024;
 constexpr uint32_t kRecRows = 16;         // first row word of a record that takes its rows along
 constexpr uint64_t kRegRecord = 1ull << 32;  // kind of a register_walk record (wide_walk<R>: R << 32; none: rows rebuilt)
 // A task looks for idle waves from this many x donate_every nodes on.  Fewer hand
-// on more and smaller frames than the waves' mailboxes serve: R-MAT 11 / R-MAT 10
-// 0.71 / 0.42 ms with 8, 1.1 / 0.36 with 3, 1.75 / 0.34 with 1.
+// on more and smaller frames, which serves small graphs and costs larger ones:
+// R-MAT 10 / 11 / 12 / 13 0.44 / 0.71 / 1.06 / 8.3 ms with 8, 0.36 / 0.54 / 1.35 /
+// 11.5 with 3, 0.33 / 0.53 / 1.86 / 13.2 with 1.
 constexpr uint32_t kDonateFrom = 8;
 enum { MAIL_NONE = 0, MAIL_RECORD, MAIL_END };
 
@@ -138,8 +139,9 @@ __device__ inline uint64_t degree_of(const uint64_t* __restrict__ rp, uint32_t u
 // it there, and one that never starts is never waited for.
 //
 // A ring has a place for every wave of its group, and a wave is registered at
-// most once at a time; a place is written only when it is empty, and emptied
-// by the donor that took it.
+// most once at a time.  A place is filled and emptied by one atomic each: where a
+// wave or a donor is held up for a whole turn of the ring, two waves or two donors
+// share a place, and every id is still kept, and taken once.
 //
 // Coherence without cache maintenance.  A device-scope acquire invalidates
 // the XCD's L2 and a device-scope release writes it back.  Instead every shared
@@ -196,8 +198,8 @@ __device__ inline RingLook ring_start(uint32_t gwave) { return RingLook{gwave % 
 // The taker of a frame without rows builds the root's bitsets again, so a task
 // hands nothing on before it has walked for half as long as its own build took
 // (a record's rows are a build of a microsecond).  With an eighth of that time and
-// three looks' nodes, R-MAT 11 / 5k-vertex Chung-Lu took 1.31 / 0.28 ms for 0.71 /
-// 0.31: more and smaller frames were handed on.
+// three looks' nodes, R-MAT 11 / 12 / 13 / 5k-vertex Chung-Lu took 0.48 / 1.33 / 11.0
+// / 0.24 ms for 0.71 / 1.06 / 8.3 / 0.27: more and smaller frames were handed on.
 __device__ inline void walk_begins(RingLook& k) {
     const uint64_t now = clock64();
     k.from = now + (now - k.begin) / 2;
@@ -220,8 +222,7 @@ __device__ inline uint32_t ring_take(const MceArgs& a, RingLook& k) {
             if ((int)atomicSub(line + 2, 1u) > 0) {
                 unsigned int* place = ring_place(a, k.r, atomicAdd(line + 1, 1u));
                 unsigned int id;
-                while ((id = ld_dev32(place)) == 0) __builtin_amdgcn_s_sleep(1);  // (being written)
-                st_dev32(place, 0);
+                while ((id = atomicExch(place, 0u)) == 0) __builtin_amdgcn_s_sleep(1);  // (being written)
                 w = id - 1;
             } else {
                 atomicAdd(line + 2, 1u);
@@ -271,8 +272,7 @@ __device__ inline bool wait_record(const MceArgs& a, uint32_t gwave) {
         if (got == MAIL_NONE) {
             const uint32_t r = gwave % kRings;
             unsigned int* place = ring_place(a, r, atomicAdd(ring_line(a, r), 1u));
-            while (ld_dev32(place) != 0) __builtin_amdgcn_s_sleep(1);  // (its last taker is emptying it)
-            st_dev32(place, gwave + 1);
+            while (atomicCAS(place, 0u, gwave + 1) != 0) __builtin_amdgcn_s_sleep(1);  // (its last taker is emptying it)
             atomicAdd(ring_line(a, r) + 2, 1u);
             while ((got = ld_dev(mail)) == MAIL_NONE) __builtin_amdgcn_s_sleep(32);
         }

@@ -26,3 +26,20 @@ def test_frequent_handing_on(g2, orc, scale):
             ms[every] = min(ex.run_mce()["stats"]["kernel_ms"] for _ in range(3))
             print("every", every, "kernel ms", ms[every], "donations", got["stats"]["donations"], flush=True)
     assert ms[0] < 3 * ms[128]
+
+
+@pytest.mark.parametrize("waves", [48, 112, 1008])
+def test_rings_as_small_as_their_groups(g2, orc, waves):
+    """large-root passes of few waves, and of 1,008: 63 in each of 16 rings of 64
+    places; every node handing on"""
+    print("case: rings, waves", waves, flush=True)
+    g = g2.gen_rmat(12, 16, 0.57, 0.19, 0.19, 9).preprocess().kcore_recode()[0]
+    ref = orc.mce(g, per_root=True)
+    with g2.Executor(device=0, mce_donate_every=1, wave_scratch_words=64, mce_small_max=1, big_waves=waves) as ex:
+        ex.transfer(g)
+        for _ in range(3):
+            got = ex.run_mce(per_root=True)
+            assert got["stats"]["big_roots"] >= waves
+            assert got["total"] == ref["total"]
+            assert np.array_equal(got["hist"], ref["hist"])
+            assert np.array_equal(got["per_root_nodes"], ref["per_root_nodes"])
