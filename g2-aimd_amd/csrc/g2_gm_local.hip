@@ -45,10 +45,10 @@
 //      cand(i) = AND of the rows of its back neighbours & order ranges &
 //      NON_EQUAL holes, recomputed word by word (no stacks); the last
 //      position is a popcount over the words its order range leaves.
-// The roots go through passes, each taking the roots the previous one
-// deferred: one wave per root with the rows in the wave's LDS (|U| <= 149);
-// one workgroup per root with the rows in the workgroup's LDS (|U| <= 448, 700, 1039); several workgroups per root with the
-// rows in a global arena.
+// The roots go through passes by their size, listed once per view before the
+// first one starts: one wave per root with the rows in the wave's LDS (|U| <=
+// 149); one workgroup per root with the rows in the workgroup's LDS (|U| <= 448,
+// 700, 1039); several workgroups per root with the rows in a global arena.
 #include <algorithm>
 #include <vector>
 
@@ -69,8 +69,7 @@ static_assert(LCTR_HOST <= LCTR_QUEUE, "counters");
 
 constexpr int kLocalBlockWaves = 4;     // gm_local_kernel: __launch_bounds__(256)
 constexpr uint32_t kLRowWords = 448;    // per-wave LDS rows (u64 words)
-constexpr uint32_t kLU = 256;           // |U| limit of a wave (triangle features; rows allow kLMembers)
-constexpr uint32_t kLMembers = 149;     // members of a root whose rows fit kLRowWords
+constexpr uint32_t kLMembers = 149;     // most members of a wave's root (their rows fit kLRowWords)
 constexpr uint32_t kLMemberRegs = (kLMembers + 63) / 64;
 constexpr uint32_t kLSlots = 512;       // hash slots over U, per wave
 // workgroup passes: threads, LDS row words, |U| limit, and workgroups per CU
@@ -108,10 +107,11 @@ struct LocalArgs {
 
 // u64 words between consecutive local rows: ceil(m/64) rounded up to odd, so
 // that lanes reading the rows of different ranks spread over the LDS banks
-__host__ __device__ inline uint32_t row_stride(uint64_t m) { return (uint32_t)((m + 63) / 64) | 1u; }
+__host__ __device__ constexpr uint32_t row_stride(uint64_t m) { return (uint32_t)((m + 63) / 64) | 1u; }
 
 // u64 words of a root's local rows
-__host__ __device__ inline uint64_t local_need(uint64_t m) { return m * row_stride(m); }
+__host__ __device__ constexpr uint64_t local_need(uint64_t m) { return m * row_stride(m); }
+static_assert(local_need(kLMembers) <= kLRowWords && local_need(kLMembers + 1) > kLRowWords, "a wave's rows");
 
 // set bit b of a local row word (the 32-bit half holding it: a 32-bit
 // atomic takes one LDS bank where the 64-bit one takes two)
@@ -785,7 +785,7 @@ __global__ __launch_bounds__(256, 7) void gm_local_kernel(LocalArgs a) {
         if constexpr (N == 2) {
             lane_total += rm;
         } else {
-            const bool mine = rm >= (uint32_t)(N - 1) && rm <= kLU && local_need(rm) <= kLRowWords;
+            const bool mine = rm >= (uint32_t)(N - 1) && rm <= kLMembers;
             uint64_t todo = ballot(mine);
             uint32_t u[kLMemberRegs];
             uint64_t lo = 0;
@@ -829,10 +829,9 @@ constexpr int block_waves(int n, bool clq, int bu) { return bu < kB3U && clq && 
 // (4-cliques) where they take 10.9 and 6.7.
 // Build: member i's row is one wave's work (wave i mod waves), cut into pieces
 // of 64 entries, kVecs pieces (of one or several members) in flight.  Which
-// member a piece belongs to is a scalar, and an entry is looked up by one LDS
-// read of its hash slot, a second only where the tag agrees (the members
-// themselves and 1 in 16 of the others).  Rows average ~400 entries on R-MAT
-// 22, of which 8% are hits.
+// member a piece belongs to is a scalar, and an entry is looked up by two LDS
+// reads, of its hash slot and of the member that slot names (build_rows).  Rows
+// average ~400 entries on R-MAT 22, of which 8% are hits.
 // Count: waves take the position-1 candidates r1 in turn; a wave's lanes share
 // their position-2 candidates, queued in LDS (cliques: the pairs of successive
 // r1 together, for 4-cliques two per lane so that four rows are read at a
@@ -1215,7 +1214,7 @@ __global__ __launch_bounds__(256) void ofill_kernel(const uint64_t* __restrict__
 __device__ inline int local_pass_of(uint32_t n, uint64_t m) {
     if (m < n - 1 || n == 2) return 0;
     const uint64_t need = local_need(m);
-    if (m <= kLU && need <= kLRowWords) return 0;
+    if (m <= kLMembers) return 0;
     if (m <= (uint64_t)kB1U && need <= (uint64_t)kB1RowWords) return 1;
     if (m <= (uint64_t)kB2U && need <= (uint64_t)kB2RowWords) return 2;
     if (m <= (uint64_t)kB3U && need <= (uint64_t)kB3RowWords) return 3;
@@ -1706,8 +1705,9 @@ static int pass_roots(g2_ctx* c, const uint64_t* orp, const uint32_t* rank, uint
 }
 
 // Passes over the roots: rows in a wave's LDS; in three sizes of workgroup LDS;
-// in global arenas sized to the largest root.  Which roots a pass takes is known before the first one starts,
-// so the passes are enqueued back to back and waited for once.
+// in global arenas sized to the largest root.  Which roots a pass takes is known
+// before the first one starts, so the passes are enqueued back to back and waited
+// for once.
 int gm_local_run(g2_ctx* c, uint64_t* count, g2_stats* st, bool bytes) {
     if (c->nv + 1 > 0x7fffffffull) return set_err(c, G2_EINVAL, "local-bitmap matching supports fewer than 2^31-1 vertices");
     windows_release(c);

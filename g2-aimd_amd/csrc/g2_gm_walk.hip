@@ -19,14 +19,15 @@
 // side and looked up in the other.
 //
 // What bounds it: chains of dependent loads (a lookup in a row is ~10 of
-// them) and, on skewed graphs, the hub roots.  So a row's bounds are searched
-// 64-ary by the whole wave, lookups keep two items per lane in flight, the
+// them) and, on skewed graphs, the hub roots.  So a list of several rounds is cut
+// to its value range 64-ary by the whole wave (a row's bounds in the closed form
+// are each lane's own, by halving), lookups keep two items per lane in flight, the
 // prefix's lists stay in LDS where they fit, and long root rows are split into
 // windows that any wave takes from one of 16 counters.  Against one candidate
 // at a time with scalar searches and a whole root (or caller's window) per
 // wave, per call on one MI355X:
 //   4 vertices, 5 edges, per-root counts, 100k-vertex Chung-Lu   58.6 -> 1.6 ms
-//   5 vertices, 8 edges, R-MAT 9 (512 vertices, 6k edges)         475 -> 1.4 ms
+//   5 vertices, 8 edges, R-MAT 9 (512 vertices, 6k edges)         475 -> 1.5 ms
 //   48 random patterns of 3-5 vertices in one launch, R-MAT 7     308 -> 0.85 ms
 #include <algorithm>
 #include <vector>

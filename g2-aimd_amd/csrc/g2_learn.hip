@@ -778,10 +778,11 @@ struct EpochArgs {
 };
 
 constexpr uint32_t kEpochTiles = 16;     // tiles per group, one per wave
-// Largest batch that takes this path.  It costs the same 27 ns a sample at any
-// batch, the three kernels less and less as more CUs work on a step: 3 epochs
-// of 50,001 samples in batches of 1536 take 4.06 ms here and 4.65 there, in
-// batches of 2048 about 4.1 and 4.1, in batches of 4096 3.4 there.
+// Largest batch that takes this path.  It costs up to 6.7 us a group of 256
+// samples at any batch, 27 ns a sample where the groups are full; the three kernels
+// cost less and less as more CUs work on a step: 3 epochs of 50,001 samples in
+// batches of 1536 take 4.06 ms here and 4.65 there, in batches of 2048 about 4.1
+// and 4.1, in batches of 4096 3.4 there.
 constexpr uint32_t kEpochBatch = 1536;
 
 struct EpochTile {

@@ -45,11 +45,14 @@ typedef struct g2_ctx g2_ctx;
 /* launch and scratch parameters (0 = library default) */
 typedef struct g2_tuning {
     uint32_t waves_per_cu;        /* resident search waves per CU of the persistent grids
-                                     (0 = each kernel's default: 16, local-bitmap matching 32) */
+                                     (0 = each kernel's default: MCE, batches and byte accounting 16,
+                                     the counting walk 20, local-bitmap matching 28) */
     uint32_t block_waves;         /* waves per workgroup */
     uint64_t wave_scratch_words;  /* per-wave u64 words for MCE local bitsets (small-root pass) */
     uint32_t big_waves;           /* large roots at a time: waves (MCE), arenas (matching) */
-    uint32_t gm_chunk;            /* level-1 candidates per matching task (0 = whole root) */
+    uint32_t gm_chunk;            /* level-1 candidates per matching task (0 = by rule: the walk cuts long
+                                     rows into windows, byte accounting takes whole roots); at least
+                                     the sources' row entries / 2^21 */
     uint32_t mce_small_max;       /* MCE roots of at most this degree run in registers
                                      (0 = 64, the most; 1 = practically off) */
     uint32_t mce_donate_every;    /* MCE: once a task has walked 8x this many nodes, the wave looks
@@ -67,8 +70,8 @@ typedef struct g2_stats {
     double   total_ms;            /* HIP-event time of the whole run on the context's stream */
     uint64_t nodes;               /* MCE search-tree nodes / GM partial-match extensions */
     uint64_t alg_bytes;           /* modelled algorithmic bytes (only with G2_RUN_ACCOUNT) */
-    uint64_t big_roots;           /* roots routed to the large-root pass (MCE, canonical matching), or
-                                     deferred by the first local-bitmap pass to the workgroup passes */
+    uint64_t big_roots;           /* MCE: roots routed to the large-root pass; local-bitmap matching:
+                                     roots of the passes after the first */
     uint64_t max_scratch_words;   /* largest per-root scratch need seen */
     double   wave_idle_frac;      /* MCE: 1 - sum of per-wave busy spans / (waves x makespan),
                                      from the GPU real-time clock (tail idleness) */
@@ -77,7 +80,7 @@ typedef struct g2_stats {
     uint32_t reserved;
     uint64_t local_pass_roots[5]; /* local-bitmap matching: roots each pass took to the end (rows in
                                      a wave's LDS; in three sizes of workgroup LDS;
-                                     in per-wave global arenas) */
+                                     in global arenas) */
     uint64_t host_spill_bytes;    /* MCE: page-locked host memory the large-root arenas used because
                                      the device budget could not hold one wave's arena (0 = none) */
     uint64_t device_bytes;        /* device memory the context holds after the run */
@@ -179,8 +182,8 @@ typedef struct g2_batch {
                                      [0, nq) (NULL = 0..nq-1) */
     uint32_t roots_per_task;      /* root tasks a wave takes per fetch (0 = 1) */
     uint32_t window;              /* level-1 window: candidates of a root row per root task
-                                     (0 = whole rows) */
-    uint32_t waves_per_cu;        /* resident waves per CU (0 = the context's tuning) */
+                                     (0 = by rule, as g2_tuning.gm_chunk) */
+    uint32_t waves_per_cu;        /* resident waves per CU (0 = the context's tuning, or 16) */
     uint32_t reserved;
     uint64_t node_budget;         /* per-query limit on partial-match extensions; a query
                                      that passes it is dropped and flagged (0 = none) */
