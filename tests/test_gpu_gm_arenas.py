@@ -37,3 +37,24 @@ def test_arenas_hold_the_stored_lists(g2, orc, d, q):
     assert got["count"] == ref["count"] == batch["counts"][0]
     assert np.array_equal(got["per_root_count"], ref["per_root_count"])
     assert solo <= cus * 16 * d * 2 * p.n * 4 + (16 << 20)
+
+
+def test_arena_of_one_list(g2, orc):
+    """an edge: its only list, of rows within and beyond the LDS pool (1,280
+    entries), alone and in a batch with patterns of 3 to 6 vertices"""
+    print("case: walk arenas, an edge", flush=True)
+    p = g2.plan_build([2, 1])
+    others = [g2.plan_for_preset(q) for q in (0, 2, 7, 10)]
+    for d in (1279, 1280, 1281, 4000):
+        g = star(g2, d, 100, d)
+        ref = orc.gm(g, orc.OrcPlan.from_buffer_copy(bytes(p)), per_root=True)
+        assert ref["count"] == g.ne // 2
+        with g2.Executor(device=0) as ex:
+            ex.transfer(g)
+            ex.set_plan(p)
+            got = ex.run_gm(per_root=True, canonical=True)
+            assert np.array_equal(got["per_root_count"], ref["per_root_count"]), d
+            assert ex.run_gm_batch([p])["counts"].tolist() == [ref["count"]]
+            counts = [orc.gm(g, orc.OrcPlan.from_buffer_copy(bytes(o)))["count"] for o in others]
+            assert ex.run_gm_batch([others[0], p, *others[1:], p])["counts"].tolist() == \
+                [counts[0], ref["count"], *counts[1:], ref["count"]]
