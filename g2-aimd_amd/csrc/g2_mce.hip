@@ -272,7 +272,8 @@ __device__ inline bool wait_record(const MceArgs& a, uint32_t gwave) {
         if (got == MAIL_NONE) {
             const uint32_t r = gwave % kRings;
             unsigned int* place = ring_place(a, r, atomicAdd(ring_line(a, r), 1u));
-            while (atomicCAS(place, 0u, gwave + 1) != 0) __builtin_amdgcn_s_sleep(1);  // (its last taker is emptying it)
+            // (until its last taker has emptied it)
+            while (ld_dev32(place) != 0 || atomicCAS(place, 0u, gwave + 1) != 0) __builtin_amdgcn_s_sleep(1);
             atomicAdd(ring_line(a, r) + 2, 1u);
             while ((got = ld_dev(mail)) == MAIL_NONE) __builtin_amdgcn_s_sleep(32);
         }
